@@ -1,6 +1,7 @@
 // C-ABI for the diatomic basis (include/hfgpu.h): handle, device tables and
 // the coupling lists of the Coulomb and exchange kernels (diatomic_jk.hip).
 #include "capi_common.hpp"
+#include <array>
 #include <cstring>
 #include <cstdlib>
 #include <cmath>
@@ -147,6 +148,12 @@ void diatomic_upload(hf_diatomic *h) {
   if (ch.empty()) ch.push_back(0.0);
   if (sg.empty()) sg.push_back(0.0);
   d.pq.upload(pq, s);
+  std::vector<double> pqo(pq.size());
+  for (size_t x = 0; x < pq.size() / TILE2; ++x)
+    for (int lane = 0; lane < 64; ++lane)
+      for (int u = 0; u < 4; ++u)
+        pqo[x * TILE2 + lane * 4 + u] = pq[x * TILE2 + (lane & 15) + TILE * ((lane >> 4) + 4 * u)];
+  d.pqo.upload(pqo, s);
   // log scale per (L,|M|, element) that brings the P and Q tiles to the same
   // magnitude, sqrt(max|P| max|Q|): P_L(cosh mu) reaches 1e75 and Q_L 1e-56
   // at L = 34, outside FP32, while their products across elements are O(1)
@@ -307,52 +314,42 @@ void diatomic_upload(hf_diatomic *h) {
   h->uploaded = true;
 }
 
-// Lists of the two-step cross-element exchange (k_dia_k2_off).  The terms of
-// output block (j,k) and (L,M) factor as fac(L,M) u(j,i) v(k,l) with u = (mod
-// Gaunt, plain Gaunt) of (j,i) and v the same of (k,l) (basis.cpp:1905-1960),
-// so R(j,k) = fac sum_i u(j,i) (x) V(i) with V_b(i) = sum_l v_b(k,l) P(i,l):
-// the V tiles of one (k, (L,|M|)) group serve every row j.  l_j + L + l_i is
-// even for every coupling, so a group splits by the parity of l_i into two
-// with disjoint rows.  A slot is one (M, i) of a group; its lt entries are the
-// (tile of (i,l), v0, v1) that pass the screen; a row's jt entries are (slot,
-// fac u0, fac u1).  Leaves d.k2 off when a column has more than K2_JMAX rows
-// or a group more than K2_SLOTS slots.
-void build_twostep(hf_diatomic *h, const std::vector<int> &act, const std::vector<int> &tile_of,
-                   const std::vector<unsigned char> &mask, const std::vector<int> &ilm_of,
-                   const std::vector<double> &fac_of, int Mext, int dmoff, hipStream_t s) {
+// Factorised exchange couplings of one column shell k and (L,|M|): the terms
+// of output block (j,k) and (L,M) factor as fac(L,M) u(j,i) v(k,l) with u =
+// (mod Gaunt, plain Gaunt) of (j,i) and v the same of (k,l)
+// (basis.cpp:1905-1960), so R(j,k) = fac sum_i u(j,i) (x) V(i) with V_b(i) =
+// sum_l v_b(k,l) P(i,l), and the V tiles serve every row j.  A slot is one
+// (M, i); its lt entries are the (tile of (i,l), v0, v1) that pass the screen;
+// a row's jt entries are (slot, fac u0, fac u1).  l_j + L + l_i is even for
+// every coupling, so the slots of one parity of l_i have rows of their own.
+struct CoupleGroup {
+  typedef std::pair<int, std::pair<double, double>> Entry;
+  int ilm, par;
+  std::vector<std::pair<int, int>> slots;  // (M, i)
+  std::vector<std::vector<Entry>> lt, jt;  // per slot: (tile, v); per row: (slot, c)
+};
+
+// The groups of every column shell k (ascending ilm, then parity) over its
+// rows[k] (ascending shell).
+std::vector<std::vector<CoupleGroup>> couple_groups(hf_diatomic *h, const std::vector<std::vector<int>> &rows,
+                                                    const std::vector<int> &tile_of,
+                                                    const std::vector<unsigned char> &mask,
+                                                    const std::vector<int> &ilm_of,
+                                                    const std::vector<double> &fac_of, int Mext, int dmoff) {
   const DiatomicSetup &S = h->host;
-  DiatomicDevice &d = h->dev;
-  const int Na = S.Nang(), Nel = S.Nel();
+  const DiatomicDevice &d = h->dev;
+  const int Na = S.Nang(), nlm = d.n_lm, gL = d.gL;
   const auto &lv = S.lval;
   const auto &mv = S.mval;
-  d.k2 = false;
-  d.n_wg_k2 = 0;
-  if (!d.tiled || Nel < 2 || act.empty()) return;
-  // rows of every column shell k
-  std::vector<std::vector<int>> rows(Na);
-  for (int jk : act) rows[jk % Na].push_back(jk / Na);
-  std::vector<int> ks;
-  for (int k = 0; k < Na; ++k) {
-    if (rows[k].empty()) continue;
-    if ((int)rows[k].size() > K2_JMAX) return;
-    ks.push_back(k);
-  }
-  struct Group {
-    int ilm, par;
-    std::vector<std::pair<int, int>> slots;               // (M, i)
-    std::vector<std::vector<std::pair<int, std::pair<double, double>>>> lt;  // per slot: (tile, v)
-    std::vector<std::vector<std::pair<int, std::pair<double, double>>>> jt;  // per row: (slot, c)
-  };
-  const int nlm = d.n_lm, gL = d.gL;
   std::vector<std::vector<int>> sector(2 * dmoff + 1);  // shells by m + dmoff
   for (int a = 0; a < Na; ++a) sector[mv[a] + dmoff].push_back(a);
-  std::vector<std::vector<Group>> groups(ks.size());
-  bool fits = true;
+  std::vector<std::vector<CoupleGroup>> groups(Na);
 #pragma omp parallel for schedule(dynamic)
-  for (size_t kq = 0; kq < ks.size(); ++kq) {
-    const int k = ks[kq], mk = mv[k];
+  for (int k = 0; k < Na; ++k) {
+    const int mk = mv[k];
     const std::vector<int> &js = rows[k];
-    std::vector<Group> &G = groups[kq];
+    if (js.empty()) continue;
+    std::vector<CoupleGroup> &G = groups[k];
     std::vector<int> gidx((size_t)2 * nlm, -1);
     std::vector<int> Lk;
     for (int L = 0; L < gL; ++L)
@@ -387,7 +384,7 @@ void build_twostep(hf_diatomic *h, const std::vector<int> &act, const std::vecto
             if (sl < 0) {
               // the slot's density blocks (i,l) that pass the screen; a group
               // is opened only with its first non-empty slot
-              std::vector<std::pair<int, std::pair<double, double>>> ltv;
+              std::vector<CoupleGroup::Entry> ltv;
               for (int l : Lk) {
                 const int tl = mask[(size_t)i * Na + l] ? tile_of[(size_t)i * Na + l] : -1;
                 if (tl < 0) continue;
@@ -397,126 +394,241 @@ void build_twostep(hf_diatomic *h, const std::vector<int> &act, const std::vecto
               if (ltv.empty()) continue;
               if (g < 0) {
                 g = (int)G.size();
-                G.push_back(Group{ilm, par, {}, {},
-                                  std::vector<std::vector<std::pair<int, std::pair<double, double>>>>(js.size())});
+                G.push_back(CoupleGroup{ilm, par, {}, {}, std::vector<std::vector<CoupleGroup::Entry>>(js.size())});
               }
               sl = (int)G[g].slots.size();
               G[g].slots.push_back({M, i});
               G[g].lt.push_back(std::move(ltv));
             }
-            Group &gr = G[g];
-            gr.jt[q].push_back({sl, {fac * u0, fac * u1}});
+            G[g].jt[q].push_back({sl, {fac * u0, fac * u1}});
           }
         }
       }
-    std::sort(G.begin(), G.end(),
-              [](const Group &a, const Group &b) { return a.ilm < b.ilm || (a.ilm == b.ilm && a.par < b.par); });
-    for (const Group &gr : G)
-      if ((int)gr.slots.size() > K2_SLOTS) {
-#pragma omp critical
-        fits = false;
-      }
+    std::sort(G.begin(), G.end(), [](const CoupleGroup &a, const CoupleGroup &b) {
+      return a.ilm < b.ilm || (a.ilm == b.ilm && a.par < b.par);
+    });
   }
-  if (!fits) return;
-  // flatten
-  std::vector<int> kshell, kj(1, 0), jshell, kg(1, 0), gilm, gslot(1, 0), gjt, sl(1, 0), lt, jto, jts;
-  std::vector<double> ltv, jtc;
-  std::vector<double> kcost(ks.size(), 0.0);
+  return groups;
+}
+
+// Lists of the two-step cross-element exchange (k_dia_k2_off) from the
+// groups of every column shell.  The rows of a column with one m and parity
+// of l share their slots, so they are dealt to waves in such sets (a wave
+// reads each slot tile once for its rows), the waves of a workgroup divided
+// over its sets so that the largest number of rows in a wave is least; a
+// column with more rows than a workgroup holds gets several.  The two
+// parities of an (L,|M|) share one group when their slots fit the K2_SLOTS
+// tiles of LDS (half the barriers, and the rows of both parities keep all
+// waves busy), else each has its own, cut again when it still does not fit
+// (the sums over slots are linear).
+void build_twostep(hf_diatomic *h, const std::vector<std::vector<int>> &rows,
+                   const std::vector<std::vector<CoupleGroup>> &groups, hipStream_t s) {
+  const DiatomicSetup &S = h->host;
+  DiatomicDevice &d = h->dev;
+  const int Na = S.Nang(), Nel = S.Nel();
+  d.k2 = false;
+  d.n_wg_k2 = 0;
+  if (!d.tiled || Nel < 2 || !d.finite) return;
+  if (std::getenv("HFGPU_EXCHANGE_TWOSTEP") && std::atoi(std::getenv("HFGPU_EXCHANGE_TWOSTEP")) == 0) return;
+  std::vector<int> kshell, wrows, kg(1, 0), gilm, gslot(1, 0), sl(1, 0), lt, jo(1, 0), js;
+  std::vector<double> ltv, jtc, kcost;
   double n_lt = 0.0, n_jt = 0.0, frad = 0.0;
-  for (size_t kq = 0; kq < ks.size(); ++kq) {
-    kshell.push_back(ks[kq]);
-    for (int j : rows[ks[kq]]) jshell.push_back(j);
-    kj.push_back((int)jshell.size());
-    for (const Group &gr : groups[kq]) {
-      gilm.push_back(gr.ilm);
-      gjt.push_back((int)jto.size());
-      for (size_t x = 0; x < gr.slots.size(); ++x) {
-        for (auto &e : gr.lt[x]) {
-          lt.push_back(e.first);
-          ltv.push_back(e.second.first);
-          ltv.push_back(e.second.second);
-        }
-        sl.push_back((int)lt.size());
-        n_lt += (double)gr.lt[x].size();
-        kcost[kq] += 2.0 * (double)gr.lt[x].size();
+  // radial products per slot (H) and per row: two 16x16x16 each
+  double f_slot = 0.0, f_row = 0.0, sum_off = 0.0;
+  for (int e = 0; e < Nel; ++e)
+    for (int f = 0; f < Nel; ++f)
+      if (d.sym ? e > f : e != f) {
+        const double a = S.rad.ni[e], b = S.rad.ni[f];
+        f_slot += 4.0 * a * b * b;
+        f_row += 4.0 * a * a * b;
+        sum_off += a * b;
       }
-      gslot.push_back((int)sl.size() - 1);
-      jto.push_back((int)jts.size());
-      for (auto &rowv : gr.jt) {
-        for (auto &e : rowv) {
-          jts.push_back(e.first);
-          jtc.push_back(e.second.first);
-          jtc.push_back(e.second.second);
+  typedef std::vector<std::pair<const CoupleGroup *, int>> SlotList;
+  for (int k = 0; k < Na; ++k) {
+    // sets of rows (positions in rows[k]) by (m, parity of l)
+    std::map<std::pair<int, int>, std::vector<int>> sets;
+    for (size_t q = 0; q < rows[k].size(); ++q)
+      sets[{S.mval[rows[k][q]], S.lval[rows[k][q]] & 1}].push_back((int)q);
+    // workgroups of whole sets, or of as much of a set as fits
+    std::vector<std::vector<std::vector<int>>> wgs(1);
+    int waves = 0;
+    for (auto &kv : sets)
+      for (size_t q0 = 0; q0 < kv.second.size();) {
+        if (waves == K2_WAVES) {
+          wgs.emplace_back();
+          waves = 0;
         }
-        jto.push_back((int)jts.size());
-        n_jt += (double)rowv.size();
-        if (!rowv.empty()) {
-          frad += d.sym ? d.h_rad_low[gr.ilm] : d.h_rad_off[gr.ilm];
-          kcost[kq] += (double)rowv.size() + 24.0;
-        }
+        const size_t q1 = std::min(kv.second.size(), q0 + (size_t)(K2_WAVES - waves) * K2_ROWS);
+        wgs.back().emplace_back(kv.second.begin() + q0, kv.second.begin() + q1);
+        waves += (int)((q1 - q0 + K2_ROWS - 1) / K2_ROWS);
+        q0 = q1;
       }
+    for (const auto &set_list : wgs) {
+      if (set_list.empty()) continue;
+      std::vector<int> nw;
+      int used_w = 0;
+      for (const auto &st : set_list) {
+        nw.push_back(((int)st.size() + K2_ROWS - 1) / K2_ROWS);
+        used_w += nw.back();
+      }
+      auto most = [&](size_t x) { return ((int)set_list[x].size() + nw[x] - 1) / nw[x]; };
+      for (; used_w < K2_WAVES; ++used_w) {
+        size_t best = 0;
+        for (size_t x = 1; x < nw.size(); ++x)
+          if (most(x) > most(best)) best = x;
+        if (most(best) <= 1) break;
+        ++nw[best];
+      }
+      std::vector<std::vector<int>> wr;  // rows of every wave
+      std::vector<int> part;
+      for (size_t x = 0; x < set_list.size(); ++x)
+        for (int u = 0; u < nw[x]; ++u) {
+          const size_t n = set_list[x].size(), a = n * u / nw[x], b = n * (u + 1) / nw[x];
+          wr.emplace_back(set_list[x].begin() + a, set_list[x].begin() + b);
+          part.insert(part.end(), wr.back().begin(), wr.back().end());
+        }
+      wr.resize(K2_WAVES);
+      double cost = 0.0;
+      kshell.push_back(k);
+      for (const auto &w : wr)
+        for (int r = 0; r < K2_ROWS; ++r) wrows.push_back(r < (int)w.size() ? rows[k][w[r]] : -1);
+      auto emit = [&](int ilm, const SlotList &ss) {
+        gilm.push_back(ilm);
+        std::map<std::pair<const CoupleGroup *, int>, int> at;
+        for (const auto &x : ss) {
+          const int z = (int)at.size();
+          at[x] = z;
+          for (const auto &e : x.first->lt[x.second]) {
+            lt.push_back(e.first);
+            ltv.push_back(e.second.first);
+            ltv.push_back(e.second.second);
+          }
+          // in fours: the padding repeats a tile of the slot with zero weights
+          while (lt.size() % 4) {
+            lt.push_back(lt.back());
+            ltv.insert(ltv.end(), 2, 0.0);
+          }
+          sl.push_back((int)lt.size());
+          n_lt += (double)x.first->lt[x.second].size();
+          frad += f_slot;
+          cost += (double)x.first->lt[x.second].size() + 8.0;
+        }
+        gslot.push_back((int)sl.size() - 1);
+        std::vector<const CoupleGroup *> gs(1, ss.front().first);
+        if (ss.back().first != ss.front().first) gs.push_back(ss.back().first);
+        for (const auto &w : wr) {
+          std::map<int, std::array<double, 2 * K2_ROWS>> cf;  // slot -> coefficients of the wave's rows
+          for (size_t r = 0; r < w.size(); ++r) {
+            bool any = false;
+            for (const CoupleGroup *g : gs)
+              for (const auto &e : g->jt[w[r]]) {
+                const auto it = at.find({g, e.first});
+                if (it == at.end()) continue;
+                auto &c = cf.emplace(it->second, std::array<double, 2 * K2_ROWS>{}).first->second;
+                c[2 * r] = e.second.first;
+                c[2 * r + 1] = -e.second.second;
+                n_jt += 1.0;
+                any = true;
+              }
+            if (any) {
+              frad += f_row;
+              cost += 8.0;
+            }
+          }
+          for (const auto &x : cf) {
+            js.push_back(x.first);
+            jtc.insert(jtc.end(), x.second.begin(), x.second.end());
+          }
+          if (js.size() % 2) {  // in twos
+            js.push_back(js.back());
+            jtc.insert(jtc.end(), 2 * K2_ROWS, 0.0);
+          }
+          cost += (double)(cf.size() * w.size());
+          jo.push_back((int)js.size());
+        }
+      };
+      const std::vector<CoupleGroup> &G = groups[k];
+      for (size_t a = 0; a < G.size();) {
+        size_t b = a;
+        std::vector<SlotList> parts;
+        size_t total = 0;
+        for (; b < G.size() && G[b].ilm == G[a].ilm; ++b) {
+          SlotList ss;
+          std::vector<unsigned char> used(G[b].slots.size(), 0);
+          for (int q : part)
+            for (const auto &e : G[b].jt[q]) used[e.first] = 1;
+          for (size_t z = 0; z < used.size(); ++z)
+            if (used[z]) ss.push_back({&G[b], (int)z});
+          total += ss.size();
+          if (!ss.empty()) parts.push_back(std::move(ss));
+        }
+        if (parts.size() == 2 && total <= (size_t)K2_SLOTS) {
+          parts[0].insert(parts[0].end(), parts[1].begin(), parts[1].end());
+          parts.pop_back();
+        }
+        for (const SlotList &ss : parts)
+          for (size_t z = 0; z < ss.size(); z += K2_SLOTS)
+            emit(G[a].ilm, SlotList(ss.begin() + z, ss.begin() + std::min(ss.size(), z + K2_SLOTS)));
+        a = b;
+      }
+      kg.push_back((int)gilm.size());
+      kcost.push_back(cost);
     }
-    kg.push_back((int)gilm.size());
   }
-  // workgroups: element pairs of the launch dealt to XCDs (pair index % 8),
-  // columns in decreasing cost within each pair
+  if (gilm.empty()) return;
+  // workgroups: the element pairs one after another, columns in decreasing
+  // cost within each, are cut into eight runs of equal cost, one per XCD (few
+  // pairs' slices of the density tiles per L2); an XCD takes its run column by
+  // column, so neighbouring CUs, which share a scalar cache, read the same
+  // lists (N2: 5.1 ms against 5.7 pair by pair)
   std::vector<int> efs;
   for (int e = 0; e < Nel; ++e)
     for (int f = 0; f < Nel; ++f)
       if (d.sym ? e > f : e != f) efs.push_back(e * Nel + f);
-  std::vector<int> korder(ks.size());
-  for (size_t q = 0; q < ks.size(); ++q) korder[q] = (int)q;
+  std::vector<int> korder(kshell.size());
+  double ktot = 0.0;
+  for (size_t q = 0; q < korder.size(); ++q) {
+    korder[q] = (int)q;
+    ktot += kcost[q];
+  }
   std::sort(korder.begin(), korder.end(), [&](int a, int b) { return kcost[a] > kcost[b]; });
-  std::vector<std::vector<int>> per_xcd(8);
-  for (size_t p = 0; p < efs.size(); ++p)
-    for (int kq : korder) {
-      auto &v = per_xcd[p % 8];
-      v.push_back(kq);
-      v.push_back(efs[p]);
+  std::vector<std::vector<std::pair<int, int>>> per_xcd(8);  // (position in korder, element pair)
+  double done = 0.0;
+  const double all = ktot * (double)efs.size();
+  for (int ef : efs)
+    for (size_t q = 0; q < korder.size(); ++q) {
+      const double c = kcost[korder[q]];
+      per_xcd[std::min(7, (int)(8.0 * (done + 0.5 * c) / all))].push_back({(int)q, ef});
+      done += c;
     }
   size_t mx = 0;
-  for (auto &v : per_xcd) mx = std::max(mx, v.size() / 2);
+  for (auto &v : per_xcd) mx = std::max(mx, v.size());
   std::vector<int> wg(mx * 8 * 2, -1);
-  for (int x = 0; x < 8; ++x)
-    for (size_t q = 0; q < per_xcd[x].size() / 2; ++q) {
-      wg[(q * 8 + x) * 2] = per_xcd[x][2 * q];
-      wg[(q * 8 + x) * 2 + 1] = per_xcd[x][2 * q + 1];
+  for (int x = 0; x < 8; ++x) {
+    std::stable_sort(per_xcd[x].begin(), per_xcd[x].end());
+    for (size_t q = 0; q < per_xcd[x].size(); ++q) {
+      wg[(q * 8 + x) * 2] = korder[per_xcd[x][q].first];
+      wg[(q * 8 + x) * 2 + 1] = per_xcd[x][q].second;
     }
-  if (lt.empty()) {
-    lt.push_back(0);
-    ltv.assign(2, 0.0);
-  }
-  if (jts.empty()) {
-    jts.push_back(0);
-    jtc.assign(2, 0.0);
-  }
-  if (gilm.empty()) {
-    gilm.push_back(0);
-    gjt.push_back(0);
   }
   d.k2_wg.upload(wg, s);
   d.k2_kshell.upload(kshell, s);
-  d.k2_kj.upload(kj, s);
-  d.k2_jshell.upload(jshell, s);
+  d.k2_rows.upload(wrows, s);
   d.k2_kg.upload(kg, s);
   d.k2_gilm.upload(gilm, s);
   d.k2_gslot.upload(gslot, s);
-  d.k2_gjt.upload(gjt, s);
   d.k2_sl.upload(sl, s);
   d.k2_lt.upload(lt, s);
   d.k2_ltv.upload(ltv, s);
-  d.k2_jto.upload(jto, s);
-  d.k2_jts.upload(jts, s);
+  d.k2_jo.upload(jo, s);
+  d.k2_js.upload(js, s);
   d.k2_jtc.upload(jtc, s);
+  hip_check(hipStreamSynchronize(s), "two-step list upload");  // before the host lists go
   d.n_wg_k2 = (int)(mx * 8);
-  // per element pair: 4 flops per lt entry (two channels) and 8 per jt entry
-  // (four channels) on every tile entry, plus the radial products
-  double sum_off = 0.0;
-  for (int e = 0; e < Nel; ++e)
-    for (int f = 0; f < Nel; ++f)
-      if (d.sym ? e > f : e != f) sum_off += (double)S.rad.ni[e] * S.rad.ni[f];
-  d.flops_off_k2 = frad + (4.0 * n_lt + 8.0 * n_jt) * sum_off;
-  d.k2 = std::getenv("HFGPU_EXCHANGE_TWOSTEP") == nullptr || std::atoi(std::getenv("HFGPU_EXCHANGE_TWOSTEP")) != 0;
+  // per element pair and tile entry 4 flops per lt entry (two channels) and
+  // 4 per jt entry (two row sums), plus the radial products
+  d.flops_off_k2 = frad + 4.0 * (n_lt + n_jt) * sum_off;
+  d.k2 = true;
 }
 
 // Exchange coupling lists for the density blocks that pass the norm screen
@@ -541,7 +653,13 @@ void build_exchange_lists(hf_diatomic *h, hipStream_t s) {
         const unsigned char m = mask[(size_t)i * Na + l] | mask[(size_t)l * Na + i];
         mask[(size_t)i * Na + l] = mask[(size_t)l * Na + i] = m;
       }
-  if (!d.screen_mask.empty() && mask == d.screen_mask && d.sym == d.list_sym) return;
+  // a density with infinities or NaNs (or beyond FP32's range) takes the
+  // one-step kernels, whose sums hold exactly the coupled terms (no padding,
+  // no shared rows)
+  bool finite = true;
+  for (size_t q = 0; q < mask.size(); ++q) finite = finite && d.h_bnorm.p[q] < 1e30;
+  if (!d.screen_mask.empty() && mask == d.screen_mask && d.sym == d.list_sym && finite == d.finite) return;
+  d.finite = finite;
   int mabs = 0;
   for (int m : mv) mabs = std::max(mabs, std::abs(m));
   const int dmoff = 2 * mabs;
@@ -766,7 +884,9 @@ void build_exchange_lists(hf_diatomic *h, hipStream_t s) {
     d.n_src = (int)src.size();
     d.src_blk.upload(src, s);
     d.term_tile.upload(tt, s);
-    build_twostep(h, act, id, mask, ilm_of, fac_of, Mext, dmoff, s);
+    std::vector<std::vector<int>> rows(Na);  // of every column shell k
+    for (int jk : act) rows[jk % Na].push_back(jk / Na);
+    build_twostep(h, rows, couple_groups(h, rows, id, mask, ilm_of, fac_of, Mext, dmoff), s);
   }
   d.term_f.upload(tf, s);
   hip_check(hipStreamSynchronize(s), "exchange list upload");

@@ -26,6 +26,7 @@
 // 16) stays in the L2 of the XCD that works on it.
 #include "hfgpu_internal.hpp"
 #include "device_common.hpp"
+#include <type_traits>
 
 // terms in flight per lane in the cross-element gathers, and that launch's
 // waves per SIMD
@@ -613,14 +614,24 @@ __global__ void __launch_bounds__(NT) k_dia_k_in(DKArgs<T> A) {
 // --- Cross-element exchange in two steps ----------------------------------------
 //
 // One workgroup per (column shell k, element pair (e,f)); each wave owns up to
-// three rows j of the column and keeps their output tiles in registers over
-// all coupled (L,|M|) groups of k.  Per group (and parity class of l_i): the
-// slot tiles V_b(i) = sum_l v_b(k,l) P(i,l) of the pair are formed in LDS
-// (waves split the slots), then each owned row gathers its four channel tiles
-// R00 = sum c0 V0, R02 = -sum c0 V1, R20 = -sum c1 V0, R22 = sum c1 V1 from LDS
-// and applies the disjoint P/Q factors as k_dia_k_off does.  The rows share
-// each V tile, so the L2 gathers drop from |S_j| |S_k| per row and group to
-// |S_k| per slot.
+// three rows j of the column (of one m and parity of l, which share their
+// slots) and keeps their output tiles in registers over all coupled (L,|M|)
+// groups of k.  Per group: the slot tiles V_b(i) = sum_l v_b(k,l) P(i,l) of
+// the pair are gathered (waves split the slots) and multiplied by the column
+// side's disjoint factors at once, H(i) = V0 j0' - V1 j2', which goes to LDS;
+// then each wave sums G0 = sum c0 H, G1 = -sum c1 H of its rows from LDS and
+// adds i0 G0 + i2 G1 (the four channel tiles R00 = sum c0 V0, R02 = -sum c0 V1,
+// R20 = -sum c1 V0, R22 = sum c1 V1 of k_dia_k_off never exist).  The rows
+// share each H tile, so the L2 gathers drop from |S_j| |S_k| per row and group
+// to |S_k| per slot, and a row costs two 16x16x16 products and one LDS tile
+// per slot and wave.  FP32 adds each group's products to the rows in FP64 (in
+// FP32 the sum over all groups lost a quarter of a digit).
+// N2 (lmax 16, 8 elements): 5.1 ms, 9.5 ms with the four channel tiles formed
+// per row; 13.6 ms of matrix time over 1024 SIMDs (23% busy), the rest is
+// latency: tile gathers (2.2 ms of it), list loads and the two barriers per
+// group.  Two 512-thread workgroups per CU (16 waves) measured fastest: 384
+// threads 7.3, 256 threads 6.8, one of 1024 over two element pairs 5.4 ms;
+// the lists staged in LDS 5.4, eight gathers in flight 5.2 ms.
 
 template <typename T>
 struct DK2Args {
@@ -631,105 +642,134 @@ struct DK2Args {
   int Nel, Nang;
   const int *first, *ni, *skip;
   const long long *poff;
-  const T *pq;
-  const int *wg, *kshell, *kj, *jshell, *kg, *gilm, *gslot, *gjt, *sl, *lt, *jto, *jts;
+  const T *pqo;        // P/Q tiles in operand order
+  const double *lsig;  // FP32 only: log scale of the (ilm, element) P/Q tiles
+  const int *wg, *kshell, *rows, *kg, *gilm, *gslot, *sl, *lt, *jo, *js;
   const T *ltv, *jtc;
   int sym;
 };
 
+// Slot tiles sit in LDS as two halves [half][lane][2], so that a wave's
+// 16-byte accesses are contiguous (no bank conflicts).
 template <typename T>
-__global__ void __launch_bounds__(K2_THREADS) k_dia_k2_off(DK2Args<T> A) {
+__device__ inline typename Mma<T>::acc_t h_load(const T *H, int lane) {
+  typedef T v2 __attribute__((ext_vector_type(2)));
+  const v2 a = *reinterpret_cast<const v2 *>(H + 2 * lane), b = *reinterpret_cast<const v2 *>(H + 128 + 2 * lane);
+  return typename Mma<T>::acc_t{a[0], a[1], b[0], b[1]};
+}
+template <typename T>
+__device__ inline void h_store(T *H, int lane, typename Mma<T>::acc_t v) {
+  typedef T v2 __attribute__((ext_vector_type(2)));
+  *reinterpret_cast<v2 *>(H + 2 * lane) = v2{v[0], v[1]};
+  *reinterpret_cast<v2 *>(H + 128 + 2 * lane) = v2{v[2], v[3]};
+}
+
+template <typename T>
+__global__ void __launch_bounds__(K2_THREADS) __attribute__((amdgpu_waves_per_eu(4))) k_dia_k2_off(DK2Args<T> A) {
   typedef Mma<T> MM;
   typedef typename MM::acc_t acc_t;
   typedef acc_t vec;
-  constexpr int NW = K2_THREADS / 64, JPW = K2_JMAX / NW;
-  __shared__ T V[K2_SLOTS * 2 * TILE2];  // slot tiles V0, V1 in lane-major operand order
+  __shared__ T Hs[K2_SLOTS * TILE2];  // slot tiles H in result order (the next product's Y operand)
   const int w = blockIdx.x;
   const int kq = A.wg[2 * w], ef = A.wg[2 * w + 1];
   if (kq < 0) return;
   const int e = ef / A.Nel, f = ef - e * A.Nel;
-  const int k = A.kshell[kq], r0 = A.kj[kq], nr = A.kj[kq + 1] - r0;
+  const int k = A.kshell[kq];
   const int t = threadIdx.x, lane = t & 63, g = lane >> 4, c = lane & 15;
   const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
-  int kk[4];
+  const int *wrow = A.rows + (kq * K2_WAVES + wv) * K2_ROWS;
+  static_assert(K2_ROWS == 3, "row counts dispatched below");
+  const int nrow = wrow[2] >= 0 ? 3 : wrow[1] >= 0 ? 2 : 1;
+  v4d acc[K2_ROWS];  // one accumulator per owned row
 #pragma unroll
-  for (int s = 0; s < 4; ++s) kk[s] = MM::row(g, s);
-  acc_t acc[JPW];  // one accumulator per owned row (registers: three rows per wave)
-#pragma unroll
-  for (int r = 0; r < JPW; ++r) acc[r] = acc_t{0, 0, 0, 0};
-  const T *pt = A.pt + (size_t)ef * A.n_src * TILE2 + lane * 4;
+  for (int r = 0; r < K2_ROWS; ++r) acc[r] = v4d{0, 0, 0, 0};
+  const T *pt = A.pt + (size_t)ef * A.n_src * TILE2;
   const bool up = e > f;
   for (int gi = A.kg[kq]; gi < A.kg[kq + 1]; ++gi) {
     const int ilm = A.gilm[gi], s0 = A.gslot[gi], ns = A.gslot[gi + 1] - s0;
-    // the group's factor operands are fetched first and used after the slot
-    // phase: row side Q of e if e > f else P of e, column side the other kind
-    T a0[4], a2[4], b0[4], b2[4];
-    {
-      const T *te = A.pq + ((size_t)ilm * A.Nel + e) * 4 * TILE2, *tf = A.pq + ((size_t)ilm * A.Nel + f) * 4 * TILE2;
-      const T *i0 = te + (up ? 2 : 0) * TILE2, *i2 = te + (up ? 3 : 1) * TILE2;
-      const T *j0 = tf + (up ? 0 : 2) * TILE2, *j2 = tf + (up ? 1 : 3) * TILE2;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const int x = c + TILE * kk[s];
-        a0[s] = i0[x];
-        a2[s] = i2[x];
-        b0[s] = j0[x];
-        b2[s] = j2[x];
-      }
+    // the group's factor operands: row side Q of e if e > f else P of e,
+    // column side the other kind
+    const T *te = A.pqo + ((size_t)ilm * A.Nel + e) * 4 * TILE2 + (up ? 2 : 0) * TILE2;
+    const T *tf = A.pqo + ((size_t)ilm * A.Nel + f) * 4 * TILE2 + (up ? 0 : 2) * TILE2;
+    const vec b0 = *reinterpret_cast<const vec *>(tf + lane * 4);
+    const vec b2 = *reinterpret_cast<const vec *>(tf + TILE2 + lane * 4);
+    T rho = T(1);
+    if constexpr (sizeof(T) == 4) {
+      // FP32 tiles hold P / s and Q * s per (ilm, element): restore the
+      // pair's Q(e) P(f) or P(e) Q(f) scale, s_f / s_e or s_e / s_f
+      const double le = A.lsig[ilm * A.Nel + e], lf = A.lsig[ilm * A.Nel + f];
+      rho = (T)exp(up ? lf - le : le - lf);
     }
     __syncthreads();  // the previous group's LDS tiles are no longer read
-    for (int sq = wv; sq < ns; sq += NW) {
+    for (int sq = wv; sq < ns; sq += K2_WAVES) {
       vec v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
       const int x1 = A.sl[s0 + sq + 1];
       int x = A.sl[s0 + sq];
-      for (; x + 4 <= x1; x += 4) {
+      for (; x < x1; x += 4) {  // lists come in fours, padded with zero weights
         vec tv[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) tv[u] = *reinterpret_cast<const vec *>(pt + (size_t)A.lt[x + u] * TILE2);
+        for (int u = 0; u < 4; ++u) tv[u] = *reinterpret_cast<const vec *>(pt + (unsigned)(A.lt[x + u] * TILE2) + lane * 4);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           v0 += A.ltv[2 * (x + u)] * tv[u];
-          v1 += A.ltv[2 * (x + u) + 1] * tv[u];
+          v1 -= A.ltv[2 * (x + u) + 1] * tv[u];
         }
       }
-      for (; x < x1; ++x) {
-        const vec ta = *reinterpret_cast<const vec *>(pt + (size_t)A.lt[x] * TILE2);
-        v0 += A.ltv[2 * x] * ta;
-        v1 += A.ltv[2 * x + 1] * ta;
-      }
-      *reinterpret_cast<vec *>(V + (size_t)(2 * sq) * TILE2 + lane * 4) = v0;
-      *reinterpret_cast<vec *>(V + (size_t)(2 * sq + 1) * TILE2 + lane * 4) = v1;
+      acc_t hh = {0, 0, 0, 0};
+#pragma unroll
+      for (int s = 0; s < 4; ++s) hh = MM::step(v0[s], b0[s], hh);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) hh = MM::step(v1[s], b2[s], hh);
+      if constexpr (sizeof(T) == 4) hh *= rho;
+      h_store<T>(Hs + sq * TILE2, lane, hh);
     }
+    const vec a0 = *reinterpret_cast<const vec *>(te + lane * 4);
+    const vec a2 = *reinterpret_cast<const vec *>(te + TILE2 + lane * 4);
     __syncthreads();
-    const int *jo = A.jto + A.gjt[gi];
+    const int y1 = A.jo[gi * K2_WAVES + wv + 1];
+    const int y = A.jo[gi * K2_WAVES + wv];
+    if (y == y1) continue;
+    // the wave's rows, 1 to 3: one instantiation each, so no idle row is summed
+    auto rows = [&](auto count) {
+      constexpr int N = decltype(count)::value;
+      vec g0[N], g1[N];
 #pragma unroll
-    for (int r = 0; r < JPW; ++r) {
-      const int q = wv + NW * r;
-      if (q >= nr) break;
-      const int y0 = jo[q], y1 = jo[q + 1];
-      if (y0 == y1) continue;
-      T r00[4] = {0, 0, 0, 0}, r02[4] = {0, 0, 0, 0}, r20[4] = {0, 0, 0, 0}, r22[4] = {0, 0, 0, 0};
-      for (int y = y0; y < y1; ++y) {
-        const int slq = A.jts[y];
-        const T c0 = A.jtc[2 * y], c1 = A.jtc[2 * y + 1];
-        const vec V0 = *reinterpret_cast<const vec *>(V + (size_t)(2 * slq) * TILE2 + lane * 4);
-        const vec V1 = *reinterpret_cast<const vec *>(V + (size_t)(2 * slq + 1) * TILE2 + lane * 4);
+      for (int r = 0; r < N; ++r) g0[r] = g1[r] = vec{0, 0, 0, 0};
+      for (int q = y; q < y1; q += 2) {  // lists come in twos
+        vec hv[2];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          r00[s] += c0 * V0[s];
-          r02[s] -= c0 * V1[s];
-          r20[s] -= c1 * V0[s];
-          r22[s] += c1 * V1[s];
+        for (int u = 0; u < 2; ++u) hv[u] = h_load<T>(Hs + A.js[q + u] * TILE2, lane);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const T *cf = A.jtc + 2 * K2_ROWS * (q + u);
+#pragma unroll
+          for (int r = 0; r < N; ++r) {
+            g0[r] += cf[2 * r] * hv[u];
+            g1[r] += cf[2 * r + 1] * hv[u];
+          }
         }
       }
-      acc_t ya = {0, 0, 0, 0}, yb = {0, 0, 0, 0};
-      mma_pair<T>(r00, r20, b0, ya, yb);
-      mma_pair<T>(r02, r22, b2, ya, yb);
 #pragma unroll
-      for (int s = 0; s < 4; ++s) acc[r] = MM::step(a0[s], ya[s], acc[r]);  // acc += i0 ya
+      for (int r = 0; r < N; ++r) {
+        acc_t x = {0, 0, 0, 0};
+        if constexpr (sizeof(T) == 8) x = acc[r];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) acc[r] = MM::step(a2[s], yb[s], acc[r]);  // acc += i2 yb
-    }
+        for (int s = 0; s < 4; ++s) x = MM::step(a0[s], g0[r][s], x);  // += i0 G0
+#pragma unroll
+        for (int s = 0; s < 4; ++s) x = MM::step(a2[s], g1[r][s], x);  // += i2 G1
+        if constexpr (sizeof(T) == 8)
+          acc[r] = x;
+        else
+#pragma unroll
+          for (int s = 0; s < 4; ++s) acc[r][s] += (double)x[s];
+      }
+    };
+    if (nrow == 3)
+      rows(std::integral_constant<int, 3>());
+    else if (nrow == 2)
+      rows(std::integral_constant<int, 2>());
+    else
+      rows(std::integral_constant<int, 1>());
   }
   // the owned rows' tiles (lane holds entry (row(g,s), c)) and their mirrors
   const int ni = A.ni[e], nj = A.ni[f], fi = A.first[e], fj = A.first[f];
@@ -737,29 +777,28 @@ __global__ void __launch_bounds__(K2_THREADS) k_dia_k2_off(DK2Args<T> A) {
   const long long col = pure_row(A.skip, A.poff, k, fj + min(b, nj - 1));
   const bool scol = (b == 0 && f > 0) || (b == nj - 1 && f + 1 < A.Nel);
 #pragma unroll
-  for (int r = 0; r < JPW; ++r) {
-    const int q = wv + NW * r;
-    if (q >= nr) break;
-    const acc_t v = acc[r];
-    const int j = A.jshell[r0 + q];
+  for (int r = 0; r < K2_ROWS; ++r) {
+    const int j = wrow[r];
+    if (j < 0) break;
+    const v4d v = acc[r];
 #pragma unroll
     for (int rr = 0; rr < 4; ++rr) {
-      const int a = kk[rr];
+      const int a = MM::row(g, rr);
       if (a >= ni || b >= nj || col < 0) continue;
       const long long row = pure_row(A.skip, A.poff, j, fi + a);
       if (row < 0) continue;
       const bool srow = (a == 0 && e > 0) || (a == ni - 1 && e + 1 < A.Nel);
       double *dst = A.K + row + col * A.ldk;
       if (srow || scol)
-        atomicAdd(dst, -(double)v[rr]);
+        atomicAdd(dst, -v[rr]);
       else
-        *dst = -(double)v[rr];
+        *dst = -v[rr];
       if (A.sym) {
         double *mdst = A.K + col + row * A.ldk;
         if (srow || scol)
-          atomicAdd(mdst, -(double)v[rr]);
+          atomicAdd(mdst, -v[rr]);
         else
-          *mdst = -(double)v[rr];
+          *mdst = -v[rr];
       }
     }
   }
@@ -1263,14 +1302,17 @@ void launch_dia_k(int part, bool tiled, int64_t grid, hipStream_t s, const DKArg
 }
 
 // FP32 copy of the P/Q tiles with P kinds divided and Q kinds multiplied by
-// exp(lsig) of their (ilm, element).
-__global__ void k_scale_pq_f32(const double *pq, const double *lsig, float *pq32, int n_x) {
+// exp(lsig) of their (ilm, element), in storage and in operand order.
+__global__ void k_scale_pq_f32(const double *pq, const double *lsig, float *pq32, float *pqo32, int n_x) {
   const int x = blockIdx.x;
   if (x >= n_x) return;
   const double up = exp(-lsig[x]), dn = exp(lsig[x]);
   for (int u = threadIdx.x; u < 4 * TILE2; u += NT) {
-    const int kind = u / TILE2;
-    pq32[(size_t)x * 4 * TILE2 + u] = (float)(pq[(size_t)x * 4 * TILE2 + u] * (kind < 2 ? up : dn));
+    const int kind = u / TILE2, lane = (u & 255) >> 2;
+    const size_t o = ((size_t)x * 4 + kind) * TILE2;
+    const double f = kind < 2 ? up : dn;
+    pq32[(size_t)x * 4 * TILE2 + u] = (float)(pq[(size_t)x * 4 * TILE2 + u] * f);
+    pqo32[o + (u & 255)] = (float)(pq[o + (lane & 15) + TILE * Mma<float>::row(lane >> 4, u & 3)] * f);
   }
 }
 }  // namespace
@@ -1282,10 +1324,12 @@ void diatomic_exchange_kernels(DiatomicDevice &d, const double *P, int64_t ldp, 
   if (fp32) {
     if (!d.f32_tables) {
       d.pq32.alloc(d.pq.n);
+      d.pqo32.alloc(d.pq.n);
       d.chol32.alloc(d.chol.n);
       d.sigma32.alloc(d.sigma.n);
       const int n_x = (int)(d.pq.n / (4 * TILE2));
-      hipLaunchKernelGGL(k_scale_pq_f32, dim3(n_x), dim3(NT), 0, s, d.pq.p, d.lsig.p, d.pq32.p, n_x);
+      hipLaunchKernelGGL(k_scale_pq_f32, dim3(n_x), dim3(NT), 0, s, d.pq.p, d.lsig.p, d.pq32.p, d.pqo32.p,
+                         n_x);
       hip_check(hipGetLastError(), "scale_pq_f32");
       to_f32_launch(d.chol.p, d.chol32.p, d.chol.n, s);
       to_f32_launch(d.sigma.p, d.sigma32.p, d.sigma.n, s);
@@ -1294,6 +1338,12 @@ void diatomic_exchange_kernels(DiatomicDevice &d, const double *P, int64_t ldp, 
     if (d.term_f32_gen != d.list_gen) {
       d.term_f32.alloc(d.term_f.n);
       to_f32_launch(d.term_f.p, d.term_f32.p, d.term_f.n, s);
+      if (d.k2) {
+        d.k2_ltv32.alloc(d.k2_ltv.n);
+        d.k2_jtc32.alloc(d.k2_jtc.n);
+        to_f32_launch(d.k2_ltv.p, d.k2_ltv32.p, d.k2_ltv.n, s);
+        to_f32_launch(d.k2_jtc.p, d.k2_jtc32.p, d.k2_jtc.n, s);
+      }
       d.term_f32_gen = d.list_gen;
     }
     if (!d.tiled) {
@@ -1372,13 +1422,20 @@ void diatomic_exchange_kernels(DiatomicDevice &d, const double *P, int64_t ldp, 
       hip_check(hipGetLastError(), "diatomic_kin_lds");
       continue;
     }
-    if (part == 0 && d.k2 && !fp32) {
+    if (part == 0 && d.k2) {
       TimedLaunch tl(timer, name, s, d.flops_off_k2);
-      DK2Args<double> a{d.ptile.p, d.n_src, K, ldk, d.Nel, d.Nang, d.first.p, d.ni.p, d.skip.p, d.poff.p, d.pq.p,
-                        d.k2_wg.p, d.k2_kshell.p, d.k2_kj.p, d.k2_jshell.p, d.k2_kg.p, d.k2_gilm.p, d.k2_gslot.p,
-                        d.k2_gjt.p, d.k2_sl.p, d.k2_lt.p, d.k2_jto.p, d.k2_jts.p, d.k2_ltv.p, d.k2_jtc.p,
-                        (int)d.sym};
-      hipLaunchKernelGGL((k_dia_k2_off<double>), dim3(d.n_wg_k2), dim3(K2_THREADS), 0, s, a);
+      if (fp32) {
+        DK2Args<float> a{d.ptile32.p, d.n_src, K, ldk, d.Nel, d.Nang, d.first.p, d.ni.p, d.skip.p, d.poff.p,
+                         d.pqo32.p, d.lsig.p, d.k2_wg.p, d.k2_kshell.p, d.k2_rows.p, d.k2_kg.p, d.k2_gilm.p,
+                         d.k2_gslot.p, d.k2_sl.p, d.k2_lt.p, d.k2_jo.p, d.k2_js.p, d.k2_ltv32.p, d.k2_jtc32.p,
+                         (int)d.sym};
+        hipLaunchKernelGGL((k_dia_k2_off<float>), dim3(d.n_wg_k2), dim3(K2_THREADS), 0, s, a);
+      } else {
+        DK2Args<double> a{d.ptile.p, d.n_src, K, ldk, d.Nel, d.Nang, d.first.p, d.ni.p, d.skip.p, d.poff.p, d.pqo.p,
+                          nullptr, d.k2_wg.p, d.k2_kshell.p, d.k2_rows.p, d.k2_kg.p, d.k2_gilm.p, d.k2_gslot.p,
+                          d.k2_sl.p, d.k2_lt.p, d.k2_jo.p, d.k2_js.p, d.k2_ltv.p, d.k2_jtc.p, (int)d.sym};
+        hipLaunchKernelGGL((k_dia_k2_off<double>), dim3(d.n_wg_k2), dim3(K2_THREADS), 0, s, a);
+      }
       hip_check(hipGetLastError(), "diatomic_k2_off");
       continue;
     }

@@ -22,12 +22,12 @@ constexpr int KL_RANK_MAX = 32;
 // runs per workgroup of that kernel
 constexpr int KL_BATCH = 64;
 // two-step cross-element diatomic exchange: slot tiles per (L,|M|) group in
-// LDS, rows per column shell (three per wave), threads per workgroup
+// LDS, threads per workgroup, rows per wave
 #ifndef HFG_K2_THREADS
 #define HFG_K2_THREADS 512
 #endif
-constexpr int K2_SLOTS = 17, K2_JMAX = 24, K2_THREADS = HFG_K2_THREADS;
-static_assert(K2_THREADS % 64 == 0 && K2_JMAX % (K2_THREADS / 64) == 0, "rows split evenly over the waves");
+constexpr int K2_SLOTS = 32, K2_THREADS = HFG_K2_THREADS, K2_WAVES = K2_THREADS / 64, K2_ROWS = 3;
+static_assert(K2_THREADS % 64 == 0 && K2_THREADS <= 1024, "two-step exchange workgroup");
 
 struct Error : std::runtime_error {
   int code;
@@ -314,19 +314,24 @@ struct DiatomicDevice {
   bool f32_tables = false;
   int64_t list_gen = 0, term_f32_gen = -1; // exchange-list version, and the one term_f32 holds
   int n_wg_in = 0;
-  // Cross-element exchange in two steps (k_dia_k2_off), used when every
-  // column block has at most K2_JMAX coupled rows and every group at most
-  // K2_SLOTS slots: one workgroup per (column shell k, element pair); per
-  // coupled ((L,|M|), parity of l_i) group of k, slot tiles V_b(i) = sum_l
-  // v_b(k,l) P(i,l) (b: mod / plain Gaunt channel) in LDS, then each row j's
-  // four channel tiles R = fac sum_i u(j,i) (x) V(i) and its radial products.
+  // Cross-element exchange in two steps (k_dia_k2_off), used with the tiled
+  // density: one workgroup per (column shell k with up to K2_WAVES x K2_ROWS
+  // of its rows, element pair); per coupled (L,|M|) group of k, at most
+  // K2_SLOTS slot tiles H(i) = V0(i) j0' - V1(i) j2', V_b(i) = sum_l v_b(k,l)
+  // P(i,l) (b: mod / plain Gaunt channel), in LDS, then each row j's sums
+  // G_b = fac sum_i u_b(j,i) H(i) and K += i0 G_0 - i2 G_1.
   bool k2 = false;
+  bool finite = true;                // the lists' density has no infinite or NaN block norm
   int n_wg_k2 = 0;
-  DevArray<int> k2_wg;                    // per workgroup: (k index, element pair) or (-1, -1)
-  DevArray<int> k2_kshell, k2_kj, k2_jshell, k2_kg;  // per k: shell, rows (offsets + shells), groups
-  DevArray<int> k2_gilm, k2_gslot, k2_gjt;           // per group: ilm, slot range, offset into k2_jto
-  DevArray<int> k2_sl, k2_lt, k2_jto, k2_jts;        // slot lt ranges; lt tile ids; per (group,row) jt ranges; jt slots
-  DevArray<double> k2_ltv, k2_jtc;                   // (v0, v1) per lt; (fac u0, fac u1) per jt
+  DevArray<int> k2_wg;               // per workgroup: (k index, element pair) or (-1, -1)
+  DevArray<int> k2_kshell, k2_rows;  // per k index: shell; K2_WAVES x K2_ROWS row shells (-1: none)
+  DevArray<int> k2_kg, k2_gilm, k2_gslot;  // per k index: groups; per group: ilm, slot range
+  DevArray<int> k2_sl, k2_lt;        // per slot: lt range; per lt: tile id
+  DevArray<int> k2_jo, k2_js;        // per (group, wave): jt range; per jt: slot
+  DevArray<double> k2_ltv, k2_jtc;   // (v0, v1) per lt; K2_ROWS x (fac u0, -fac u1) per jt
+  DevArray<float> k2_ltv32, k2_jtc32;  // FP32 copies (with list_gen as term_f32)
+  DevArray<double> pqo;              // pq in matrix-core operand order: lane (g,c) holds X(c, row(g,s)) in entry s
+  DevArray<float> pqo32;
   double flops_off_k2 = 0.0;
 };
 
