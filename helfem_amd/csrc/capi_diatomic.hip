@@ -2,6 +2,7 @@
 // the coupling lists of the Coulomb and exchange kernels (diatomic_jk.hip).
 #include "capi_common.hpp"
 #include <array>
+#include <tuple>
 #include <cstring>
 #include <cstdlib>
 #include <cmath>
@@ -148,12 +149,6 @@ void diatomic_upload(hf_diatomic *h) {
   if (ch.empty()) ch.push_back(0.0);
   if (sg.empty()) sg.push_back(0.0);
   d.pq.upload(pq, s);
-  std::vector<double> pqo(pq.size());
-  for (size_t x = 0; x < pq.size() / TILE2; ++x)
-    for (int lane = 0; lane < 64; ++lane)
-      for (int u = 0; u < 4; ++u)
-        pqo[x * TILE2 + lane * 4 + u] = pq[x * TILE2 + (lane & 15) + TILE * ((lane >> 4) + 4 * u)];
-  d.pqo.upload(pqo, s);
   // log scale per (L,|M|, element) that brings the P and Q tiles to the same
   // magnitude, sqrt(max|P| max|Q|): P_L(cosh mu) reaches 1e75 and Q_L 1e-56
   // at L = 34, outside FP32, while their products across elements are O(1)
@@ -310,7 +305,7 @@ void diatomic_upload(hf_diatomic *h) {
   d.preB.alloc((size_t)std::max(nLM, 1) * Nel);
   hip_check(hipStreamSynchronize(s), "upload sync");
   diatomic_build_operator(S, d, s);
-  diatomic_op_build(d, s);
+  d.op_ready = false;
   h->uploaded = true;
 }
 
@@ -631,6 +626,128 @@ void build_twostep(hf_diatomic *h, const std::vector<std::vector<int>> &rows,
   d.k2 = true;
 }
 
+// Lists of the folded-operator in-element exchange (k_dia_kin_fold) from the
+// groups of every column shell: the rows of a group go in units of two, which
+// share the group's slots, the units of one (L,|M|) in workgroups of
+// KF_WAVES per element.  In the symmetric mode only the rows j <= k.
+void build_fold(hf_diatomic *h, const std::vector<std::vector<int>> &rows,
+                const std::vector<std::vector<CoupleGroup>> &groups, hipStream_t s) {
+  const DiatomicSetup &S = h->host;
+  DiatomicDevice &d = h->dev;
+  const int Na = S.Nang(), Nel = S.Nel(), nlm = d.n_lm;
+  d.n_wg_kf = 0;
+  if (!d.fold_in || !d.tiled || !d.finite || d.dense_in) return;
+  struct Unit {
+    int jk[KF_ROWS];
+    std::vector<int4> rec;
+    std::vector<std::array<double, 2 * KF_ROWS>> u;
+  };
+  std::vector<std::vector<Unit>> units(nlm);
+  std::vector<int4> more;
+  std::vector<double> v;
+  double f_gather = 0.0;
+  std::vector<double> f_op(Nel);
+  for (int e = 0; e < Nel; ++e) {
+    const double n = S.rad.ni[e], ns = n * (n + 1) / 2, na = n * (n - 1) / 2;
+    f_op[e] = 2.0 * (ns * (2 * ns + n * n) + na * (2 * na + n * n));
+  }
+  double n_rows = 0.0;
+  for (int k = 0; k < Na; ++k) {
+    std::map<std::vector<double>, int> runs;  // weight runs of this column
+    for (const CoupleGroup &G : groups[k]) {
+      std::vector<int> rr;
+      for (size_t q = 0; q < rows[k].size(); ++q)
+        if (!G.jt[q].empty() && (!d.sym || rows[k][q] <= k)) rr.push_back((int)q);
+      std::vector<int4> rec(G.slots.size(), make_int4(-1, 0, 0, -1));
+      auto record = [&](int z) {
+        if (rec[z].x >= 0) return rec[z];
+        // runs of consecutive tiles, the later ones chained
+        std::vector<int4> parts;
+        const auto &lt = G.lt[z];
+        for (size_t a = 0; a < lt.size();) {
+          size_t b = a + 1;
+          while (b < lt.size() && lt[b].first == lt[b - 1].first + 1) ++b;
+          std::vector<double> w;
+          for (size_t x = a; x < b; ++x) {
+            w.push_back(lt[x].second.first);
+            w.push_back(lt[x].second.second);
+          }
+          const auto ins = runs.emplace(w, (int)v.size() / 2);
+          if (ins.second) {
+            v.insert(v.end(), w.begin(), w.end());
+            while (v.size() % 8) v.push_back(0.0);
+          }
+          parts.push_back(make_int4(lt[a].first, (int)(b - a), ins.first->second, -1));
+          a = b;
+        }
+        for (size_t x = parts.size() - 1; x > 0; --x) {
+          parts[x - 1].w = (int)more.size();
+          more.push_back(parts[x]);
+        }
+        return rec[z] = parts[0];
+      };
+      for (size_t a = 0; a < rr.size(); a += KF_ROWS) {
+        Unit U;
+        std::map<int, std::array<double, 2 * KF_ROWS>> co;
+        for (int r = 0; r < KF_ROWS; ++r) {
+          const bool have = a + r < rr.size();
+          U.jk[r] = have ? rows[k][rr[a + r]] * Na + k : -1;
+          if (!have) continue;
+          n_rows += 1.0;
+          for (const auto &e : G.jt[rr[a + r]]) {
+            auto &q = co.emplace(e.first, std::array<double, 2 * KF_ROWS>{}).first->second;
+            q[2 * r] = e.second.first;
+            q[2 * r + 1] = e.second.second;
+            f_gather += 8.0;
+          }
+        }
+        for (const auto &x : co) {
+          U.rec.push_back(record(x.first));
+          U.u.push_back(x.second);
+          f_gather += 4.0 * (double)G.lt[x.first].size();
+        }
+        units[G.ilm].push_back(std::move(U));
+      }
+    }
+  }
+  std::vector<int> jk, ent(1, 0);
+  std::vector<int4> rec;
+  std::vector<double> u;
+  // workgroups: element e's on XCD e % 8, (L,|M|) by (L,|M|), so the
+  // workgroups of one operator run together and share it in that XCD's L2
+  std::vector<std::vector<int4>> per_xcd(8);
+  for (int q = 0; q < nlm; ++q) {
+    const int u0 = (int)jk.size() / KF_ROWS, nu = (int)units[q].size();
+    for (const Unit &U : units[q]) {
+      jk.insert(jk.end(), U.jk, U.jk + KF_ROWS);
+      rec.insert(rec.end(), U.rec.begin(), U.rec.end());
+      for (const auto &c : U.u) u.insert(u.end(), c.begin(), c.end());
+      ent.push_back((int)rec.size());
+    }
+    for (int e = 0; e < Nel; ++e)
+      for (int b = 0; b < nu; b += KF_WAVES)
+        per_xcd[e % 8].push_back(make_int4(q, e, u0 + b, std::min(KF_WAVES, nu - b)));
+  }
+  if (rec.empty()) return;
+  size_t mx = 0;
+  for (auto &x : per_xcd) mx = std::max(mx, x.size());
+  std::vector<int4> wg(mx * 8, make_int4(-1, 0, 0, 0));
+  for (int x = 0; x < 8; ++x)
+    for (size_t q = 0; q < per_xcd[x].size(); ++q) wg[q * 8 + x] = per_xcd[x][q];
+  if (more.empty()) more.push_back(make_int4(0, 0, 0, -1));
+  d.wg_kf.upload(wg, s);
+  d.kf_jk.upload(jk, s);
+  d.kf_ent.upload(ent, s);
+  d.kf_rec.upload(rec, s);
+  d.kf_more.upload(more, s);
+  d.kf_u.upload(u, s);
+  d.kf_v.upload(v, s);
+  hip_check(hipStreamSynchronize(s), "folded exchange list upload");  // before the host lists go
+  d.flops_in_kf = 0.0;
+  for (int e = 0; e < Nel; ++e) d.flops_in_kf += n_rows * f_op[e] + f_gather * S.rad.ni[e] * S.rad.ni[e];
+  d.n_wg_kf = (int)wg.size();
+}
+
 // Exchange coupling lists for the density blocks that pass the norm screen
 // (|P_il|_F >= 10 eps, basis.cpp:1858-1875).  For each output block (j,k):
 // runs of terms per (L,|M|), each term a density block (i,l) with
@@ -660,6 +777,12 @@ void build_exchange_lists(hf_diatomic *h, hipStream_t s) {
   for (size_t q = 0; q < mask.size(); ++q) finite = finite && d.h_bnorm.p[q] < 1e30;
   if (!d.screen_mask.empty() && mask == d.screen_mask && d.sym == d.list_sym && finite == d.finite) return;
   d.finite = finite;
+  d.screen_mask.clear();  // no lists until all of them are there
+  auto done = [&] {
+    d.screen_mask = mask;
+    d.list_sym = d.sym;
+    ++d.list_gen;
+  };
   int mabs = 0;
   for (int m : mv) mabs = std::max(mabs, std::abs(m));
   const int dmoff = 2 * mabs;
@@ -676,11 +799,88 @@ void build_exchange_lists(hf_diatomic *h, hipStream_t s) {
       ilm_of[(size_t)e.first * Mext + e.second + dmoff] = S.lmind(e.first, e.second);
       fac_of[(size_t)e.first * Mext + e.second + dmoff] = S.LMfac(e.first, e.second);
     }
+  // density tiles of the coupled blocks: by row shell, then m, parity and l of
+  // the column shell, so the sources of one slot are consecutive tiles
+  std::vector<int> id((size_t)Na * Na, -1), src;
+  for (const auto &v : bydm) src.insert(src.end(), v.begin(), v.end());
+  std::sort(src.begin(), src.end(), [&](int x, int y) {
+    const int i = x / Na, j = y / Na, a = x % Na, b = y % Na;
+    return std::make_tuple(i, mv[a], lv[a] & 1, lv[a], a) < std::make_tuple(j, mv[b], lv[b] & 1, lv[b], b);
+  });
+  for (size_t q = 0; q < src.size(); ++q) id[src[q]] = (int)q;
+  const double bytes = (double)src.size() * S.Nel() * S.Nel() * TILE2 * sizeof(double);
+  d.tiled = bytes <= exchange_tile_budget(d.ptile.n * sizeof(double) + d.ptile32.n * sizeof(float));
+  d.n_src = (int)src.size();
+  if (src.empty()) src.push_back(0);
+  d.src_blk.upload(src, s);
+  hip_check(hipStreamSynchronize(s), "exchange source upload");
+  // factorised couplings of every output block that m allows; those with any
+  // are the active ones
+  const int njk = Na * Na;
+  std::vector<int> act;
+  {
+    std::vector<std::vector<int>> rows(Na);  // of every column shell k
+    for (int k = 0; k < Na; ++k)
+      for (int j = 0; j < Na; ++j) {
+        if (h->absm && (mv[j] < 0 || mv[k] < 0)) continue;
+        const int dm = mv[j] - mv[k];
+        if (std::abs(dm) <= 2 * mabs && !bydm[dm + dmoff].empty()) rows[k].push_back(j);
+      }
+    const auto groups = couple_groups(h, rows, id, mask, ilm_of, fac_of, Mext, dmoff);
+    // work: radial flops per (block, (L,|M|)) run, 4 channels x 2 flops per term
+    // and tile entry for the Gaunt-weighted density sums
+    double frad_in = 0.0, frad_off = 0.0;
+    int64_t nterm = 0, nterm_in = 0, nrun = 0;
+    std::vector<unsigned char> active(njk, 0);
+    for (int k = 0; k < Na; ++k) {
+      std::vector<int> last(rows[k].size(), -1);
+      for (const CoupleGroup &G : groups[k])
+        for (size_t q = 0; q < rows[k].size(); ++q) {
+          if (G.jt[q].empty()) continue;
+          const bool in_done = !d.sym || rows[k][q] <= k;
+          int64_t n = 0;
+          for (const auto &e : G.jt[q]) n += (int64_t)G.lt[e.first].size();
+          nterm += n;
+          if (in_done) nterm_in += n;
+          if (last[q] != G.ilm) {
+            last[q] = G.ilm;
+            ++nrun;
+            if (in_done) frad_in += d.h_rad_in[G.ilm];
+            frad_off += d.sym ? d.h_rad_low[G.ilm] : d.h_rad_off[G.ilm];
+          }
+          active[rows[k][q] * Na + k] = 1;
+        }
+    }
+    for (int jk = 0; jk < njk; ++jk)
+      if (active[jk]) act.push_back(jk);
+    d.n_act = (int)act.size();
+    d.n_runs = nrun;
+    d.n_terms = nterm;
+    double sum_in = 0.0, sum_off = 0.0;
+    for (int e = 0; e < S.Nel(); ++e) {
+      sum_in += (double)S.rad.ni[e] * S.rad.ni[e];
+      for (int f = 0; f < S.Nel(); ++f)
+        if (d.sym ? e > f : e != f) sum_off += (double)S.rad.ni[e] * S.rad.ni[f];
+    }
+    d.flops_in = frad_in + 8.0 * (double)nterm_in * sum_in;
+    d.flops_off = frad_off + 8.0 * (double)nterm * sum_off;
+    d.flops_k_angular = 8.0 * ((double)nterm_in * sum_in + (double)nterm * sum_off);
+    d.flops_k_radial = frad_in + frad_off;
+    build_twostep(h, rows, groups, s);
+    build_fold(h, rows, groups, s);
+  }
+  // the lists of every single term only for the kernels that read them (N2:
+  // 3.8 M terms, 0.2 GB): the one-step, Cholesky-form and dense ones
+  d.n_wg_kl = 0;
+  d.n_wg_op = 0;
+  if (act.empty() || ((S.Nel() < 2 || d.k2) && d.n_wg_kf > 0)) {
+    done();
+    return;
+  }
   struct Term {
     int ilm, il;
     double f[4];
   };
-  const int njk = Na * Na;
   std::vector<std::vector<Term>> per(njk);
 #pragma omp parallel for schedule(dynamic, 4)
   for (int jk = 0; jk < njk; ++jk) {
@@ -708,16 +908,12 @@ void build_exchange_lists(hf_diatomic *h, hipStream_t s) {
     }
     std::stable_sort(out.begin(), out.end(), [](const Term &a, const Term &b) { return a.ilm < b.ilm; });
   }
-  std::vector<int> act, lstart(1, 0), rilm, rstart(1, 0), til;
+  std::vector<int> lstart(1, 0), rilm, rstart(1, 0), til;
   std::vector<double> tf;
-  // flops as executed: in the symmetric mode the cross-element launch covers
-  // the pairs e > f and the in-element one the blocks j <= k
-  double frad_in = 0.0, frad_off = 0.0;
-  int64_t nterm = 0, nterm_in = 0;
+  act.clear();
   for (int jk = 0; jk < njk; ++jk) {
     const std::vector<Term> &v = per[jk];
     if (v.empty()) continue;
-    const bool in_done = !d.sym || jk / Na <= jk % Na;
     act.push_back(jk);
     for (size_t a = 0; a < v.size();) {
       size_t b = a;
@@ -728,28 +924,12 @@ void build_exchange_lists(hf_diatomic *h, hipStream_t s) {
       }
       rilm.push_back(v[a].ilm);
       rstart.push_back((int)til.size());
-      if (in_done) frad_in += d.h_rad_in[v[a].ilm];
-      frad_off += d.sym ? d.h_rad_low[v[a].ilm] : d.h_rad_off[v[a].ilm];
       a = b;
     }
     lstart.push_back((int)rilm.size());
-    nterm += (int64_t)v.size();
-    if (in_done) nterm_in += (int64_t)v.size();
   }
   d.n_act = (int)act.size();
   d.n_runs = (int64_t)rilm.size();
-  d.n_terms = nterm;
-  // Gaunt-weighted density sums: 4 channels x 2 flops per term and tile entry
-  double sum_in = 0.0, sum_off = 0.0;
-  for (int e = 0; e < S.Nel(); ++e) {
-    sum_in += (double)S.rad.ni[e] * S.rad.ni[e];
-    for (int f = 0; f < S.Nel(); ++f)
-      if (d.sym ? e > f : e != f) sum_off += (double)S.rad.ni[e] * S.rad.ni[f];
-  }
-  d.flops_in = frad_in + 8.0 * (double)nterm_in * sum_in;
-  d.flops_off = frad_off + 8.0 * (double)nterm * sum_off;
-  d.flops_k_angular = 8.0 * ((double)nterm_in * sum_in + (double)nterm * sum_off);
-  d.flops_k_radial = frad_in + frad_off;
   // dense in-element path: runs grouped by (L,|M|); one workgroup per
   // (ilm, element, 32 runs), groups dealt round-robin to the 8 XCDs so the
   // workgroups sharing one operator table run on the same L2
@@ -787,12 +967,12 @@ void build_exchange_lists(hf_diatomic *h, hipStream_t s) {
     // the dense operator replaces 12 r n^3 by 8 n^4 per (run, element)
     double fr = 0.0;
     for (int e = 0; e < Nel; ++e) fr += 8.0 * std::pow((double)S.rad.ni[e], 4);
-    d.flops_in = (double)d.n_runs * fr + 8.0 * (double)nterm * sum_in;
+    double sum_in = 0.0;
+    for (int e = 0; e < Nel; ++e) sum_in += (double)S.rad.ni[e] * S.rad.ni[e];
+    d.flops_in = (double)d.n_runs * fr + 8.0 * (double)d.n_terms * sum_in;
   }
   // in-element workgroups of the LDS-resident kernel: runs grouped by ilm,
   // batches of KL_BATCH per (ilm, element), element e's batches on XCD e % 8
-  d.n_wg_kl = 0;
-  d.n_wg_op = 0;
   if (!d.dense_in && d.max_rank <= KL_RANK_MAX && !rilm.empty()) {
     const int Nel = S.Nel(), nr = (int)rilm.size();
     std::vector<int> run_act(nr), cnt(nlm + 1, 0), runs;
@@ -860,39 +1040,18 @@ void build_exchange_lists(hf_diatomic *h, hipStream_t s) {
   d.lrun_ilm.upload(rilm, s);
   d.lrun_tstart.upload(rstart, s);
   d.term_il.upload(til, s);
-  {
-    std::vector<int4> tpos(til.size());
-    for (size_t q = 0; q < til.size(); ++q) {
-      const int i = til[q] / Na, l = til[q] % Na;
-      tpos[q] = make_int4((int)S.poff[i], (int)(S.poff[l] - S.skip(l)), S.skip(i), S.skip(l));
-    }
-    d.term_pos.upload(tpos, s);
+  std::vector<int4> tpos(til.size());
+  std::vector<int> tt(til.size());  // each term's tile
+  for (size_t q = 0; q < til.size(); ++q) {
+    const int i = til[q] / Na, l = til[q] % Na;
+    tpos[q] = make_int4((int)S.poff[i], (int)(S.poff[l] - S.skip(l)), S.skip(i), S.skip(l));
+    tt[q] = id[til[q]];
   }
-  {
-    // source blocks referenced by the terms, and each term's tile among them
-    std::vector<int> id((size_t)Na * Na, -1), src, tt(til.size());
-    for (size_t q = 0; q < til.size(); ++q) {
-      int &x = id[til[q]];
-      if (x < 0) {
-        x = (int)src.size();
-        src.push_back(til[q]);
-      }
-      tt[q] = x;
-    }
-    const double bytes = (double)src.size() * S.Nel() * S.Nel() * TILE2 * sizeof(double);
-    d.tiled = bytes <= exchange_tile_budget(d.ptile.n * sizeof(double) + d.ptile32.n * sizeof(float));
-    d.n_src = (int)src.size();
-    d.src_blk.upload(src, s);
-    d.term_tile.upload(tt, s);
-    std::vector<std::vector<int>> rows(Na);  // of every column shell k
-    for (int jk : act) rows[jk % Na].push_back(jk / Na);
-    build_twostep(h, rows, couple_groups(h, rows, id, mask, ilm_of, fac_of, Mext, dmoff), s);
-  }
+  d.term_pos.upload(tpos, s);
+  d.term_tile.upload(tt, s);
   d.term_f.upload(tf, s);
   hip_check(hipStreamSynchronize(s), "exchange list upload");
-  d.screen_mask = mask;
-  d.list_sym = d.sym;
-  ++d.list_gen;
+  done();
 }
 
 void ensure_ready(hf_diatomic *h) {
@@ -904,6 +1063,12 @@ void ensure_ready(hf_diatomic *h) {
 void exchange_launch(hf_diatomic *h, const double *P, int64_t ldp, double *K, int64_t ldk, bool fp32 = false) {
   DiatomicDevice &d = h->dev;
   hipStream_t s = h->ctx->cur;
+  if (!d.op_ready) {
+    // the in-element operators, before the first exchange of these tables
+    // (density-functional builds without exact exchange never need them)
+    diatomic_op_build(d, h->host.rad.ni, s);
+    d.op_ready = true;
+  }
   block_stats_launch(P, ldp, d.Nrad, d.Nang, d.skip.p, d.poff.p, d.stats.p, d.h_stats.p, s);
   hip_check(hipStreamSynchronize(s), "block statistics sync");
   const bool symmetric = block_stats_reduce(d.h_stats.p, d.Nrad, d.Nang, d.h_bnorm.p);

@@ -26,6 +26,7 @@
 // 16) stays in the L2 of the XCD that works on it.
 #include "hfgpu_internal.hpp"
 #include "device_common.hpp"
+#include <algorithm>
 #include <type_traits>
 
 // terms in flight per lane in the cross-element gathers, and that launch's
@@ -922,6 +923,358 @@ __global__ void __launch_bounds__(KL_THREADS) k_dia_kin_lds(DKLArgs<T> A) {
   }
 }
 
+// --- In-element exchange with folded dense operators ---------------------------
+//
+// For one ((L,|M|), element e) the in-element tile of every coupled output
+// block is Y(a,b) = sum_xy sum_cd W_xy(ca, bd) R_xy(c,d), x, y the two channels,
+// W = B diag(sigma) B' (basis.cpp:1992-2033 contracts the factor) and R_xy =
+// sum_i u_x(j,i) V_y(i) the Gaunt-weighted density sums.  W is symmetric under
+// c <-> a, under b <-> d and as a matrix, so with tau the transposition of a
+// tile the diagonal channels commute with tau and W_20 = tau W_02 tau: the
+// symmetric and antisymmetric parts of Y separate,
+//   Y_s (a <= b) = Ts [S_00; S_22; R_02 + R_20'],   S = R + R' (R on the diagonal)
+//   Y_a (a <  b) = Ta [A_00; A_22; R_02 - R_20'],   A = R - R'
+// 120 x 465 and 105 x 435 for 15 functions: 0.20 MFLOP per (block, element)
+// against 0.41 of the plain operators and 12 r n^3 = 1.2 of the Cholesky form
+// (rank r ~ 30).  k_dia_fold_build writes Ts, Ta once per basis in operand order
+// (row tile, four k-steps, lane, step).
+// k_dia_kin_fold: one 1024-thread workgroup per ((L,|M|), e, 16 units of two
+// rows), a GEMM with 32 columns.  Each wave gathers its unit's R tiles (the two
+// rows share the slots' V tiles), folds them in registers (lanes c <= d keep
+// the symmetric entries, the others the antisymmetric ones) and stores the
+// symmetric, then the antisymmetric columns in LDS (120 KB); the waves split
+// row tiles and, beyond those, the inner extent; the operator streams from L2
+// one quad of k-steps ahead.  Column c of inner index k sits at (c + k/2) & 15,
+// which keeps stores (many k, one column) and reads (four k, all columns) free
+// of bank conflicts.  The tiles are added to K atomically (boundary entries are
+// shared with the cross-element launch, the (L,|M|) of a block with other
+// workgroups).
+// N2 (lmax 16, 8 elements, 60 k rows x 8 elements): 4.0 ms against 13.0 of
+// k_dia_kin_lds, FP32 (lmax 12, 6 elements) 1.0 against 2.1; 1.5 ms of it the
+// matrix pipe's, the gathers 0.65, the output 0.55, the folding the rest (one
+// workgroup per CU, its phases one after another).
+
+struct DFoldBuildArgs {
+  const double *chol, *sigma;
+  const int *chol_off, *chol_rank, *ni;
+  int Nel;
+  size_t size;
+  double *T;  // [ilm*Nel + e][size]
+};
+
+// q-th pair a <= b (anti: a < b) in the order b (b + 1) / 2 + a (b (b - 1) / 2 + a)
+__device__ inline void fold_pair(int q, bool anti, int &a, int &b) {
+  b = anti ? 1 : 0;
+  for (int first = 0, w = 1; q >= first + w; ++b) {
+    first += w;
+    ++w;
+  }
+  a = q - (anti ? b * (b - 1) / 2 : b * (b + 1) / 2);
+}
+
+// Workgroups ((ilm, e), one of FB_PARTS shares of the row tiles); the channel
+// tiles sit in LDS when the rank allows (LDS), else they are read in place.
+// Bound by LDS reads (two per product and vector); N2: 1792 operators of 0.9 MB
+// in 3 ms (21 ms with the tiles read from L2).
+constexpr int FB_THREADS = 1024, FB_PARTS = 4;
+
+template <bool LDS>
+__global__ void __launch_bounds__(FB_THREADS) k_dia_fold_build(DFoldBuildArgs A) {
+  __shared__ double Ml[LDS ? KL_RANK_MAX * 2 * TILE2 : 1];
+  __shared__ double sgl[LDS ? KL_RANK_MAX : 1];
+  __shared__ int2 pairs[2][TILE * (TILE + 1) / 2];
+  const int x = blockIdx.y, e = x % A.Nel, n = A.ni[e];
+  const int rank = A.chol_rank[x], off = A.chol_off[x];
+  const double *Mg = A.chol + (size_t)off * 2 * TILE2, *sg = A.sigma + off;
+  if (LDS) {
+    for (int q = threadIdx.x; q < rank * 2 * TILE2; q += FB_THREADS) Ml[q] = Mg[q];
+    for (int q = threadIdx.x; q < rank; q += FB_THREADS) sgl[q] = sg[q];
+  }
+  for (int q = threadIdx.x; q < 2 * kf_pairs(n, false); q += FB_THREADS) {
+    const bool anti = q >= kf_pairs(n, false);
+    const int r = anti ? q - kf_pairs(n, false) : q;
+    int a, b;
+    if (!anti || r < kf_pairs(n, true)) {
+      fold_pair(r, anti, a, b);
+      pairs[anti][r] = make_int2(a, b);
+    }
+  }
+  __syncthreads();
+  const double *M = LDS ? Ml : Mg, *sv = LDS ? sgl : sg;
+  // sum_p sigma_p Mx(c,a) My(b,d) + sn sum_p sigma_p Mx(c2,a2) My(b2,d2)
+  auto two = [&](int cx, int cy, int o1, int o2, int o3, int o4, double sn) {
+    const double *p1 = M + cx * TILE2 + o1, *p2 = M + cy * TILE2 + o2, *p3 = M + cx * TILE2 + o3,
+                 *p4 = M + cy * TILE2 + o4;
+    double v = 0.0, w = 0.0;
+    for (int p = 0; p < rank; ++p) {
+      const int q = p * 2 * TILE2;
+      v += sv[p] * p1[q] * p2[q];
+      w += sv[p] * p3[q] * p4[q];
+    }
+    return v + sn * w;
+  };
+  auto at = [](int r, int c) { return r + TILE * c; };
+  const int rs = kf_tiles(n, false), ra = kf_tiles(n, true);
+  for (int tile = blockIdx.x; tile < rs + ra; tile += FB_PARTS) {
+    const bool anti = tile >= rs;
+    const int rt = anti ? tile - rs : tile;
+    const int np = kf_pairs(n, anti), K = kf_inner(n, anti);
+    const double sn = anti ? -1.0 : 1.0;
+    double *out = A.T + (size_t)x * A.size + (anti ? (size_t)16 * rs * kf_inner(n, false) : 0) + (size_t)16 * rt * K;
+    for (int q = threadIdx.x; q < 16 * K; q += FB_THREADS) {
+      const int quad = q >> 8, lane = (q >> 2) & 63, st = q & 3;
+      const int row = 16 * rt + (lane & 15), k = 16 * quad + 4 * st + (lane >> 4);
+      double v = 0.0;
+      if (row < np && k < 2 * np + n * n) {
+        const int a = pairs[anti][row].x, b = pairs[anti][row].y;
+        if (k < 2 * np) {
+          const int ch = k >= np;
+          const int c = pairs[anti][k - ch * np].x, d = pairs[anti][k - ch * np].y;
+          v = two(ch, ch, at(c, a), at(b, d), at(d, a), at(b, c), sn);
+          // c == d (symmetric half only): one entry, and both sums are it
+          v *= 0.5;
+        } else {
+          const int c = (k - 2 * np) % n, d = (k - 2 * np) / n;
+          v = 0.5 * two(0, 1, at(c, a), at(b, d), at(c, b), at(a, d), sn);
+        }
+      }
+      out[q] = v;
+    }
+  }
+}
+
+template <typename T>
+struct DFoldArgs {
+  double *K;
+  int64_t ldk;
+  int Nel, Nang;
+  const int *first, *ni, *skip;
+  const long long *poff;
+  const T *Top;
+  size_t size;
+  const int4 *wg;
+  const int *jk, *ent;
+  const int4 *rec, *more;
+  const T *u, *v;
+  const T *pt;  // tiled density
+  int n_src;
+  int sym;
+};
+
+// V0, V1 of one slot: sources in runs of consecutive tiles, four loads in
+// flight (a run's weights are padded with zeros; the padding rereads its last tile).
+template <typename T>
+__device__ inline void slot_sums(const T *pt, int4 r, const int4 *more, const T *v, int lane,
+                                 typename Mma<T>::acc_t &v0, typename Mma<T>::acc_t &v1) {
+  typedef typename Mma<T>::acc_t vec;
+  v0 = v1 = vec{0, 0, 0, 0};
+  for (;;) {
+    for (int x = 0; x < r.y; x += 4) {
+      vec tv[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        tv[u] = *reinterpret_cast<const vec *>(pt + (size_t)(r.x + min(x + u, r.y - 1)) * TILE2 + lane * 4);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        v0 += v[2 * (r.z + x + u)] * tv[u];
+        v1 += v[2 * (r.z + x + u) + 1] * tv[u];
+      }
+    }
+    if (r.w < 0) break;
+    r = more[r.w];
+  }
+}
+
+// One half (symmetric or antisymmetric) of the GEMM: the wave's row tile rt
+// over the quads [q0, q1) and both column tiles.
+template <typename T>
+__device__ inline void fold_gemm(const T *top, const T *X, int rt, int nq, int q0, int q1, int lane,
+                                 typename Mma<T>::acc_t acc[2]) {
+  typedef Mma<T> MM;
+  typedef typename MM::acc_t vec;
+  const int g = lane >> 4, c = lane & 15;
+  const T *tp = top + (size_t)rt * nq * 256 + lane * 4;
+  const T *Xg = X + g * 16;
+  vec cur = *reinterpret_cast<const vec *>(tp + (size_t)q0 * 256);
+  for (int q = q0; q < q1; ++q) {
+    const vec nxt = *reinterpret_cast<const vec *>(tp + (size_t)min(q + 1, q1 - 1) * 256);
+#pragma unroll
+    for (int st = 0; st < 4; ++st) {
+      const int k = 16 * q + 4 * st;  // + g
+      const int pos = k * 16 + ((c + ((k + g) >> 1)) & 15);
+      const T b0 = Xg[pos], b1 = Xg[nq * 256 + pos];
+      acc[0] = MM::step(cur[st], b0, acc[0]);
+      acc[1] = MM::step(cur[st], b1, acc[1]);
+    }
+    cur = nxt;
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(KF_THREADS) k_dia_kin_fold(DFoldArgs<T> A) {
+  typedef Mma<T> MM;
+  typedef typename MM::acc_t vec;
+  extern __shared__ char fold_lds[];
+  T *X = reinterpret_cast<T *>(fold_lds);
+  const int4 wg = A.wg[blockIdx.x];
+  const int ilm = wg.x, e = wg.y, u0 = wg.z, nu = wg.w;
+  if (ilm < 0) return;
+  const int t = threadIdx.x, lane = t & 63, g = lane >> 4, c = lane & 15;
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int n = A.ni[e], fe = A.first[e];
+  const int nS = kf_pairs(n, false), nA = kf_pairs(n, true);
+  const int qS = kf_inner(n, false) / 16, qA = kf_inner(n, true) / 16;
+  const int rS = kf_tiles(n, false), rA = kf_tiles(n, true);
+  int kk[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) kk[s] = MM::row(g, s);
+  // 1. the unit's tiles R_xy(c, kk) = sum u_x V_y of its two rows
+  vec r00[KF_ROWS], r02[KF_ROWS], r20[KF_ROWS], r22[KF_ROWS];
+#pragma unroll
+  for (int r = 0; r < KF_ROWS; ++r) r00[r] = r02[r] = r20[r] = r22[r] = vec{0, 0, 0, 0};
+  if (wv < nu) {
+    const T *pt = A.pt + (size_t)(e * A.Nel + e) * A.n_src * TILE2;
+    for (int q = A.ent[u0 + wv]; q < A.ent[u0 + wv + 1]; ++q) {
+      vec v0, v1;
+      slot_sums<T>(pt, A.rec[q], A.more, A.v, lane, v0, v1);
+#pragma unroll
+      for (int r = 0; r < KF_ROWS; ++r) {
+        const T c0 = A.u[2 * KF_ROWS * q + 2 * r], c1 = A.u[2 * KF_ROWS * q + 2 * r + 1];
+        r00[r] += c0 * v0;
+        r02[r] += c0 * v1;
+        r20[r] += c1 * v0;
+        r22[r] += c1 * v1;
+      }
+    }
+    // 2. fold: transposes through the wave's own 16 x 17 scratch
+    T *sc = X + wv * (TILE * 17);
+    auto transposed = [&](const vec &r) {
+      vec o;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) sc[kk[s] * 17 + c] = r[s];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int s = 0; s < 4; ++s) o[s] = sc[c * 17 + kk[s]];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      return o;
+    };
+#pragma unroll
+    for (int r = 0; r < KF_ROWS; ++r) {
+      const vec t00 = transposed(r00[r]), t22 = transposed(r22[r]), t20 = transposed(r20[r]);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        // c < kk: S(c, kk); c == kk: R; c > kk: A(kk, c)
+        const T d00 = c < kk[s] ? t00[s] : T(0), d22 = c < kk[s] ? t22[s] : T(0);
+        r00[r][s] = c > kk[s] ? t00[s] - r00[r][s] : r00[r][s] + d00;
+        r22[r][s] = c > kk[s] ? t22[s] - r22[r][s] : r22[r][s] + d22;
+        const T up = r02[r][s] + t20[s], um = r02[r][s] - t20[s];
+        r02[r][s] = up;
+        r20[r][s] = um;
+      }
+    }
+  }
+  __syncthreads();
+  // 3. columns of one half in LDS: X[column tile][k][16]
+  auto columns = [&](bool anti) {
+    const int np = anti ? nA : nS, nq = anti ? qA : qS;
+    if (wv < nu)
+#pragma unroll
+      for (int r = 0; r < KF_ROWS; ++r) {
+        const int col = KF_ROWS * wv + r, cc = col & 15;
+        T *Xc = X + (col >> 4) * nq * 256;
+        auto put = [&](int k, T x) { Xc[k * 16 + ((cc + (k >> 1)) & 15)] = x; };
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          if (c >= n || kk[s] >= n) continue;
+          const int lo = min(c, kk[s]), hi = max(c, kk[s]);
+          if (anti ? c > kk[s] : c <= kk[s]) {
+            const int p = (anti ? hi * (hi - 1) / 2 : hi * (hi + 1) / 2) + lo;
+            put(p, r00[r][s]);
+            put(np + p, r22[r][s]);
+          }
+          put(2 * np + c + n * kk[s], anti ? r20[r][s] : r02[r][s]);
+        }
+      }
+    // the padding of the inner extent meets zero operator entries: keep it finite
+    const int k0 = 2 * np + n * n;
+    for (int q = t; q < (16 * nq - k0) * 32; q += KF_THREADS)
+      X[(q & 1) * nq * 256 + (k0 + (q >> 5)) * 16 + ((q >> 1) & 15)] = T(0);
+  };
+  const T *top = A.Top + (size_t)(ilm * A.Nel + e) * A.size;
+  vec aS[2] = {vec{0, 0, 0, 0}, vec{0, 0, 0, 0}}, aA[2] = {vec{0, 0, 0, 0}, vec{0, 0, 0, 0}};
+  // waves: row tile, and a share of the inner extent
+  const int kS = KF_WAVES / rS, kA = rA > 0 ? KF_WAVES / rA : 1;
+  columns(false);
+  __syncthreads();
+  const int hS = wv / rS, hA = rA > 0 ? wv / rA : 1;
+  if (hS < kS) fold_gemm<T>(top, X, wv - hS * rS, qS, qS * hS / kS, qS * (hS + 1) / kS, lane, aS);
+  __syncthreads();
+  columns(true);
+  __syncthreads();
+  if (rA > 0 && hA < kA)
+    fold_gemm<T>(top + (size_t)16 * rS * 16 * qS, X, wv - hA * rA, qA, qA * hA / kA, qA * (hA + 1) / kA, lane, aA);
+  __syncthreads();
+  // 4. partial tiles to LDS (rows rotated as the columns above), then the
+  // blocks' entries: Y(a,b) = Y_s + Y_a, Y(b,a) = Y_s - Y_a
+  T *Ys = X, *Ya = X + kS * rS * 512;
+  auto partial = [&](T *Y, int h, int rt, int nr, const vec acc[2]) {
+#pragma unroll
+    for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int row = kk[s];
+        Y[((h * nr + rt) * 2 + ct) * 256 + row * 16 + ((c + (row >> 1)) & 15)] = acc[ct][s];
+      }
+  };
+  if (hS < kS) partial(Ys, hS, wv - hS * rS, rS, aS);
+  if (rA > 0 && hA < kA) partial(Ya, hA, wv - hA * rA, rA, aA);
+  __syncthreads();
+  // a wave adds its own rows' blocks; entry x = lo + n hi of the tile, four per
+  // lane, the same places for every row, written consecutively in lo both as
+  // K(j lo, k hi) and as the mirror K(k lo, j hi) = Y(hi, lo)
+  if (wv >= nu) return;
+  int lo[4], hi[4], ps[4], pa[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int x = min(lane + 64 * i, n * n - 1);
+    hi[i] = x / n;
+    lo[i] = lane + 64 * i < n * n ? x - hi[i] * n : -1;
+    const int mn = min(max(lo[i], 0), hi[i]), mx = max(lo[i], hi[i]);
+    const int p = mx * (mx + 1) / 2 + mn, q = max(mx * (mx - 1) / 2 + mn, 0);
+    ps[i] = ((p >> 4) * 512 + (p & 15) * 16) | ((p & 15) >> 1) << 24;  // offset of the row, rotation
+    pa[i] = mn == mx ? -1 : (((q >> 4) * 512 + (q & 15) * 16) | ((q & 15) >> 1) << 24);
+  }
+#pragma unroll
+  for (int r = 0; r < KF_ROWS; ++r) {
+    const int jk = A.jk[KF_ROWS * (u0 + wv) + r];
+    if (jk < 0) break;
+    const int j = jk / A.Nang, k = jk - j * A.Nang;
+    const int col = KF_ROWS * wv + r, ct = (col >> 4) * 256, cc = col & 15;
+    const int sj = A.skip[j], sk = A.skip[k];
+    const long long oj = A.poff[j] + fe - sj, ok = A.poff[k] + fe - sk;
+    const bool both = A.sym && j != k;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (lo[i] < 0) continue;
+      const int os = (ps[i] & 0xffffff) + ct + ((cc + (ps[i] >> 24)) & 15);
+      double vs = 0.0, va = 0.0;
+      for (int h = 0; h < kS; ++h) vs += (double)Ys[os + h * rS * 512];
+      if (pa[i] >= 0) {
+        const int oa = (pa[i] & 0xffffff) + ct + ((cc + (pa[i] >> 24)) & 15);
+        for (int h = 0; h < kA; ++h) va += (double)Ya[oa + h * rA * 512];
+      }
+      if (lo[i] > hi[i]) va = -va;  // Y(lo, hi) = Y_s + Y_a for lo < hi
+      if (fe + lo[i] >= sj && fe + hi[i] >= sk) atomicAdd(A.K + (oj + lo[i]) + (ok + hi[i]) * A.ldk, -(vs + va));
+      if (both && fe + lo[i] >= sk && fe + hi[i] >= sj)
+        atomicAdd(A.K + (ok + lo[i]) + (oj + hi[i]) * A.ldk, -(vs - va));
+    }
+  }
+}
+
 // --- In-element exchange as a dense operator on the matrix cores ---------------
 //
 // For one ((L,|M|), element e) every coupled output block's in-element tile
@@ -1202,24 +1555,58 @@ __global__ void __launch_bounds__(NT) k_dia_mirror(double *K, int64_t ldk, int N
 
 }  // namespace
 
-void diatomic_op_build(DiatomicDevice &d, hipStream_t s) {
-  d.op_in = false;
+namespace {
+// P/Q tiles in matrix-core operand order (FP64 lanes).
+__global__ void __launch_bounds__(NT) k_pq_operands(const double *pq, double *pqo) {
+  const size_t o = (size_t)blockIdx.x * TILE2;
+  const int u = threadIdx.x, lane = u >> 2;
+  pqo[o + u] = pq[o + (lane & 15) + TILE * Mma<double>::row(lane >> 4, u & 3)];
+}
+}  // namespace
+
+void diatomic_op_build(DiatomicDevice &d, const std::vector<int> &ni, hipStream_t s) {
+  d.pqo.alloc(d.pq.n);
+  static_assert(NT == TILE2, "one thread per tile entry");
+  hipLaunchKernelGGL(k_pq_operands, dim3((unsigned)(d.pq.n / TILE2)), dim3(NT), 0, s, d.pq.p, d.pqo.p);
+  hip_check(hipGetLastError(), "pq_operands");
+  d.op_in = d.fold_in = false;
   d.Top2.release();
+  d.Tfold.release();
+  d.Tfold32.release();
   const size_t nx = (size_t)d.n_lm * d.Nel;
   if (nx == 0 || d.max_rank > 2 * TILE2) return;
-  // opt-in: on N2 (lmax 16) the Cholesky-form kernel is faster (13.1 against
-  // 16.2 ms): each workgroup streams its 1.75 MB operator for 16 runs
   const char *env = std::getenv("HFGPU_EXCHANGE_OP");
-  if (!env || std::atoi(env) == 0) return;
+  if (env && std::atoi(env) == 0) return;
   size_t fr = 0, tot = 0;
   hip_check(hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
-  const size_t bytes = nx * OP_TSIZE * sizeof(double);
-  if (bytes > fr / 4) return;  // keep three quarters of the free memory for densities and tiles
-  d.Top2.alloc(nx * OP_TSIZE);
-  DOpBuildArgs a{d.chol.p, d.sigma.p, d.chol_off.p, d.chol_rank.p, d.ni.p, d.Nel, d.Top2.p};
-  hipLaunchKernelGGL(k_dia_op_build, dim3((unsigned)(nx * OP_KS)), dim3(NT), 0, s, a);
-  hip_check(hipGetLastError(), "diatomic_op_build");
-  d.op_in = true;
+  // keep three quarters of the free memory for densities and tiles
+  if (env) {
+    // on N2 (lmax 16) slower than the Cholesky-form kernel (16.2 against 13.1
+    // ms): each workgroup streams its 1.75 MB operator for 16 runs
+    if (nx * OP_TSIZE * sizeof(double) > fr / 4) return;
+    d.Top2.alloc(nx * OP_TSIZE);
+    DOpBuildArgs a{d.chol.p, d.sigma.p, d.chol_off.p, d.chol_rank.p, d.ni.p, d.Nel, d.Top2.p};
+    hipLaunchKernelGGL(k_dia_op_build, dim3((unsigned)(nx * OP_KS)), dim3(NT), 0, s, a);
+    hip_check(hipGetLastError(), "diatomic_op_build");
+    d.op_in = true;
+    return;
+  }
+  d.fold_n = *std::max_element(ni.begin(), ni.end());
+  const size_t size = kf_size(d.fold_n);
+  if (nx * size * sizeof(double) > fr / 4) return;
+  d.Tfold.alloc(nx * size);
+  const size_t step = (size_t)(65535 / d.Nel) * d.Nel;  // whole (L,|M|) within the grid's y limit
+  for (size_t x = 0; x < nx; x += step) {
+    const unsigned cnt = (unsigned)std::min(step, nx - x);
+    DFoldBuildArgs a{d.chol.p, d.sigma.p, d.chol_off.p + x, d.chol_rank.p + x, d.ni.p, d.Nel, size,
+                     d.Tfold.p + x * size};
+    if (d.max_rank <= KL_RANK_MAX)
+      hipLaunchKernelGGL(k_dia_fold_build<true>, dim3(FB_PARTS, cnt), dim3(FB_THREADS), 0, s, a);
+    else
+      hipLaunchKernelGGL(k_dia_fold_build<false>, dim3(FB_PARTS, cnt), dim3(FB_THREADS), 0, s, a);
+    hip_check(hipGetLastError(), "diatomic_fold_build");
+  }
+  d.fold_in = true;
 }
 
 void diatomic_coulomb_launch(const DiatomicDevice &d, const double *P, int64_t ldp, double *J, int64_t ldj,
@@ -1301,6 +1688,26 @@ void launch_dia_k(int part, bool tiled, int64_t grid, hipStream_t s, const DKArg
     hipLaunchKernelGGL((k_dia_k_in<T, false>), gd, bd, 0, s, a);
 }
 
+template <typename T>
+void launch_fold(const DiatomicDevice &d, const T *top, const T *u, const T *v, const T *pt, double *K, int64_t ldk,
+                 hipStream_t s) {
+  const int n = d.fold_n;
+  // the columns of one half, or all partial tiles of both, or the transposes' scratch
+  size_t lds = (size_t)32 * std::max(kf_inner(n, false), kf_inner(n, true));
+  for (int m = 1; m <= n; ++m) {  // elements of any size up to n
+    const int a = kf_tiles(m, false), b = kf_tiles(m, true);
+    lds = std::max(lds, (size_t)512 * (a * (KF_WAVES / a) + (b ? b * (KF_WAVES / b) : 0)));
+  }
+  lds = std::max(lds, (size_t)KF_WAVES * TILE * 17) * sizeof(T);
+  const void *f = reinterpret_cast<const void *>(&k_dia_kin_fold<T>);
+  if (lds > 64 * 1024)
+    hip_check(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "fold LDS size");
+  DFoldArgs<T> a{K, ldk, d.Nel, d.Nang, d.first.p, d.ni.p, d.skip.p, d.poff.p, top, kf_size(n), d.wg_kf.p, d.kf_jk.p,
+                 d.kf_ent.p, d.kf_rec.p, d.kf_more.p, u, v, pt, d.n_src, (int)d.sym};
+  hipLaunchKernelGGL(k_dia_kin_fold<T>, dim3(d.n_wg_kf), dim3(KF_THREADS), lds, s, a);
+  hip_check(hipGetLastError(), "diatomic_kin_fold");
+}
+
 // FP32 copy of the P/Q tiles with P kinds divided and Q kinds multiplied by
 // exp(lsig) of their (ilm, element), in storage and in operand order.
 __global__ void k_scale_pq_f32(const double *pq, const double *lsig, float *pq32, float *pqo32, int n_x) {
@@ -1344,6 +1751,12 @@ void diatomic_exchange_kernels(DiatomicDevice &d, const double *P, int64_t ldp, 
         to_f32_launch(d.k2_ltv.p, d.k2_ltv32.p, d.k2_ltv.n, s);
         to_f32_launch(d.k2_jtc.p, d.k2_jtc32.p, d.k2_jtc.n, s);
       }
+      if (d.n_wg_kf > 0) {
+        d.kf_u32.alloc(d.kf_u.n);
+        d.kf_v32.alloc(d.kf_v.n);
+        to_f32_launch(d.kf_u.p, d.kf_u32.p, d.kf_u.n, s);
+        to_f32_launch(d.kf_v.p, d.kf_v32.p, d.kf_v.n, s);
+      }
       d.term_f32_gen = d.list_gen;
     }
     if (!d.tiled) {
@@ -1385,6 +1798,19 @@ void diatomic_exchange_kernels(DiatomicDevice &d, const double *P, int64_t ldp, 
       hip_check(hipGetLastError(), "diatomic_kin_gemm");
       hipLaunchKernelGGL(k_dia_kin_reduce, dim3(d.n_act * d.Nel), dim3(NT), 0, s, r);
       hip_check(hipGetLastError(), "diatomic_kin_reduce");
+      continue;
+    }
+    if (part == 1 && d.n_wg_kf > 0) {
+      TimedLaunch tl(timer, name, s, d.flops_in_kf);
+      if (fp32) {
+        if (d.Tfold32.n != d.Tfold.n) {
+          d.Tfold32.alloc(d.Tfold.n);
+          to_f32_launch(d.Tfold.p, d.Tfold32.p, d.Tfold.n, s);
+        }
+        launch_fold<float>(d, d.Tfold32.p, d.kf_u32.p, d.kf_v32.p, d.ptile32.p, K, ldk, s);
+      } else {
+        launch_fold<double>(d, d.Tfold.p, d.kf_u.p, d.kf_v.p, d.ptile.p, K, ldk, s);
+      }
       continue;
     }
     if (part == 1 && d.op_in && d.tiled && !fp32 && d.n_wg_op > 0) {

@@ -29,6 +29,21 @@ constexpr int KL_BATCH = 64;
 constexpr int K2_SLOTS = 32, K2_THREADS = HFG_K2_THREADS, K2_WAVES = K2_THREADS / 64, K2_ROWS = 3;
 static_assert(K2_THREADS % 64 == 0 && K2_THREADS <= 1024, "two-step exchange workgroup");
 
+// in-element diatomic exchange with folded operators: threads (16 waves of two
+// rows), so columns, per workgroup; bytes of one (L,|M|, element) operator at
+// the largest element size
+constexpr int KF_THREADS = 1024, KF_WAVES = KF_THREADS / 64, KF_ROWS = 2, KF_COLS = KF_WAVES * KF_ROWS;
+static_assert(KF_COLS == 32, "two 16-column tiles");
+// extents of the folded operators of an n-function element: pairs a <= b (a <
+// b), their inner extent (both diagonal channels' pairs and the n^2 mixed
+// entries) padded to 16
+constexpr int kf_pairs(int n, bool anti) { return anti ? n * (n - 1) / 2 : n * (n + 1) / 2; }
+constexpr int kf_inner(int n, bool anti) { return (2 * kf_pairs(n, anti) + n * n + 15) / 16 * 16; }
+constexpr int kf_tiles(int n, bool anti) { return (kf_pairs(n, anti) + 15) / 16; }
+constexpr size_t kf_size(int n) {
+  return (size_t)16 * kf_tiles(n, false) * kf_inner(n, false) + (size_t)16 * kf_tiles(n, true) * kf_inner(n, true);
+}
+
 struct Error : std::runtime_error {
   int code;
   Error(int c, const std::string &m) : std::runtime_error(m), code(c) {}
@@ -299,6 +314,23 @@ struct DiatomicDevice {
   DevArray<double> Top2;
   DevArray<int> wg_op;
   int n_wg_op = 0;
+  // in-element exchange as dense operators folded by the transposition
+  // symmetries (k_dia_kin_fold), built on the device before the first exchange
+  // when they fit the budget; per workgroup (ilm, e, first unit, units); per unit two rows
+  // (output blocks jk, -1: none) and its entries: a slot's source record and
+  // the rows' weights (fac u0, fac u1)
+  bool fold_in = false;
+  bool op_ready = false;                  // diatomic_op_build has run for the uploaded tables
+  int fold_n = 0;                         // largest element size
+  DevArray<double> Tfold;                 // [n_lm*Nel][kf_size(fold_n)]
+  DevArray<float> Tfold32;
+  DevArray<int4> wg_kf;
+  DevArray<int> kf_jk, kf_ent;
+  DevArray<int4> kf_rec, kf_more;         // (first tile, tiles, first weight, next record in kf_more or -1)
+  DevArray<double> kf_u, kf_v;            // 2 KF_ROWS per entry; (v0, v1) per source, runs zero-padded to fours
+  DevArray<float> kf_u32, kf_v32;
+  int n_wg_kf = 0;
+  double flops_in_kf = 0.0;
   // Density tiles of the screened source blocks in gather order
   // ([e*Nel+f][src][lane][4], see k_dia_ptile), rebuilt per exchange call;
   // src_blk lists the blocks i*Nang+l, term_tile maps each term to its tile.
@@ -485,9 +517,11 @@ bool symmetric_exchange_allowed();
 void diatomic_exchange_kernels(DiatomicDevice &d, const double *P, int64_t ldp, double *K, int64_t ldk,
                                hipStream_t s, KernelTimer *timer, bool fp32 = false);
 void diatomic_build_operator(const DiatomicSetup &S, DiatomicDevice &d, hipStream_t s);
-// the matrix-core operators of k_dia_kin_op from the device Cholesky tiles
-// (opt-in with HFGPU_EXCHANGE_OP=1; sets d.op_in when they fit the budget)
-void diatomic_op_build(DiatomicDevice &d, hipStream_t s);
+// the in-element operators from the device Cholesky tiles, when they fit the
+// budget: folded ones (k_dia_kin_fold, sets d.fold_in; the default), or the
+// plain ones of k_dia_kin_op with HFGPU_EXCHANGE_OP=1 (d.op_in); neither with
+// HFGPU_EXCHANGE_OP=0 (the Cholesky-form kernel)
+void diatomic_op_build(DiatomicDevice &d, const std::vector<int> &ni, hipStream_t s);
 constexpr int OP_RUNS = 16;  // runs per k_dia_kin_op workgroup
 
 }  // namespace hfg

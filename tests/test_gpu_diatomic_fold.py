@@ -1,0 +1,67 @@
+"""The in-element diatomic exchange with folded operators at every shape of its
+tiles: element sizes from one function to a full 16 x 16 tile (row tiles, inner
+extents and their splits over the waves all follow the size), units with one
+and two rows, and the forms it stands in for.
+
+Bar: FP64 1e-12 of max|K| against the oracle (src/diatomic/basis.cpp:1818-2089),
+as the other parity tests; FP32 1.25 times the Cholesky-form kernel's error on
+the same inputs, or where an element holds so few functions that no sum
+averages the roundings out, the four of one product (density, both weights and
+operator, 2^-24 each): 2.4e-7."""
+import numpy as np
+import pytest
+
+import helfem_amd as H
+import oracle as O
+from helfem_amd.synthetic import random_symmetric
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-12
+
+
+def relerr(a, b):
+    return float(np.max(np.abs(a - b)) / max(np.max(np.abs(b)), 1e-300))
+
+
+@pytest.mark.parametrize("nodes", [2, 3, 4, 6, 9, 12, 16])
+def test_element_sizes(nodes, gpu_ctx, monkeypatch):
+    import torch
+    print(f"[gpu] folded in-element exchange, {nodes} nodes", flush=True)
+    ob = O.DiatomicBasis(3, 1, 3.0, [3, 2], 2, nnodes=nodes)
+    ob.compute_tei()
+    b = {}
+    for form in ("fold", "0"):
+        if form == "0":
+            monkeypatch.setenv("HFGPU_EXCHANGE_OP", "0")
+        b[form] = H.DiatomicBasis(3, 1, 3.0, [3, 2], 2, nnodes=nodes, ctx=gpu_ctx)
+        b[form].compute_tei()
+        b[form].exchange(torch.zeros((ob.Nbf, ob.Nbf), dtype=torch.float64, device="cuda"))  # the form is fixed here
+    S = random_symmetric(ob.Nbf, seed=2101)
+    G = S + 0.3 * np.triu(random_symmetric(ob.Nbf, seed=2102))
+    for P in (S, G):
+        Kr = ob.exchange(P)
+        Pd = torch.as_tensor(P, device="cuda")
+        e64 = {f: relerr(x.exchange(Pd).cpu().numpy(), Kr) for f, x in b.items()}
+        e32 = {f: relerr(x.exchange(Pd, precision="fp32").cpu().numpy(), Kr) for f, x in b.items()}
+        print(e64, e32, flush=True)
+        assert e64["fold"] <= TOL and e64["0"] <= TOL
+        assert e32["fold"] <= max(1.25 * e32["0"], 4 * 2.0 ** -24)
+
+
+def test_one_element_and_density_holes(gpu_ctx):
+    """A single element (no cross-element launch) and a density without some
+    of its shell blocks (runs of tiles with gaps)."""
+    import torch
+    print("[gpu] folded in-element exchange, one element, sparse density", flush=True)
+    for nel in (1, 2):
+        ob = O.DiatomicBasis(2, 1, 1.5, [4, 3], nel, nnodes=6)
+        ob.compute_tei()
+        hb = H.DiatomicBasis(2, 1, 1.5, [4, 3], nel, nnodes=6, ctx=gpu_ctx)
+        hb.compute_tei()
+        P = random_symmetric(ob.Nbf, seed=2103)
+        sh = np.asarray(hb.pure_idx) // hb.Nrad
+        rng = np.random.default_rng(2104)
+        keep = rng.random((hb.Nang, hb.Nang)) < 0.6
+        keep = keep & keep.T
+        P = P * keep[sh][:, sh]
+        assert relerr(hb.exchange(torch.as_tensor(P, device="cuda")).cpu().numpy(), ob.exchange(P)) <= TOL
