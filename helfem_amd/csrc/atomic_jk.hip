@@ -465,6 +465,270 @@ void launch_atomic_k(int part, bool tiled, int64_t grid, hipStream_t s, const KA
     hipLaunchKernelGGL(k_atomic_k_in_f32<false>, gd, bd, 0, s, a);
 }
 
+// --- Cross-element exchange by density classes -----------------------------------
+//
+// K_jk(e,f) = sum_L A_L [sum_il g(j,L,i) g(k,L,l) P_il(e,f)] B_L', M = m_j - m_i =
+// m_k - m_l.  l_j + L + l_i and l_k + L + l_l are even, so the outputs of one
+// (m_j - m_k, parities) draw on two classes of density blocks, one for even and
+// one for odd L: at most 58 of the 231 blocks of an m-diagonal lmax = 6 density,
+// 116 KB.  One workgroup per (element pair, up to eight units of one output
+// class) loads them into LDS, one class after the other; a wave's unit is one
+// column k with up to four rows j of one m and parity, which share the column
+// sums w = sum_l g(k,L,l) P_il; the multipoles of a unit are split over two to
+// four waves, which is what keeps a CU busy with one such workgroup.  Per L a
+// wave forms its rows' tiles R_j = sum_i g(j,L,i) w_i in matrix-operand layout and
+// adds A R B'.  Eight entries' coefficients come in one vector load (a value per
+// lane, broadcast by readlane): as scalar loads they would share their counter
+// with the LDS reads, and every tile read would wait for them.
+// Bound by the LDS reads and the vector sums between them.  Xe (lmax = mmax = 6,
+// 25 elements): 2.86 ms one block at a time from L2 (k_atomic_k_off_f64), 1.75 ms
+// here (1.87 with one wave per unit, 2.83 with uniform coefficient loads).
+
+template <typename T>
+struct KCArgs {
+  const T *pt;  // tiled density
+  int n_src;
+  double *K;
+  int64_t ldk;
+  int Nel, Nrad, Nang;
+  const int *first, *ni;
+  const T *rs, *rb, *Lscale;
+  const int4 *wg;
+  const int2 *stage;
+  const int *jk, *us, *ub;
+  const int4 *blk;
+  const int *eh;
+  const T *ec;
+  const int *efl;
+  int n_ef, n_wg, max_rows, sym;
+};
+
+// Tiles in LDS: FP64 as two halves [half][lane][2], FP32 as [lane][4], so that
+// a wave's 16-byte reads are contiguous.
+template <typename T>
+__device__ inline typename Mma<T>::acc_t lds_tile(const T *t, int lane) {
+  typedef typename Mma<T>::acc_t vec;
+  if constexpr (sizeof(T) == 8) {
+    typedef T v2 __attribute__((ext_vector_type(2)));
+    const v2 a = *reinterpret_cast<const v2 *>(t + 2 * lane), b = *reinterpret_cast<const v2 *>(t + 128 + 2 * lane);
+    return vec{a[0], a[1], b[0], b[1]};
+  } else {
+    return *reinterpret_cast<const vec *>(t + 4 * lane);
+  }
+}
+
+// lane l's value in a scalar register
+__device__ inline double lane_value(double v, int l) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+__device__ inline float lane_value(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+template <typename T>
+__device__ inline void kc_body(const KCArgs<T> &A, int w) {
+  typedef Mma<T> MM;
+  typedef typename MM::acc_t vec;
+  extern __shared__ char kc_smem[];
+  T *tiles = reinterpret_cast<T *>(kc_smem);
+  const int xcd = w & 7, loc = w >> 3;
+  const int efi = (loc / A.n_wg) * 8 + xcd;
+  if (efi >= A.n_ef) return;
+  const int4 wg = A.wg[loc - (loc / A.n_wg) * A.n_wg];
+  const int ef = A.efl[efi], e = ef / A.Nel, f = ef - e * A.Nel;
+  const int t = threadIdx.x, lane = t & 63, g = lane >> 4, c = lane & 15;
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  int kk[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) kk[s] = MM::row(g, s);
+  const int split = kc_split(wg.y), un = wv / split, part = wv - un * split;
+  const bool mine = un < wg.y;
+  const int unit = wg.x + (mine ? un : 0);
+  const int *jk = A.jk + unit * KC_ROWS;
+  const int nrow = jk[3] >= 0 ? 4 : jk[2] >= 0 ? 3 : jk[1] >= 0 ? 2 : 1;
+  v4d acc[KC_ROWS];
+#pragma unroll
+  for (int r = 0; r < KC_ROWS; ++r) acc[r] = v4d{0, 0, 0, 0};
+  // row and column side's element matrices of multipole L
+  auto factors = [&](int L, T as[4], T bs[4]) {
+    const size_t te = ((size_t)L * A.Nel + e) * TILE2, tf = ((size_t)L * A.Nel + f) * TILE2;
+    const T *At = (e > f) ? A.rb + te : A.rs + te;
+    const T *Bt = (e > f) ? A.rs + tf : A.rb + tf;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      as[s] = At[c + TILE * kk[s]];
+      bs[s] = Bt[c + TILE * kk[s]];
+    }
+  };
+  for (int st = 0; st < wg.w; ++st) {
+    const int2 sg = A.stage[wg.z + st];
+    if (st) __syncthreads();
+    {
+      const int4 *src = reinterpret_cast<const int4 *>(A.pt + ((size_t)ef * A.n_src + sg.x) * TILE2);
+      int4 *dst = reinterpret_cast<int4 *>(tiles);
+      constexpr int PER = TILE2 * sizeof(T) / 16;  // 16-byte units per tile
+      for (int q = t; q < sg.y * PER; q += 64 * KC_WAVES) {
+        const int u = q & (PER - 1);
+        dst[sizeof(T) == 8 ? q - u + (u & 1) * 64 + (u >> 1) : q] = src[q];
+      }
+    }
+    __syncthreads();
+    if (!mine) continue;
+    const int b0 = A.ub[A.us[unit] + st], b1 = A.ub[A.us[unit] + st + 1];
+    if (b0 == b1) continue;
+    // eight entries at a time: one coefficient per lane, the headers in lanes
+    // 0-7, the next eight (of this block or the wave's next) fetched ahead
+    if (b0 + part >= b1) continue;
+    int4 bk = A.blk[b0 + part];
+    int h = A.eh[bk.y + (lane & 7)];
+    T cf = A.ec[(size_t)bk.y * 8 + lane];
+    for (int b = b0 + part; b < b1; b += split) {
+      const int4 bn = A.blk[min(b + split, b1 - 1)];
+      T as[4], bs[4];
+      factors(bk.x, as, bs);
+      const T msc = A.Lscale ? A.Lscale[bk.x] : T(1);
+      auto rows = [&](auto count) {
+        constexpr int N = decltype(count)::value;
+        vec R[N];
+#pragma unroll
+        for (int r = 0; r < N; ++r) R[r] = vec{0, 0, 0, 0};
+        for (int x = bk.y; x < bk.z; x += 8) {
+          const int nx = x + 8 < bk.z ? x + 8 : bn.y;
+          const int hn = A.eh[nx + (lane & 7)];
+          const T cn = A.ec[(size_t)nx * 8 + lane];
+#pragma unroll
+          for (int z = 0; z < 8; ++z) {
+            if (x + z >= bk.z) break;
+            const int hs = __builtin_amdgcn_readlane(h, z);
+            const T *tp = tiles + (hs & 0xffff) * TILE2;
+            const int last = hs >> 16;
+            const vec t0 = lds_tile<T>(tp, lane), t1 = lds_tile<T>(tp + min(last, 1) * TILE2, lane);
+            vec wsum = lane_value(cf, 8 * z + 4) * t0;
+            wsum += lane_value(cf, 8 * z + 5) * t1;
+            if (last >= 2) {
+              const vec t2 = lds_tile<T>(tp + 2 * TILE2, lane), t3 = lds_tile<T>(tp + last * TILE2, lane);
+              wsum += lane_value(cf, 8 * z + 6) * t2;
+              wsum += lane_value(cf, 8 * z + 7) * t3;
+            }
+#pragma unroll
+            for (int r = 0; r < N; ++r) R[r] += lane_value(cf, 8 * z + r) * wsum;
+          }
+          h = hn;
+          cf = cn;
+        }
+#pragma unroll
+        for (int r = 0; r < N; ++r) {
+          R[r] *= msc;
+          vec y = {0, 0, 0, 0};
+#pragma unroll
+          for (int s = 0; s < 4; ++s) y = MM::step(R[r][s], bs[s], y);  // Y = R B'
+          vec x = {0, 0, 0, 0};
+          if constexpr (sizeof(T) == 8) x = acc[r];
+#pragma unroll
+          for (int s = 0; s < 4; ++s) x = MM::step(as[s], y[s], x);  // += A Y
+          if constexpr (sizeof(T) == 8)
+            acc[r] = x;
+          else
+#pragma unroll
+            for (int s = 0; s < 4; ++s) acc[r][s] += (double)x[s];
+        }
+      };
+      if (nrow == 4)
+        rows(std::integral_constant<int, 4>());
+      else if (nrow == 3)
+        rows(std::integral_constant<int, 3>());
+      else if (nrow == 2)
+        rows(std::integral_constant<int, 2>());
+      else
+        rows(std::integral_constant<int, 1>());
+      bk = bn;
+    }
+  }
+  if (split > 1) {
+    // the unit's waves' tiles, added up by the first of them
+    double *sum = reinterpret_cast<double *>(kc_smem);
+    __syncthreads();
+    if (mine && part > 0)
+#pragma unroll
+      for (int r = 0; r < KC_ROWS; ++r)
+        if (r < nrow) {
+          double *o = sum + (((size_t)un * (split - 1) + part - 1) * A.max_rows + r) * TILE2 + 2 * lane;
+          *reinterpret_cast<double2 *>(o) = make_double2(acc[r][0], acc[r][1]);
+          *reinterpret_cast<double2 *>(o + 128) = make_double2(acc[r][2], acc[r][3]);
+        }
+    __syncthreads();
+    if (mine && part == 0)
+      for (int q = 0; q < split - 1; ++q)
+#pragma unroll
+        for (int r = 0; r < KC_ROWS; ++r)
+          if (r < nrow) acc[r] += lds_tile<double>(sum + (((size_t)un * (split - 1) + q) * A.max_rows + r) * TILE2, lane);
+  }
+  if (!mine || part > 0) return;
+  const int ni = A.ni[e], nj = A.ni[f], fi = A.first[e], fj = A.first[f];
+  const bool scol = (c == 0 && f > 0) || (c == nj - 1 && f + 1 < A.Nel);
+#pragma unroll
+  for (int r = 0; r < KC_ROWS; ++r) {
+    if (jk[r] < 0) break;
+    const int j = jk[r] / A.Nang, k = jk[r] - j * A.Nang;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int a = kk[s];
+      if (a >= ni || c >= nj) continue;
+      const int64_t row = (int64_t)j * A.Nrad + fi + a, col = (int64_t)k * A.Nrad + fj + c;
+      const bool srow = (a == 0 && e > 0) || (a == ni - 1 && e + 1 < A.Nel);
+      const double v = acc[r][s];
+      double *dst = A.K + row + col * A.ldk;
+      if (srow || scol)
+        atomicAdd(dst, -v);
+      else
+        *dst = -v;
+      if (A.sym) {
+        double *mdst = A.K + col + row * A.ldk;
+        if (srow || scol)
+          atomicAdd(mdst, -v);
+        else
+          *mdst = -v;
+      }
+    }
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(64 * KC_WAVES) __attribute__((amdgpu_waves_per_eu(4))) k_atomic_kc_off(KCArgs<T> A) {
+  kc_body<T>(A, blockIdx.x);
+}
+
+// Bytes of LDS: a stage's tiles, then the partial row tiles.
+template <typename T>
+size_t kc_bytes(const AtomicDevice &d) {
+  return std::max((size_t)d.kc_tiles * TILE2 * sizeof(T), (size_t)d.kc_parts * TILE2 * sizeof(double));
+}
+void kc_lds(const void *f, size_t bytes) {
+  if (bytes > 64 * 1024)
+    hip_check(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes), "class exchange LDS size");
+}
+
+template <typename T>
+KCArgs<T> kc_args(const AtomicDevice &d, const T *pt, const T *rs, const T *rb, const T *Lscale, const T *ec, double *K,
+                  int64_t ldk, const int *efl, int n_ef) {
+  if (!pt || !rs || !rb || !ec || !efl) throw Error(-5, "class exchange tables are not on the device");
+  return KCArgs<T>{pt, d.n_src, K, ldk, d.Nel, d.Nrad, d.Nang, d.first.p, d.ni.p, rs, rb, Lscale, d.kc_wg.p,
+                   d.kc_stage.p, d.kc_jk.p, d.kc_us.p, d.kc_ub.p, d.kc_blk.p, d.kc_eh.p, ec, efl, n_ef, d.n_wg_kc,
+                   d.kc_rows, (int)d.sym};
+}
+
+template <typename T>
+void launch_kc(const AtomicDevice &d, const KCArgs<T> &a, hipStream_t s) {
+  const int64_t grid = (int64_t)(((a.n_ef + 7) / 8) * 8) * a.n_wg;
+  if (grid > 0x7fffffff) throw Error(-1, "exchange grid too large");
+  const size_t lds = kc_bytes<T>(d);
+  kc_lds(reinterpret_cast<const void *>(&k_atomic_kc_off<T>), lds);
+  hipLaunchKernelGGL(k_atomic_kc_off<T>, dim3((unsigned)grid), dim3(64 * KC_WAVES), lds, s, a);
+  hip_check(hipGetLastError(), "atomic_kc_off");
+}
+
 // --- Range-separated exchange with non-separable (erfc) element pairs ------------
 //
 // One workgroup per (coupled output block, element pair (e,f)), all pairs
@@ -843,6 +1107,206 @@ void atomic_coulomb_launch(const AtomicDevice &d, const double *P, int64_t ldp, 
   }
 }
 
+// Classes, units and entries of k_atomic_kc_off for the density blocks of
+// `mask`; src is reordered so that a class' blocks are consecutive tiles.
+// Leaves d.kc off where its tiles are not used or hold infinities (rows of a
+// wave share sums, and padded sources reread a tile with zero weight).
+static void build_classes(AtomicDevice &d, const std::vector<unsigned char> &mask, int64_t n_runs,
+                          std::vector<int> &src, hipStream_t s) {
+  const int Na = d.Nang, nL = d.N_L;
+  const std::vector<int> &lv = d.h_lv, &mv = d.h_mv;
+  d.kc = false;
+  d.n_wg_kc = 0;
+  // class of a block: m_i - m_l, parities; then row shell by m, l; column shell by l
+  typedef std::array<int, 3> Cls;
+  auto cls = [&](int il) { return Cls{mv[il / Na] - mv[il % Na], lv[il / Na] & 1, lv[il % Na] & 1}; };
+  src.clear();
+  for (int il = 0; il < Na * Na; ++il)
+    if (mask[il]) src.push_back(il);
+  auto key = [&](int il) {
+    const int i = il / Na, l = il % Na;
+    const Cls x = cls(il);
+    return std::array<int, 7>{x[0], x[1], x[2], mv[i], lv[i], i, lv[l]};
+  };
+  std::sort(src.begin(), src.end(), [&](int a, int b) { return key(a) < key(b); });
+  if (!d.tiled || !d.finite || d.Nel < 2 || src.empty()) return;
+  const char *env = std::getenv("HFGPU_EXCHANGE_CLASSES");
+  if (env ? std::atoi(env) == 0 : (double)d.n_terms < KC_MIN_TERMS * (double)n_runs) return;
+  // stages of every class, cut between row shells; a row shell holds at most
+  // one m_l, so a stage always fits one (at most 129 shells of one m would not)
+  struct Stage {
+    int first, n;
+  };
+  std::map<Cls, std::vector<Stage>> stages;
+  std::vector<int> stage_of(src.size());  // within its class
+  for (size_t a = 0; a < src.size();) {
+    size_t b = a;
+    while (b < src.size() && cls(src[b]) == cls(src[a]) && src[b] / Na == src[a] / Na) ++b;
+    if (b - a > (size_t)KC_TILES) return;
+    auto &v = stages[cls(src[a])];
+    if (v.empty() || v.back().n + (int)(b - a) > KC_TILES) v.push_back({(int)a, 0});
+    v.back().n += (int)(b - a);
+    for (size_t q = a; q < b; ++q) stage_of[q] = (int)v.size() - 1;
+    a = b;
+  }
+  std::vector<int> at((size_t)Na * Na, -1);
+  for (size_t q = 0; q < src.size(); ++q) at[src[q]] = (int)q;
+  std::vector<std::vector<int>> sector;  // shells by m, ascending l
+  int mmin = 0, mmax = 0;
+  for (int m : mv) {
+    mmin = std::min(mmin, m);
+    mmax = std::max(mmax, m);
+  }
+  sector.resize(mmax - mmin + 1);
+  for (int a = 0; a < Na; ++a) sector[mv[a] - mmin].push_back(a);
+  for (auto &v : sector) std::sort(v.begin(), v.end(), [&](int a, int b) { return lv[a] < lv[b]; });
+  struct Unit {
+    int jk[KC_ROWS];
+    double cost;
+    std::vector<std::vector<int4>> blk;  // per stage: (L, entries), entry ranges local to the unit
+    std::vector<int> eh;
+    std::vector<double> ec;
+  };
+  std::map<Cls, std::vector<Unit>> units;
+  double flops = 0.0;
+  for (int k = 0; k < Na; ++k)
+    for (int mj = mmin; mj <= mmax; ++mj)
+      for (int pj = 0; pj < 2; ++pj) {
+        std::vector<int> js;
+        for (int j : sector[mj - mmin])
+          if ((lv[j] & 1) == pj) js.push_back(j);
+        const int dm = mj - mv[k], pk = lv[k] & 1;
+        for (size_t j0 = 0; j0 < js.size(); j0 += KC_ROWS) {
+          const int nr = std::min(KC_ROWS, (int)(js.size() - j0));
+          Unit U;
+          U.cost = 0.0;
+          for (int r = 0; r < KC_ROWS; ++r) U.jk[r] = r < nr ? js[j0 + r] * Na + k : -1;
+          // stages: the class of even L, then that of odd L
+          for (int pL = 0; pL < 2; ++pL) {
+            const auto it = stages.find(Cls{dm, pj ^ pL, pk ^ pL});
+            const int ns = it == stages.end() ? 0 : (int)it->second.size();
+            const size_t base = U.blk.size();
+            U.blk.resize(base + ns);
+            if (!ns) continue;
+            for (int L = pL; L < nL; L += 2) {
+              std::vector<std::vector<std::pair<int, std::array<double, KC_ROWS + KC_SRC>>>> ent(ns);
+              for (int mi = mmin; mi <= mmax; ++mi) {
+                const int M = mj - mi, ml = mv[k] - M;
+                if (std::abs(M) > L || ml < mmin || ml > mmax) continue;
+                for (int i : sector[mi - mmin]) {
+                  std::array<double, KC_ROWS + KC_SRC> c{};
+                  bool any = false;
+                  for (int r = 0; r < nr; ++r) {
+                    c[r] = d.h_g[((size_t)js[j0 + r] * Na + i) * nL + L] * (4.0 * M_PI / double(2 * L + 1));
+                    any = any || c[r] != 0.0;
+                  }
+                  if (!any) continue;
+                  int first = -1, n = 0, stg = 0;
+                  auto flush = [&] {
+                    if (n) ent[stg].push_back({(first - it->second[stg].first) | (n - 1) << 16, c});
+                    n = 0;
+                    for (int z = 0; z < KC_SRC; ++z) c[KC_ROWS + z] = 0.0;
+                  };
+                  for (int l : sector[ml - mmin]) {
+                    const double v = d.h_g[((size_t)k * Na + l) * nL + L];
+                    const int q = at[(size_t)i * Na + l];
+                    if (v == 0.0 || q < 0) continue;
+                    if (n == KC_SRC || (n && q != first + n)) flush();
+                    if (!n) {
+                      first = q;
+                      stg = stage_of[q];
+                    }
+                    c[KC_ROWS + n++] = v;
+                    flops += 2.0;
+                  }
+                  flush();
+                }
+              }
+              for (int x = 0; x < ns; ++x) {
+                if (ent[x].empty()) continue;
+                const int e0 = (int)U.eh.size();
+                for (auto &y : ent[x]) {
+                  U.eh.push_back(y.first);
+                  U.ec.insert(U.ec.end(), y.second.begin(), y.second.end());
+                }
+                flops += 2.0 * nr * (double)ent[x].size();
+                U.blk[base + x].push_back(make_int4(L, e0, (int)U.eh.size(), 0));
+                U.cost += 8.0 * (double)ent[x].size() + 16.0 * nr;
+              }
+            }
+          }
+          static_assert(KC_ROWS + KC_SRC == 8, "eight coefficients an entry, eight entries a wave load");
+          if (!U.eh.empty()) units[Cls{dm, pj, pk}].push_back(std::move(U));
+        }
+      }
+  std::vector<int4> wg, blk;
+  std::vector<int2> stage;
+  std::vector<int> jk, us, ub, eh;
+  std::vector<double> ec;
+  std::vector<std::pair<double, int4>> order;
+  d.kc_tiles = 1;
+  d.kc_rows = 1;
+  d.kc_parts = 0;
+  for (auto &kv : units) {
+    auto &v = kv.second;
+    std::stable_sort(v.begin(), v.end(), [](const Unit &a, const Unit &b) { return a.cost > b.cost; });
+    const int s0 = (int)stage.size();
+    for (int pL = 0; pL < 2; ++pL) {
+      const auto it = stages.find(Cls{kv.first[0], kv.first[1] ^ pL, kv.first[2] ^ pL});
+      if (it == stages.end()) continue;
+      for (const Stage &x : it->second) {
+        stage.push_back(make_int2(x.first, x.n));
+        d.kc_tiles = std::max(d.kc_tiles, x.n);
+      }
+    }
+    for (size_t a = 0; a < v.size(); a += KC_UNITS) {
+      const int n = std::min(KC_UNITS, (int)(v.size() - a));
+      order.push_back({v[a].cost, make_int4((int)us.size(), n, s0, (int)stage.size() - s0)});
+      for (int x = 0; x < n; ++x) {
+        const Unit &U = v[a + x];
+        jk.insert(jk.end(), U.jk, U.jk + KC_ROWS);
+        for (int r = 0; r < KC_ROWS; ++r)
+          if (U.jk[r] >= 0) d.kc_rows = std::max(d.kc_rows, r + 1);
+        us.push_back((int)ub.size());
+        ub.push_back((int)blk.size());
+        const int e0 = (int)eh.size();
+        for (const auto &sb : U.blk) {
+          for (const int4 &b : sb) blk.push_back(make_int4(b.x, b.y + e0, b.z + e0, 0));
+          ub.push_back((int)blk.size());
+        }
+        eh.insert(eh.end(), U.eh.begin(), U.eh.end());
+        ec.insert(ec.end(), U.ec.begin(), U.ec.end());
+      }
+    }
+  }
+  if (order.empty()) return;
+  if (!env && (int64_t)order.size() * (d.Nel * (d.Nel - 1) / (d.sym ? 2 : 1)) < KC_MIN_WGS) return;
+  std::stable_sort(order.begin(), order.end(),
+                   [](const std::pair<double, int4> &a, const std::pair<double, int4> &b) { return a.first > b.first; });
+  for (auto &x : order) {
+    wg.push_back(x.second);
+    d.kc_parts = std::max(d.kc_parts, x.second.y * (kc_split(x.second.y) - 1) * d.kc_rows);
+  }
+  eh.resize(eh.size() + 8, 0);  // eight entries are read at a time
+  ec.resize(ec.size() + 8 * (KC_ROWS + KC_SRC), 0.0);
+  d.kc_wg.upload(wg, s);
+  d.kc_stage.upload(stage, s);
+  d.kc_jk.upload(jk, s);
+  d.kc_us.upload(us, s);
+  d.kc_ub.upload(ub, s);
+  d.kc_blk.upload(blk, s);
+  d.kc_eh.upload(eh, s);
+  d.kc_ec.upload(ec, s);
+  hip_check(hipStreamSynchronize(s), "class list upload");  // before the host lists go
+  d.n_wg_kc = (int)wg.size();
+  double area = 0.0;
+  for (int e = 0; e < d.Nel; ++e)
+    for (int f = 0; f < d.Nel; ++f)
+      if (d.sym ? e > f : e != f) area += (double)d.h_ni[e] * d.h_ni[f];
+  d.flops_kc = flops * area;
+  d.kc = true;
+}
+
 // Compact the static coupling lists to the density blocks that pass the
 // norm screen (|P_il|_F >= 10 eps, TwoDBasis.cpp:949-952).  The result only
 // changes when the screening pattern does, so it is cached by pattern.
@@ -858,13 +1322,17 @@ static void compact_exchange_lists(AtomicDevice &d, hipStream_t s) {
         const unsigned char m = mask[(size_t)i * Na + l] | mask[(size_t)l * Na + i];
         mask[(size_t)i * Na + l] = mask[(size_t)l * Na + i] = m;
       }
-  if (mask == d.screen_mask && !d.screen_mask.empty() && d.sym == d.list_sym) return;
+  bool finite = true;
+  for (size_t q = 0; q < mask.size(); ++q) finite = finite && d.h_bnorm.p[q] < 1e30;
+  if (mask == d.screen_mask && !d.screen_mask.empty() && d.sym == d.list_sym && finite == d.finite) return;
+  d.finite = finite;
+  d.screen_mask.clear();  // no lists until all of them are there
   std::vector<int> act, tstart(1, 0), til;
   std::vector<double> tc;
   // flops as executed: in the symmetric mode the cross-element launch covers
   // the pairs e > f and the in-element one the blocks j <= k
   double frad_off = 0.0, frad_in = 0.0;
-  int64_t nterm_in = 0;
+  int64_t nterm_in = 0, n_runs = 0;  // (block, L) with any term
   for (size_t a = 0; a < d.h_act.size(); ++a) {
     const size_t n0 = til.size();
     const bool in_done = !d.sym || d.h_act[a] / Na <= d.h_act[a] % Na;
@@ -878,6 +1346,7 @@ static void compact_exchange_lists(AtomicDevice &d, hipStream_t s) {
           tc.push_back(d.h_tc[q]);
         }
       if (til.size() > before) {
+        ++n_runs;
         frad_off += d.sym ? d.h_radL_low[L] : d.h_radL[L] - d.h_radL_in[L];
         if (in_done) frad_in += d.h_radL_in[L];
       }
@@ -899,6 +1368,7 @@ static void compact_exchange_lists(AtomicDevice &d, hipStream_t s) {
   }
   d.flops_in = frad_in + 2.0 * (double)nterm_in * area_in;
   d.flops_off = frad_off + 2.0 * (double)d.n_terms * area_off;
+  d.frad_off = frad_off;
   d.flops_k_radial = frad_in + frad_off;
   d.flops_k_angular = d.flops_in + d.flops_off - d.flops_k_radial;
   if (d.dense_in && !act.empty()) {
@@ -967,21 +1437,20 @@ static void compact_exchange_lists(AtomicDevice &d, hipStream_t s) {
     d.term_off.upload(toff, s);
   }
   {
-    // source blocks referenced by the terms, and each term's tile among them
+    // source blocks, and each term's tile among them
     std::vector<int> id((size_t)Na * Na, -1), src, tt(til.size());
-    for (size_t q = 0; q < til.size(); ++q) {
-      int &x = id[til[q]];
-      if (x < 0) {
-        x = (int)src.size();
-        src.push_back(til[q]);
-      }
-      tt[q] = x;
-    }
-    const double bytes = (double)src.size() * d.Nel * d.Nel * TILE2 * sizeof(double);
+    size_t n_mask = 0;
+    for (unsigned char m : mask) n_mask += m;
+    const double bytes = (double)n_mask * d.Nel * d.Nel * TILE2 * sizeof(double);
     d.tiled = bytes <= exchange_tile_budget(d.ptile.n * sizeof(double) + d.ptile32.n * sizeof(float));
+    build_classes(d, mask, n_runs, src, s);
+    for (size_t q = 0; q < src.size(); ++q) id[src[q]] = (int)q;
+    for (size_t q = 0; q < til.size(); ++q) tt[q] = std::max(id[til[q]], 0);
     d.n_src = (int)src.size();
+    if (src.empty()) src.push_back(0);
     d.src_blk.upload(src, s);
     d.term_tile.upload(tt, s);
+    hip_check(hipStreamSynchronize(s), "exchange source upload");
   }
   d.term_c.upload(tc, s);
   hip_check(hipStreamSynchronize(s), "exchange list upload");
@@ -1006,6 +1475,34 @@ static bool exchange_prologue(AtomicDevice &d, const double *P, int64_t ldp, dou
   compact_exchange_lists(d, s);
   fill_zero_launch(K, nbf, nbf, ldk, s);
   return d.n_act > 0;
+}
+
+// FP32 copies of the radial tables and of the current lists' weights (and of
+// P where the kernels gather from it) for the reduced-precision exchange.
+static void prepare_f32(AtomicDevice &d, const double *P, int64_t ldp, hipStream_t s) {
+  if (!d.f32_tables) {
+    d.rs32.alloc(d.rs.n);
+    d.rb32.alloc(d.rb.n);
+    d.chol32.alloc(d.chol.n);
+    to_f32_launch(d.rs.p, d.rs32.p, d.rs.n, s);
+    to_f32_launch(d.rb.p, d.rb32.p, d.rb.n, s);
+    to_f32_launch(d.chol.p, d.chol32.p, d.chol.n, s);
+    d.f32_tables = true;
+  }
+  if (d.term_c32_gen != d.list_gen) {
+    d.term_c32.alloc(d.term_c.n);
+    to_f32_launch(d.term_c.p, d.term_c32.p, d.term_c.n, s);
+    if (d.kc) {
+      d.kc_ec32.alloc(d.kc_ec.n);
+      to_f32_launch(d.kc_ec.p, d.kc_ec32.p, d.kc_ec.n, s);
+    }
+    d.term_c32_gen = d.list_gen;
+  }
+  if (!d.tiled) {
+    const int64_t nbf = (int64_t)d.Nrad * d.Nang;
+    d.P32.alloc((size_t)nbf * nbf);
+    mat_to_f32_launch(P, ldp, d.P32.p, nbf, s);
+  }
 }
 
 // The tiled density of this call (FP64 or FP32), when the tiles are in use.
@@ -1044,6 +1541,11 @@ void atomic_rs_exchange_launch(AtomicDevice &d, const double *P, int64_t ldp, do
                       d.term_off.p, d.term_c.p, efl, n_ef, d.rs_Lscale.p,
                       d.tiled ? d.ptile.p : nullptr, d.term_tile.p, d.n_src, (int)d.sym};
       TimedLaunch tl(timer, "atomic_rs_k_yukawa", s);
+      if (part == 0 && d.kc) {
+        launch_kc<double>(d, kc_args<double>(d, d.ptile.p, d.y_rs.p, d.y_rb.p, d.rs_Lscale.p, d.kc_ec.p, K, ldk, efl, n_ef),
+                          s);
+        continue;
+      }
       launch_atomic_k(part, d.tiled, grid, s, a);
       hip_check(hipGetLastError(), "atomic_rs_k");
     }
@@ -1065,26 +1567,7 @@ void atomic_exchange_launch(AtomicDevice &d, const double *P, int64_t ldp, doubl
                             hipStream_t s, KernelTimer *timer, bool fp32) {
   const int64_t nbf = (int64_t)d.Nrad * d.Nang;
   if (!exchange_prologue(d, P, ldp, K, ldk, s, true)) return;
-  if (fp32) {
-    if (!d.f32_tables) {
-      d.rs32.alloc(d.rs.n);
-      d.rb32.alloc(d.rb.n);
-      d.chol32.alloc(d.chol.n);
-      to_f32_launch(d.rs.p, d.rs32.p, d.rs.n, s);
-      to_f32_launch(d.rb.p, d.rb32.p, d.rb.n, s);
-      to_f32_launch(d.chol.p, d.chol32.p, d.chol.n, s);
-      d.f32_tables = true;
-    }
-    if (d.term_c32_gen != d.list_gen) {
-      d.term_c32.alloc(d.term_c.n);
-      to_f32_launch(d.term_c.p, d.term_c32.p, d.term_c.n, s);
-      d.term_c32_gen = d.list_gen;
-    }
-    if (!d.tiled) {
-      d.P32.alloc((size_t)nbf * nbf);
-      mat_to_f32_launch(P, ldp, d.P32.p, nbf, s);
-    }
-  }
+  if (fp32) prepare_f32(d, P, ldp, s);
   build_density_tiles(d, P, ldp, fp32, s, timer);
   // two launches: element pairs e != f and the in-element tiles; boundary
   // rows/cols shared by neighbouring tiles are accumulated atomically in both
@@ -1109,7 +1592,14 @@ void atomic_exchange_launch(AtomicDevice &d, const double *P, int64_t ldp, doubl
     const int64_t grid = (int64_t)n_ef_pad * d.n_act;
     if (grid > 0x7fffffff) throw Error(-1, "exchange grid too large");
     const int *efl = part == 0 ? (d.sym ? d.ef_low.p : d.ef_off.p) : d.ef_in.p;
-    TimedLaunch tl(timer, name, s, flops);
+    TimedLaunch tl(timer, name, s, part == 0 && d.kc ? d.frad_off + d.flops_kc : flops);
+    if (part == 0 && d.kc) {
+      if (fp32)
+        launch_kc<float>(d, kc_args<float>(d, d.ptile32.p, d.rs32.p, d.rb32.p, nullptr, d.kc_ec32.p, K, ldk, efl, n_ef), s);
+      else
+        launch_kc<double>(d, kc_args<double>(d, d.ptile.p, d.rs.p, d.rb.p, nullptr, d.kc_ec.p, K, ldk, efl, n_ef), s);
+      continue;
+    }
     if (fp32) {
       KArgs<float> a{d.P32.p, nbf, K, ldk, d.Nel, d.Nrad, d.Nang, d.N_L, d.n_act, d.first.p, d.ni.p,
                      d.rs32.p, d.rb32.p, d.chol32.p, d.chol_off.p, d.chol_rank.p, d.act_jk.p, d.term_start.p,
@@ -1430,27 +1920,7 @@ void atomic_batch_exchange(AtomicBatch &b, const double *const *P, const int64_t
     const bool symmetric = block_stats_reduce(b.h_stats.p + b.stats_off[i], d.Nrad, d.Nang, d.h_bnorm.p);
     d.sym = !d.dense_in && symmetric_exchange_allowed() && symmetric;
     compact_exchange_lists(d, s);
-    if (fp32[i] && d.n_act > 0) {
-      if (!d.f32_tables) {
-        d.rs32.alloc(d.rs.n);
-        d.rb32.alloc(d.rb.n);
-        d.chol32.alloc(d.chol.n);
-        to_f32_launch(d.rs.p, d.rs32.p, d.rs.n, s);
-        to_f32_launch(d.rb.p, d.rb32.p, d.rb.n, s);
-        to_f32_launch(d.chol.p, d.chol32.p, d.chol.n, s);
-        d.f32_tables = true;
-      }
-      if (d.term_c32_gen != d.list_gen) {
-        d.term_c32.alloc(d.term_c.n);
-        to_f32_launch(d.term_c.p, d.term_c32.p, d.term_c.n, s);
-        d.term_c32_gen = d.list_gen;
-      }
-      const int64_t nbf = (int64_t)d.Nrad * d.Nang;
-      if (!d.tiled) {
-        d.P32.alloc((size_t)nbf * nbf);
-        mat_to_f32_launch(P[i], ldp[i], d.P32.p, nbf, s);
-      }
-    }
+    if (fp32[i] && d.n_act > 0) prepare_f32(d, P[i], ldp[i], s);
     if (d.tiled && d.n_act > 0) {
       const size_t nt = (size_t)d.Nel * d.Nel * d.n_src * TILE2;
       if (fp32[i])
@@ -1595,6 +2065,14 @@ void atomic_batch_exchange(AtomicBatch &b, const double *const *P, const int64_t
     }
   // 5. the launch sequence: zero K, density tiles, cross- and in-element kernels
   std::vector<long long> sig{sF[n], spd.back(), spf.back()};
+  // the captured launches hold table addresses: sections that moved are a new graph
+  for (size_t o : {(size_t)(uintptr_t)base, oF, osF, opd, ospd, opf, ospf})
+    sig.push_back((long long)o);
+  for (int c = 0; c < 4; ++c)
+    for (int p = 0; p < 2; ++p) {
+      sig.push_back((long long)ok[c][p]);
+      sig.push_back((long long)osk[c][p]);
+    }
   for (int c = 0; c < 4; ++c)
     for (int p = 0; p < 2; ++p) {
       sig.push_back(sk[c][p].back());

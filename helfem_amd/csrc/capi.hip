@@ -134,12 +134,16 @@ void atomic_upload(hf_atomic *h) {
     }
   const int nlm = (int)lmL.size();
   std::vector<std::vector<std::pair<int, double>>> pairs(nlm);
+  d.h_lv = lv;
+  d.h_mv = mv;
+  d.h_g.assign((size_t)Na * Na * nL, 0.0);
   for (int k = 0; k < Na; ++k)
     for (int l = 0; l < Na; ++l) {
       const int M = mv[k] - mv[l];
       for (int L = std::max(std::abs(lv[k] - lv[l]), std::abs(M)); L <= lv[k] + lv[l]; ++L) {
         const double c = gaunt_coeff(lv[k], mv[k], L, M, lv[l], mv[k] - M);
         if (c == 0.0) continue;
+        d.h_g[((size_t)k * Na + l) * nL + L] = c;
         pairs[lmIndex[(size_t)L * (2 * Mmax + 1) + (M + Mmax)]].push_back({k * Na + l, c});
       }
     }

@@ -29,6 +29,18 @@ constexpr int KL_BATCH = 64;
 constexpr int K2_SLOTS = 32, K2_THREADS = HFG_K2_THREADS, K2_WAVES = K2_THREADS / 64, K2_ROWS = 3;
 static_assert(K2_THREADS % 64 == 0 && K2_THREADS <= 1024, "two-step exchange workgroup");
 
+// cross-element atomic exchange by density classes: waves per workgroup, units
+// per workgroup, rows per unit, sources per entry, most tiles in LDS at once
+// (the FP64 tiles then take 144 of 160 KB)
+// used from KC_MIN_TERMS terms per coupled (output block, L) on (lmax = 5: 12),
+// and KC_MIN_WGS workgroups in the launch; exchange of an m-diagonal density
+// without / with it: lmax 4, 20 elements 770 / 799 us (FP32 691 / 669); lmax 5,
+// 25 elements 2493 / 1943; lmax 6, 10 elements 891 / 758, 4 elements 287 / 304
+constexpr double KC_MIN_TERMS = 10.0;
+constexpr int KC_MIN_WGS = 256;
+constexpr int KC_WAVES = 16, KC_UNITS = 8, KC_ROWS = 4, KC_SRC = 4, KC_TILES = 72;
+// waves per unit: the multipoles of a unit are split over them
+__host__ __device__ constexpr int kc_split(int units) { return units > 4 ? KC_WAVES / KC_UNITS : 12 / units > 4 ? 4 : 12 / units; }
 // in-element diatomic exchange with folded operators: threads (16 waves of two
 // rows), so columns, per workgroup; bytes of one (L,|M|, element) operator at
 // the largest element size
@@ -238,6 +250,27 @@ struct AtomicDevice {
   DevArray<int> src_blk, term_tile;
   int n_src = 0;
   bool tiled = false;
+  // Cross-element exchange by density classes (k_atomic_kc_off), used with the
+  // tiled density.  The density blocks (i,l) of one class (m_i - m_l, parities
+  // of l_i and l_l) are consecutive tiles; a workgroup holds a class (or a
+  // stage of it) of one element pair in LDS and its waves a unit each: up to
+  // KC_ROWS rows j of one column k, of one m and parity.  Per unit and stage:
+  // blocks (L, entries); per entry up to KC_SRC consecutive tiles of one row
+  // shell i with their weights g(k,L,l), and the rows' 4pi/(2L+1) g(j,L,i).
+  bool kc = false, finite = true;         // finite: no infinite or NaN block norm
+  int n_wg_kc = 0;                        // workgroups per element pair
+  int kc_rows = 0, kc_tiles = 0, kc_parts = 0;         // most rows of a unit, tiles of a stage, partial row tiles of a workgroup
+  std::vector<int> h_lv, h_mv;
+  std::vector<double> h_g;                // [j][i][L] Gaunt coefficients (M = mj - mi)
+  DevArray<int4> kc_wg;                   // first unit, units, first stage, stages
+  DevArray<int2> kc_stage;                // first tile, tiles
+  DevArray<int> kc_jk, kc_ub;             // rows of a unit; its block range per stage (offset by kc_us)
+  DevArray<int> kc_us;
+  DevArray<int4> kc_blk;                  // (L, first entry, last entry + 1, 0)
+  DevArray<int> kc_eh;                    // per entry: first LDS tile | (tiles - 1) << 16
+  DevArray<double> kc_ec;                 // per entry: KC_ROWS row weights, KC_SRC source weights
+  DevArray<float> kc_ec32;
+  double flops_kc = 0.0, frad_off = 0.0;  // angular flops of this form, radial ones of the launch
   // FP32 copies for the reduced-precision exchange (built on first use)
   DevArray<float> rs32, rb32, chol32, term_c32, P32;
   bool f32_tables = false;

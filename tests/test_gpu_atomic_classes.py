@@ -1,0 +1,89 @@
+"""The cross-element atomic exchange by density classes (k_atomic_kc_off), forced
+on bases of every shape (HFGPU_EXCHANGE_CLASSES=1; by itself it takes large
+angular bases only) against the oracle and the one-block-at-a-time kernel (=0).
+
+Bar: FP64 1e-12 of max|K| against the oracle (src/atomic/TwoDBasis.cpp:880-999);
+FP32 1.25 times the other kernel's error on the same inputs or the roundings of
+one product (density, two weights, factor: 2^-24 each)."""
+import numpy as np
+import pytest
+
+import helfem_amd as H
+import oracle as O
+from helfem_amd.synthetic import random_symmetric
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-12
+
+
+def relerr(a, b):
+    return float(np.max(np.abs(a - b)) / max(np.max(np.abs(b)), 1e-300))
+
+
+def _bases(monkeypatch, ctx, args, kw):
+    """The basis with the kernel on and off; the choice is made at the first build."""
+    import torch
+    out = []
+    for env in ("1", "0"):
+        monkeypatch.setenv("HFGPU_EXCHANGE_CLASSES", env)
+        b = H.AtomicBasis(*args, ctx=ctx, **kw)
+        b.compute_tei()
+        out.append(b)
+    return out, lambda b, P, **k: b.exchange(torch.as_tensor(P, device="cuda"), **k).cpu().numpy()
+
+
+@pytest.mark.parametrize("lmax,mmax,nel,nodes", [(0, 0, 2, 15), (2, 2, 3, 16), (3, 1, 2, 5), (4, 2, 2, 3)])
+def test_against_oracle(lmax, mmax, nel, nodes, gpu_ctx, monkeypatch):
+    print(f"[gpu] class exchange lmax={lmax} mmax={mmax}, {nel} elements, {nodes} nodes", flush=True)
+    (on, off), K = _bases(monkeypatch, gpu_ctx, (10, lmax, mmax, nel), dict(nnodes=nodes))
+    ob = O.AtomicBasis(10, lmax, mmax, nel, nnodes=nodes)
+    ob.compute_tei()
+    S = random_symmetric(ob.Nbf, seed=2201)
+    G = S + 0.3 * np.triu(random_symmetric(ob.Nbf, seed=2202))
+    sh = np.arange(ob.Nbf) // on.Nrad
+    rng = np.random.default_rng(2203)
+    keep = rng.random((on.Nang, on.Nang)) < 0.5
+    D = S * (keep & keep.T)[sh][:, sh]  # runs of tiles with gaps
+    for P in (S, G, D):
+        Kr = ob.exchange(P)
+        monkeypatch.setenv("HFGPU_EXCHANGE_CLASSES", "1")
+        assert relerr(K(on, P), Kr) <= TOL
+        e1 = relerr(K(on, P, precision="fp32"), Kr)
+        monkeypatch.setenv("HFGPU_EXCHANGE_CLASSES", "0")
+        assert relerr(K(off, P), Kr) <= TOL
+        e0 = relerr(K(off, P, precision="fp32"), Kr)
+        print(f"fp32 error {e1:.2e}, other kernel {e0:.2e}", flush=True)
+        assert e1 <= max(1.25 * e0, 4 * 2.0 ** -24)
+
+
+def test_several_stages(gpu_ctx, monkeypatch):
+    """lmax = 9: 167 tiles of one class, three stages of LDS, runs of five
+    sources; the oracle takes minutes here, the other kernel stands in."""
+    print("[gpu] class exchange in several stages", flush=True)
+    (on, off), K = _bases(monkeypatch, gpu_ctx, (10, 9, 9, 2), dict(nnodes=3))
+    P = random_symmetric(on.Nbf, seed=2204)
+    m = np.repeat(on.mval, on.Nrad)
+    P[m[:, None] != m[None, :]] = 0.0
+    monkeypatch.setenv("HFGPU_EXCHANGE_CLASSES", "1")
+    K1 = K(on, P)
+    monkeypatch.setenv("HFGPU_EXCHANGE_CLASSES", "0")
+    assert relerr(K1, K(off, P)) <= TOL
+
+
+def test_yukawa_and_infinite_density(gpu_ctx, monkeypatch):
+    """The Yukawa exchange through its own factors, and an infinite entry that
+    reaches only the blocks coupled to its own."""
+    import torch
+    print("[gpu] class exchange, Yukawa factors and an infinite entry", flush=True)
+    (on, off), K = _bases(monkeypatch, gpu_ctx, (4, 3, 2, 3), dict(nnodes=8))
+    P = random_symmetric(on.Nbf, seed=2205)
+    R, N = [], []
+    Q = P.copy()
+    Q[2, 3] = Q[3, 2] = np.inf
+    for env, b in (("1", on), ("0", off)):
+        monkeypatch.setenv("HFGPU_EXCHANGE_CLASSES", env)
+        b.compute_yukawa(0.4)
+        R.append(b.rs_exchange(torch.as_tensor(P, device="cuda")).cpu().numpy())
+        N.append(K(b, Q))
+    assert relerr(R[0], R[1]) <= TOL
+    assert np.array_equal(np.isfinite(N[0]), np.isfinite(N[1]))
