@@ -69,41 +69,51 @@ void xc_upload(hf_dftgrid *g) {
   int mmax = 0;
   for (int m : mv) mmax = std::max(mmax, std::abs(m));
   d.dmax = (g->atomic || g->full3d) ? 2 * mmax : 0;
-  const int nd = 2 * d.dmax + 1;
-  // shell pairs within reach of the phi grid, numbered row by row
-  std::vector<int> rstart(Na + 1, 0), rb, rp;
-  std::vector<std::vector<int>> byd_a(nd), byd_b(nd), byd_p(nd);
-  int np = 0;
-  for (int a = 0; a < Na; ++a) {
-    for (int b = 0; b < Na; ++b) {
-      const int dd = mv[a] - mv[b];
-      if (std::abs(dd) > d.dmax) continue;
-      rb.push_back(b);
-      rp.push_back(np);
-      byd_a[dd + d.dmax].push_back(a);
-      byd_b[dd + d.dmax].push_back(b);
-      byd_p[dd + d.dmax].push_back(np);
-      ++np;
-    }
-    rstart[a + 1] = (int)rb.size();
-  }
-  d.npair = np;
-  // pairs renumbered by class d (x = position in the d-sorted order): the
-  // work arrays D, W are indexed by x, and rx maps each row-list entry to it
-  std::vector<int> dstart(nd + 1, 0), da, db, px(np), xd;
+  const int nd = d.dmax + 1, nk = g->mang / 2 + 1;
+  d.nk = nk;
+  // shell pairs within reach of the phi grid, once each (m_a >= m_b), by class
+  // d = m_a - m_b
+  std::vector<int2> pab;
+  std::vector<int> xd, xstart(nd + 1, 0), pstart;
+  int all = 0;
   for (int dd = 0; dd < nd; ++dd) {
-    for (size_t j = 0; j < byd_p[dd].size(); ++j) px[byd_p[dd][j]] = (int)da.size() + (int)j;
-    da.insert(da.end(), byd_a[dd].begin(), byd_a[dd].end());
-    db.insert(db.end(), byd_b[dd].begin(), byd_b[dd].end());
-    xd.insert(xd.end(), byd_a[dd].size(), dd);
-    dstart[dd + 1] = (int)da.size();
+    for (int a = 0; a < Na; ++a)
+      for (int b = 0; b < Na; ++b) {
+        if (mv[a] - mv[b] != dd) continue;
+        all += dd > 0 ? 2 : 1;
+        if (dd == 0 && b < a) continue;
+        pab.push_back(make_int2(a, b));
+        xd.push_back(dd);
+      }
+    xstart[dd + 1] = (int)pab.size();
   }
-  std::vector<int> rx(rp.size());
-  for (size_t q = 0; q < rp.size(); ++q) rx[q] = px[rp[q]];
-  const size_t lds = sizeof(double) * ((size_t)np + (size_t)g->lang * nd + (size_t)g->lang * g->mang);
+  const int np = (int)pab.size();
+  d.npair = np;
+  d.npair_all = all;
+  // size limits of the entry point, counted unfolded
+  const size_t unfolded = (size_t)all + (size_t)g->lang * (2 * d.dmax + 1) + (size_t)g->lang * g->mang;
+  const size_t lds = sizeof(double) * unfolded;
   if (lds > 64 * 1024)
     throw Error(HF_EINVAL, "angular basis and DFT grid too large for one workgroup's LDS (need shell pairs + "
                            "lang*(4 mmax + 1) + lang*mang <= 8192)");
+  // pieces of the class sums: runs of at most 32 pairs of one class, longer ones
+  // where the LDS of an evaluation would pass its unfolded size (a single piece
+  // of a single class takes none)
+  std::vector<int4> piece;
+  for (int len = 32;; len *= 2) {
+    piece.clear();
+    pstart.assign(1, 0);
+    for (int dd = 0; dd < nd; ++dd) {
+      for (int q = xstart[dd]; q < xstart[dd + 1]; q += len)
+        piece.push_back(make_int4(dd, q, std::min(xstart[dd + 1], q + len), 0));
+      pstart.push_back((int)piece.size());
+    }
+    d.npiece = (int)piece.size();
+    const bool fits = (size_t)np + (size_t)g->lang * (nd + std::max(nk, d.npiece)) <= unfolded &&
+                      xc_gga_point_lds(d, 1, false) <= xc_gga_limit_lds(d, 1, false) &&
+                      xc_gga_point_lds(d, 1, true) <= xc_gga_limit_lds(d, 1, true);
+    if (len >= np || fits) break;
+  }
   d.lds_pol_ok = 2 * lds <= 64 * 1024;
   if (sizeof(double) * ((size_t)nrad * TILE + 4 * TILE2) > 64 * 1024) throw Error(HF_EINVAL, "radial quadrature too large");
   std::vector<double> xq, wq, xt, wt;
@@ -116,16 +126,17 @@ void xc_upload(hf_dftgrid *g) {
   }
   const double dphi = 2.0 * kPi / g->mang;
   std::vector<double> R((size_t)Nel * nrad * TILE, 0.0), wpt((size_t)Nel * nrad * g->lang);
-  std::vector<double> th((size_t)g->lang * Na), cs((size_t)nd * g->mang);
+  std::vector<double> th((size_t)g->lang * Na), cs((size_t)nd * nk), pw(nk);
   for (int t = 0; t < g->lang; ++t)
     for (int a = 0; a < Na; ++a) th[(size_t)t * Na + a] = theta_value(lv[a], mv[a], xt[t]);
   for (int dd = 0; dd < nd; ++dd)
-    for (int k = 0; k < g->mang; ++k) cs[(size_t)dd * g->mang + k] = std::cos(double(dd - d.dmax) * (k * dphi));
+    for (int k = 0; k < nk; ++k) cs[(size_t)dd * nk + k] = std::cos(double(dd) * (k * dphi));
+  for (int k = 0; k < nk; ++k) pw[k] = k == 0 || 2 * k == g->mang ? 1.0 : 2.0;
   // Theta_a(t) Theta_b(t) per pair x, in both orders ([t][x] and [x][t])
   std::vector<double> thx((size_t)g->lang * np), thxt((size_t)np * g->lang);
   for (int t = 0; t < g->lang; ++t)
     for (int x = 0; x < np; ++x) {
-      const double v = th[(size_t)t * Na + da[x]] * th[(size_t)t * Na + db[x]];
+      const double v = th[(size_t)t * Na + pab[x].x] * th[(size_t)t * Na + pab[x].y];
       thx[(size_t)t * np + x] = v;
       thxt[(size_t)x * g->lang + t] = v;
     }
@@ -161,22 +172,21 @@ void xc_upload(hf_dftgrid *g) {
   d.R.upload(R, s);
   d.wpt.upload(wpt, s);
   d.cs.upload(cs, s);
-  d.rstart.upload(rstart, s);
-  d.rb.upload(rb, s);
-  d.rx.upload(rx, s);
-  d.dstart.upload(dstart, s);
+  d.pw.upload(pw, s);
+  d.pab.upload(pab, s);
   d.xd.upload(xd, s);
+  d.piece.upload(piece, s);
+  d.pstart.upload(pstart, s);
   d.thx.upload(thx, s);
   d.thxt.upload(thxt, s);
   // gradient tables (GGA): d/dr R (atomic, R = B/r) or d/dmu R (diatomic,
   // R = B), the inverse scale factors of the three gradient components per
-  // point, sin(d phi), d/dtheta (Theta_a Theta_b), and the transposed pair of
-  // each row-list entry; the host vectors live until the stream sync below
+  // point, sin(d phi), d/dtheta (Theta_a Theta_b); the host vectors live until
+  // the stream sync below
   std::vector<double> dR((size_t)Nel * nrad * TILE, 0.0), gsc((size_t)Nel * nrad * g->lang * 3);
-  std::vector<double> sn((size_t)nd * g->mang), thd((size_t)g->lang * np), thdt((size_t)np * g->lang);
+  std::vector<double> sn((size_t)nd * nk), thd((size_t)g->lang * np), thdt((size_t)np * g->lang);
   std::vector<double> thdd((size_t)g->lang * np), thddt((size_t)np * g->lang), thmm((size_t)g->lang * np),
       thmmt((size_t)np * g->lang);
-  std::vector<int> rxT(rb.size());
   {
     for (int e = 0; e < Nel; ++e) {
       const Blk v = g->atomic ? rad.rderiv(xq, e) : rad.values(1, xq, e);
@@ -202,36 +212,27 @@ void xc_upload(hf_dftgrid *g) {
       }
     }
     for (int dd = 0; dd < nd; ++dd)
-      for (int k = 0; k < g->mang; ++k) sn[(size_t)dd * g->mang + k] = std::sin(double(dd - d.dmax) * (k * dphi));
+      for (int k = 0; k < nk; ++k) sn[(size_t)dd * nk + k] = std::sin(double(dd) * (k * dphi));
     std::vector<double> dth((size_t)g->lang * Na);
     for (int t = 0; t < g->lang; ++t)
       for (int a = 0; a < Na; ++a) dth[(size_t)t * Na + a] = theta_deriv(lv[a], mv[a], xt[t]);
     for (int t = 0; t < g->lang; ++t)
       for (int x = 0; x < np; ++x) {
-        const size_t A = (size_t)t * Na + da[x], B = (size_t)t * Na + db[x];
+        const size_t A = (size_t)t * Na + pab[x].x, B = (size_t)t * Na + pab[x].y;
         const double v = dth[A] * th[B] + th[A] * dth[B];
         thd[(size_t)t * np + x] = v;
         thdt[(size_t)x * g->lang + t] = v;
-        const double vd = dth[A] * dth[B], vm = double(mv[da[x]] * mv[db[x]]) * th[A] * th[B];
+        const double vd = dth[A] * dth[B], vm = double(mv[pab[x].x] * mv[pab[x].y]) * th[A] * th[B];
         thdd[(size_t)t * np + x] = vd;
         thddt[(size_t)x * g->lang + t] = vd;
         thmm[(size_t)t * np + x] = vm;
         thmmt[(size_t)x * g->lang + t] = vm;
-      }
-    std::vector<int> xid((size_t)Na * Na, -1);
-    for (int a = 0; a < Na; ++a)
-      for (int q = rstart[a]; q < rstart[a + 1]; ++q) xid[(size_t)a * Na + rb[q]] = rx[q];
-    for (int a = 0; a < Na; ++a)
-      for (int q = rstart[a]; q < rstart[a + 1]; ++q) {
-        rxT[q] = xid[(size_t)rb[q] * Na + a];
-        need(rxT[q] >= 0, "pair list is not symmetric");
       }
     d.dR.upload(dR, s);
     d.gsc.upload(gsc, s);
     d.sn.upload(sn, s);
     d.thd.upload(thd, s);
     d.thdt.upload(thdt, s);
-    d.rxT.upload(rxT, s);
     d.thdd.upload(thdd, s);
     d.thddt.upload(thddt, s);
     d.thmm.upload(thmm, s);
@@ -267,7 +268,7 @@ void eval_fxc(hf_dftgrid *g, int x_func, int c_func, const double *P, int64_t ld
   XCGridDevice &d = g->dev;
   const bool gen = xc_generic(x_func, c_func);
   if (gen) {
-    if (xc_point_lds(d, x_func, c_func, Pb != nullptr) > 160 * 1024)
+    if (xc_limit_lds(d, x_func, c_func, Pb != nullptr) > 160 * 1024)
       throw Error(HF_EINVAL, "angular basis and DFT grid too large for one workgroup's LDS in the GGA evaluation");
     d.E.alloc(d.D.n);
     d.Y.alloc(d.W.n);

@@ -407,32 +407,37 @@ struct DiatomicDevice {
 // Atomic grid: R = B/r at the radial Chebyshev points, Theta_a = Y_a(theta, 0)
 // on the cos(theta) rule, mang even phi points.  Pure-m diatomic grid: R = B
 // at the mu points, Theta_a = Y_a(nu, 0), one phi "point" (the phi integral is
-// analytic), only shell pairs with m_a = m_b.  Shell pairs (a, b) with
-// |m_a - m_b| <= dmax are numbered p = 0..npair-1.
+// analytic), only shell pairs with m_a = m_b.  Everything on the grid is
+// symmetric in a pair's shells and even in phi, so the shell pairs {a, b} with
+// 0 <= d = m_a - m_b <= dmax are numbered once each, x = 0..npair-1 by class d,
+// and the phi points k <= mang / 2 stand for k and mang - k.
 struct XCGridDevice {
-  int Nel = 0, Nrad = 0, Nang = 0, nrad = 0, lang = 0, mang = 0, dmax = 0, npair = 0;
+  int Nel = 0, Nrad = 0, Nang = 0, nrad = 0, lang = 0, mang = 0, dmax = 0, npair = 0, npiece = 0, nk = 0;
+  int npair_all = 0;         // ordered pairs, for the size limits of the entry points
   int64_t Nbf = 0;
-  bool lds_pol_ok = false;   // the polarized point kernel's LDS fits
+  bool lds_pol_ok = false;   // the polarized evaluation is within those limits
   DevArray<int> first, ni, skip;
   DevArray<long long> poff;
   DevArray<double> R;        // [Nel][nrad][TILE]
   DevArray<double> wpt;      // [Nel][nrad][lang] quadrature weight (phi weight included)
-  DevArray<double> cs;       // [2 dmax + 1][mang] cos(d phi_k)
-  DevArray<int> rstart, rb, rx;       // pairs of row a: b and pair index x
-  DevArray<int> dstart, xd;           // pairs x bucketed by d = m_a - m_b + dmax; d of each x
+  DevArray<double> cs;       // [dmax + 1][nk] cos(d phi_k)
+  DevArray<double> pw;       // [nk] phi points that k stands for (1 or 2)
+  DevArray<int2> pab;        // per pair: shells (a, b), m_a >= m_b
+  DevArray<int> xd;          // per pair: class d
+  DevArray<int4> piece;      // runs of pairs of one class: (d, first, last + 1, 0)
+  DevArray<int> pstart;      // [dmax + 2]: pieces of each class
   DevArray<double> thx, thxt;         // Theta_a(t) Theta_b(t): [lang][npair] and [npair][lang]
-  DevArray<double> D, W;     // D [Nel][nrad][npair], W [Nel][npair][nrad]
+  DevArray<double> D, W;     // [Nel][nrad][npair]
   DevArray<double> Db, Wb;   // second spin of a polarized evaluation
   // gradient (GGA) tables and work arrays
   DevArray<double> dR;       // [Nel][nrad][TILE] d/dr (atomic) or d/dmu (diatomic) of R
   DevArray<double> gsc;      // [Nel][nrad][lang][3] inverse scale factors 1/h of the gradient components
-  DevArray<double> sn;       // [2 dmax + 1][mang] sin(d phi_k)
+  DevArray<double> sn;       // [dmax + 1][nk] sin(d phi_k)
   DevArray<double> thd, thdt;  // d/dtheta (Theta_a Theta_b): [lang][npair] and [npair][lang]
-  DevArray<int> rxT;         // per row-list entry: pair index of the transposed pair (b, a)
-  DevArray<double> E, Y;     // E [Nel][nrad][npair] (d/dr on the row), Y [Nel][npair][nrad]
+  DevArray<double> E, Y;     // [Nel][nrad][npair] (E: d/dr on the row)
   DevArray<double> Eb, Yb;
   // kinetic energy density (meta-GGA): Theta'_a Theta'_b and m_a m_b Theta_a Theta_b
-  // ([lang][npair] and [npair][lang]), F = R' P R' [Nel][nrad][npair], Z [Nel][npair][nrad]
+  // ([lang][npair] and [npair][lang]), F = R' P R', Z [Nel][nrad][npair]
   DevArray<double> thdd, thddt, thmm, thmmt;
   DevArray<double> F, Z, Fb, Zb;
   DevArray<double> part;     // [Nel*nrad][3]: Exc, Nel and Ekin (integral of tau) partial sums
@@ -526,8 +531,12 @@ void xc_grid_launch(XCGridDevice &g, int xf, int cf, double thr, const double *P
 // true when (xf, cf) is not the plain lda_x + lda_c_vwn pair: the general
 // point kernel (GGA terms, any supported functional) runs
 bool xc_generic(int xf, int cf);
-// dynamic LDS of the point kernel that xc_grid_launch will use
-size_t xc_point_lds(const XCGridDevice &g, int xf, int cf, bool pol);
+// LDS bytes by which the entry points limit the general evaluation (shell pairs
+// and phi points counted unfolded)
+size_t xc_limit_lds(const XCGridDevice &g, int xf, int cf, bool pol);
+// LDS bytes of the general point kernel for ns spins, and the unfolded limit
+size_t xc_gga_point_lds(const XCGridDevice &g, int ns, bool tau);
+size_t xc_gga_limit_lds(const XCGridDevice &g, int ns, bool tau);
 // true when the pair needs the kinetic energy density (meta-GGA)
 bool xc_tau(int xf, int cf);
 

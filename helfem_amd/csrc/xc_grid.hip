@@ -46,6 +46,16 @@
 // S_d = sum_k (w vtau / 2) cos(d phi_k), per pair
 //   H += sum_i R'_r R'_s Z(x) + R_r R_s sum_t (c_2^2 Theta'_a Theta'_b + c_3^2 m_a m_b Theta_a Theta_b) S_d,
 //   Z(x) = sum_t c_1^2 Theta_a Theta_b S_d.
+//
+// Everything above is symmetric in the two shells of a pair and even in phi
+// (g_3 and U_3 are odd, and enter with the odd sin), so a pair {a, b} is taken
+// once, with D and F of both orders added, E of both orders with the derivative
+// on the row, one W and Y for H_ab and H_ba = H_ab', classes d >= 0, and the phi
+// points k <= mang / 2 with weight 2 for k and mang - k.  That and one radial
+// workgroup per run of pairs instead of per shell or pair: J + XC builds of Xe
+// (lmax 6, 25 elements, LDA) 2.57 -> 1.56 ms, O (lmax 3, 12 elements, polarized
+// PBE) 0.75 -> 0.42 ms, N2 (16 shells per |m| <= 2, 7 elements, pure-m LDA)
+// 1.59 -> 0.98 ms.
 #include "hfgpu_internal.hpp"
 #include "device_common.hpp"
 #include "xc_func.hpp"
@@ -145,142 +155,233 @@ struct XCArgs {
   int64_t ldp;
   double *H;
   int64_t ldh;
-  int Nel, Nang, nrad, lang, mang, nd, xf, cf, npair;
+  int Nel, Nang, nrad, lang, nk, nd, npiece, xf, cf, npair;
   double thr;
   const int *first, *ni, *skip;
   const long long *poff;
-  const int *rstart, *rb, *rx, *dstart, *xd;
-  const double *R, *wpt, *thx, *thxt, *cs;
+  const int2 *pab;
+  const int *xd, *pstart;
+  const int4 *piece;
+  const double *R, *wpt, *thx, *thxt, *cs, *pw;
   double *D, *W, *part;
   double *Db, *Wb;  // second spin (polarized evaluation), else null
-  // gradient terms (k_xc_rad_in<true>, k_xc_point_gga, k_xc_rad_out<true>);
+  // gradient terms (k_xc_rad_in<1>, k_xc_point_gga, k_xc_rad_out<1>);
   // gsc [Nel][nrad][lang][3] = 1/(h_1, h_2, h_3) per point
   const double *dR, *gsc, *sn, *thd, *thdt;
-  const int *rxT;
   double *E, *Y, *Eb, *Yb;
   // kinetic energy density terms (meta-GGA)
   const double *thdd, *thddt, *thmm, *thmmt;
   double *F, *Z, *Fb, *Zb;
 };
 
-// One workgroup per (element, shell a).  The pairs (a, b) of row a go in
-// groups of J = 256 / nrad (1 to 8, xc_pairs_per_group): their P tiles are staged in LDS, and
-// thread t takes (pair t / nrad, radial point t % nrad), so every thread of
-// the workgroup has a point (J nrad of 256 busy).  A thread keeps R_i in
-// registers; the R rows sit in LDS at an odd stride (17), so neighbouring
-// points read different banks, and the tile reads of a wave touch at most two
-// tiles (broadcast).  R and the tiles are zero outside the element.
-constexpr int XC_RS = TILE + 1;
+// Both radial kernels take a run of consecutive pairs {a, b} of one element per
+// workgroup and the radial points in runs of XR_PTS, so that the arrays
+// [point][pair] are read and written in runs of pairs.
+constexpr int XR_PAIRS = 16, XR_PTS = 80, XR_RS = TILE + 1, XR_WS = XR_PAIRS + 1;
+// k_xc_rad_in: XI_J pairs contracted at a time by 40 threads each, two points
+// per thread; XI_PAIRS pairs per workgroup, XI_J where that leaves CUs idle
+constexpr int XI_J = 6, XI_PAIRS = 12, XI_WS = XI_PAIRS + 1, XI_PT = XR_PTS / 2;
+static_assert(XI_J * XI_PT <= NT && XI_PAIRS % XI_J == 0, "pairs of a batch");
 
-__host__ __device__ inline int xc_pairs_per_group(int nrad) { return min(8, max(1, NT / nrad)); }
-
-// MODE 0: D only (LDA); 1: also E (GGA); 2: also F = sum R'_r P R'_s (meta-GGA)
+// D(x) = sum_rs R_r (P_ab + P_ba') R_s of every pair and radial point (P_aa for
+// a = b), folded over r <= s: 136 terms; with GGA also E = sum_rs R'_r (P_ab +
+// P_ba) R_s (the derivative on the row), with tau F = sum_rs R'_r (P_ab + P_ba')
+// R'_s.  A thread takes two points of a pair with R in registers, so that each
+// broadcast tile read serves two; the R rows sit in LDS at an odd stride.  R and
+// the tiles are zero outside the element.  blockIdx.y: spin.  Bound by the LDS
+// tile reads and the chain shell offsets -> P -> LDS of each batch.  Xe LDA 260
+// (a workgroup per shell, ordered pairs) -> 240 (one point per thread, folded)
+// -> 169 us; O polarized PBE 2 x 75 -> 41 us, there with XI_J pairs per workgroup
+// (XI_PAIRS: half as many workgroups, fewer than 512 leave CUs idle).
+// MODE 0: D only (LDA); 1: also E (GGA); 2: also F (meta-GGA)
 template <int MODE>
-__global__ void __launch_bounds__(NT) k_xc_rad_in(XCArgs A) {
-  const int e = blockIdx.x / A.Nang, a = blockIdx.x - e * A.Nang;
+__global__ void __launch_bounds__(NT) k_xc_rad_in(XCArgs A, XCArgs B, int per) {
+  if (blockIdx.y) A = B;
+  const int groups = (A.npair + per - 1) / per;
+  const int e = blockIdx.x / groups, x0 = (blockIdx.x - e * groups) * per;
   const int t = threadIdx.x;
   const int ni = A.ni[e], f0 = A.first[e];
-  const int J = xc_pairs_per_group(A.nrad);
+  const int np = min(per, A.npair - x0);
   extern __shared__ double sm[];
-  double *sR = sm;                                        // [nrad][XC_RS]
-  double *sdR = sm + A.nrad * XC_RS;                      // [nrad][XC_RS] with GGA
-  double *sP = sm + (MODE ? 2 : 1) * A.nrad * XC_RS;      // [J][TILE2]
-  for (int q = t; q < A.nrad * TILE; q += NT) {
-    sR[(q >> 4) * XC_RS + (q & 15)] = A.R[(size_t)e * A.nrad * TILE + q];
-    if (MODE) sdR[(q >> 4) * XC_RS + (q & 15)] = A.dR[(size_t)e * A.nrad * TILE + q];
-  }
-  const int q0 = A.rstart[a], q1 = A.rstart[a + 1];
-  for (int qb = q0; qb < q1; qb += J) {
-    __syncthreads();
-    for (int x = t; x < J * TILE2; x += NT) {
-      const int j = x >> 8, y = x & 255, r = y & 15, s = y >> 4, q = qb + j;
-      double v = 0.0;
-      if (q < q1 && r < ni && s < ni) {
-        const long long row = grid_row(A.skip, A.poff, a, f0 + r), col = grid_row(A.skip, A.poff, A.rb[q], f0 + s);
-        if (row >= 0 && col >= 0) v = A.P[row + col * A.ldp];
-      }
-      sP[x] = v;
+  double *sR = sm;                                   // [XR_PTS][XR_RS]
+  double *sdR = sR + XR_PTS * XR_RS;                 // with GGA
+  double *sS = sR + (MODE ? 2 : 1) * XR_PTS * XR_RS;  // [XI_J][TILE2], folded to r <= s
+  double *sG = sS + XI_J * TILE2;                    // with GGA: not folded
+  double *sO = sS + (MODE ? 2 : 1) * XI_J * TILE2;   // [MODE + 1][XR_PTS][XI_WS]
+  const int r = t & 15, s = t >> 4;
+  const int j = t / XI_PT, i = t - j * XI_PT;
+  for (int i0 = 0; i0 < A.nrad; i0 += XR_PTS) {
+    const int nq = min(XR_PTS, A.nrad - i0);
+    for (int q = t; q < XR_PTS * TILE; q += NT) {
+      const bool in = (q >> 4) < nq;
+      sR[(q >> 4) * XR_RS + (q & 15)] = in ? A.R[((size_t)e * A.nrad + i0) * TILE + q] : 0.0;
+      if (MODE) sdR[(q >> 4) * XR_RS + (q & 15)] = in ? A.dR[((size_t)e * A.nrad + i0) * TILE + q] : 0.0;
     }
-    __syncthreads();
-    for (int item = t; item < J * A.nrad; item += NT) {
-      const int j = item / A.nrad, i = item - j * A.nrad, q = qb + j;
-      if (q >= q1) continue;
-      const double *Pt = sP + j * TILE2;
-      const double *Ri = sR + i * XC_RS, *dRi = sdR + i * XC_RS;
-      double ri[TILE];
+    for (int xb = 0; xb < np; xb += XI_J) {
+      __syncthreads();
 #pragma unroll
-      for (int s = 0; s < TILE; ++s) ri[s] = Ri[s];
-      double d = 0.0, eg = 0.0, fk = 0.0;
-#pragma unroll
-      for (int r = 0; r < TILE; ++r) {
-        double tr = 0.0, trd = 0.0;
-#pragma unroll
-        for (int s = 0; s < TILE; ++s) {
-          tr += Pt[r + TILE * s] * ri[s];
-          if (MODE == 2) trd += Pt[r + TILE * s] * dRi[s];
+      for (int jj = 0; jj < XI_J; ++jj) {
+        double gv = 0.0;
+        if (xb + jj < np && r < ni && s < ni) {
+          const int2 ab = A.pab[x0 + xb + jj];
+          const long long ra = grid_row(A.skip, A.poff, ab.x, f0 + r), cb = grid_row(A.skip, A.poff, ab.y, f0 + s);
+          if (ra >= 0 && cb >= 0) gv = A.P[ra + cb * A.ldp];
+          if (ab.x != ab.y) {
+            const long long rb = grid_row(A.skip, A.poff, ab.y, f0 + r), ca = grid_row(A.skip, A.poff, ab.x, f0 + s);
+            if (rb >= 0 && ca >= 0) gv += A.P[rb + ca * A.ldp];
+          }
         }
-        d += ri[r] * tr;
-        if (MODE) eg += dRi[r] * tr;
-        if (MODE == 2) fk += dRi[r] * trd;
+        sS[jj * TILE2 + t] = gv;
+        if (MODE) sG[jj * TILE2 + t] = gv;
       }
-      const size_t o = ((size_t)e * A.nrad + i) * A.npair + A.rx[q];
-      A.D[o] = d;
-      if (MODE) A.E[o] = eg;
-      if (MODE == 2) A.F[o] = fk;
+      __syncthreads();
+      if (r < s)  // only r > s is read
+#pragma unroll
+        for (int jj = 0; jj < XI_J; ++jj) sS[jj * TILE2 + t] += sS[jj * TILE2 + s + TILE * r];
+      __syncthreads();
+      if (j < XI_J && xb + j < np) {
+        const double *St = sS + j * TILE2, *Gt = sG + j * TILE2;
+        const double *dR0 = sdR + i * XR_RS, *dR1 = dR0 + XI_PT * XR_RS;
+        double r0[TILE], r1[TILE];
+#pragma unroll
+        for (int c = 0; c < TILE; ++c) {
+          r0[c] = sR[i * XR_RS + c];
+          r1[c] = sR[(i + XI_PT) * XR_RS + c];
+        }
+        double d0 = 0.0, d1 = 0.0;
+#pragma unroll
+        for (int c = 0; c < TILE; ++c) {
+          double t0 = 0.0, t1 = 0.0;
+#pragma unroll
+          for (int k = 0; k <= c; ++k) {
+            const double v = St[k + TILE * c];
+            t0 += v * r0[k];
+            t1 += v * r1[k];
+          }
+          d0 += r0[c] * t0;
+          d1 += r1[c] * t1;
+        }
+        double *o = sO + i * XI_WS + xb + j;
+        o[0] = d0;
+        o[XI_PT * XI_WS] = d1;
+        if (MODE) {
+          double e0 = 0.0, e1 = 0.0;
+          for (int k = 0; k < TILE; ++k) {
+            double t0 = 0.0, t1 = 0.0;
+#pragma unroll
+            for (int c = 0; c < TILE; ++c) {
+              const double v = Gt[k + TILE * c];
+              t0 += v * r0[c];
+              t1 += v * r1[c];
+            }
+            e0 += dR0[k] * t0;
+            e1 += dR1[k] * t1;
+          }
+          o[XR_PTS * XI_WS] = e0;
+          o[(XR_PTS + XI_PT) * XI_WS] = e1;
+        }
+        if (MODE == 2) {
+#pragma unroll
+          for (int c = 0; c < TILE; ++c) {
+            r0[c] = dR0[c];
+            r1[c] = dR1[c];
+          }
+          double f0k = 0.0, f1k = 0.0;
+#pragma unroll
+          for (int c = 0; c < TILE; ++c) {
+            double t0 = 0.0, t1 = 0.0;
+#pragma unroll
+            for (int k = 0; k <= c; ++k) {
+              const double v = St[k + TILE * c];
+              t0 += v * r0[k];
+              t1 += v * r1[k];
+            }
+            f0k += r0[c] * t0;
+            f1k += r1[c] * t1;
+          }
+          o[2 * XR_PTS * XI_WS] = f0k;
+          o[(2 * XR_PTS + XI_PT) * XI_WS] = f1k;
+        }
+      }
     }
+    __syncthreads();
+    for (int q = t; q < nq * per; q += NT) {
+      const int p = q / per, x = q - p * per;
+      if (x >= np) continue;
+      const size_t o = ((size_t)e * A.nrad + i0 + p) * A.npair + x0 + x;
+      A.D[o] = sO[p * XI_WS + x];
+      if (MODE) A.E[o] = sO[(XR_PTS + p) * XI_WS + x];
+      if (MODE == 2) A.F[o] = sO[(2 * XR_PTS + p) * XI_WS + x];
+    }
+    __syncthreads();
   }
 }
 
-// One workgroup per (element, radial point).  With A.Db set the density of
-// the second spin is contracted alongside and the polarized functional used.
-// The pairs x are numbered by class d = m_a - m_b, so the class sums read
-// contiguous runs of D and of the Theta_a Theta_b table: thread (d, t) forms
-// C_d(t) from the [x][t] table (lanes of one d read consecutive t), and
-// thread x forms W(x) from the [t][x] table (lanes read consecutive x).
-// LDA point kernel workgroup: its 37 KB of LDS per radial point (Xe-sized
-// bases) lets four 256-thread groups share a CU, which measured fastest
-// (Xe: 256 / 512 / 1024 threads 0.82 / 1.10 / 0.98 ms).
-#ifndef HFG_XC_LDA_POINT_NT
-#define HFG_XC_LDA_POINT_NT 256
-#endif
-constexpr int LP_NT = HFG_XC_LDA_POINT_NT, LP_WAVES = LP_NT / 64;
-static_assert(LP_NT % 64 == 0 && LP_NT <= 1024, "LDA point kernel workgroup");
+// Class sums out[c][d][t] = sum_{x in d} table_c[x][t] src_c[x] of one radial
+// point: threads (piece, t) form partial sums over at most 32 pairs (lanes read
+// consecutive t), then (d, t) add the class' pieces in order.
+template <typename Table, typename Source>
+__device__ inline void class_sums(const XCArgs &A, int ncs, Table table, Source src, double *partial, double *out) {
+  const int lang = A.lang, npc = A.npiece * lang;
+  const bool one = A.npiece == 1 && A.nd == 1;  // the piece is the sum
+  if (one) partial = out;
+  for (int q = threadIdx.x; q < ncs * npc; q += blockDim.x) {
+    const int c = q / npc, r = q - c * npc, p = r / lang, tt = r - p * lang;
+    const int4 pc = A.piece[p];
+    const double *tab = table(c) + tt, *s = src(c);
+    double v = 0.0;
+#pragma unroll 4
+    for (int x = pc.y; x < pc.z; ++x) v += tab[(size_t)x * lang] * s[x];
+    partial[q] = v;
+  }
+  __syncthreads();
+  if (one) return;
+  for (int q = threadIdx.x; q < ncs * A.nd * lang; q += blockDim.x) {
+    const int c = q / (A.nd * lang), r = q - c * A.nd * lang, d = r / lang, tt = r - d * lang;
+    double v = 0.0;
+    for (int p = A.pstart[d]; p < A.pstart[d + 1]; ++p) v += partial[c * npc + p * lang + tt];
+    out[q] = v;
+  }
+  __syncthreads();
+}
 
-__global__ void __launch_bounds__(LP_NT) k_xc_point(XCArgs A) {
+// One workgroup per (element, radial point); with A.Db set the density of the
+// second spin is contracted alongside and the polarized functional used.  The
+// pairs x are numbered by class d = m_a - m_b, so the class sums read contiguous
+// runs of D and of the Theta_a Theta_b table, and thread x forms W(x) from the
+// [t][x] table (lanes read consecutive x).  Bound by the two Theta tables read
+// from L2 for every radial point (Xe: 2 x 0.35 MB) and the latency of the chain of
+// phases: Xe LDA 811 (ordered pairs, all phi points) -> 156 us, N2 pure-m
+// 629 -> 73 us.
+constexpr int LP_MAX = 512;
+
+__global__ void __launch_bounds__(LP_MAX) k_xc_point(XCArgs A) {
   const int e = blockIdx.x / A.nrad, i = blockIdx.x - e * A.nrad;
-  const int t = threadIdx.x;
-  const int np = A.npair, nd = A.nd, lang = A.lang, mang = A.mang, nang = lang * mang;
+  const int t = threadIdx.x, nt = blockDim.x;
+  const int np = A.npair, nd = A.nd, lang = A.lang, nk = A.nk, nang = lang * nk;
   const bool pol = A.Db != nullptr;
   const int ns = pol ? 2 : 1;
   extern __shared__ double sm[];
   double *sD = sm;                    // [ns][np]
   double *sC = sD + ns * np;          // [ns][nd][lang]
-  double *sV = sC + ns * nd * lang;   // [ns][lang][mang]
-  __shared__ double red[2 * LP_WAVES];
+  double *sV = sC + ns * nd * lang;   // [ns][lang][nk]; first the partial class sums
+  __shared__ double red[2 * LP_MAX / 64];
   const size_t row = ((size_t)e * A.nrad + i) * np;
-  for (int x = t; x < np; x += LP_NT) {
+  for (int x = t; x < np; x += nt) {
     sD[x] = A.D[row + x];
     if (pol) sD[np + x] = A.Db[row + x];
   }
   __syncthreads();
-  for (int q = t; q < ns * nd * lang; q += LP_NT) {
-    const int sp = q / (nd * lang), qq = q - sp * nd * lang;
-    const int d = qq / lang, tt = qq - d * lang;
-    const double *D = sD + sp * np;
-    double c = 0.0;
-    for (int x = A.dstart[d]; x < A.dstart[d + 1]; ++x) c += A.thxt[(size_t)x * lang + tt] * D[x];
-    sC[q] = c;
-  }
-  __syncthreads();
+  class_sums(A, ns, [&](int) { return A.thxt; }, [&](int c) { return sD + c * np; }, sV, sC);
   const double *wp = A.wpt + ((size_t)e * A.nrad + i) * lang;
   double ex = 0.0, ne = 0.0;
-  for (int q = t; q < nang; q += LP_NT) {
-    const int tt = q / mang, k = q - tt * mang;
+  for (int q = t; q < nang; q += nt) {
+    const int tt = q / nk, k = q - tt * nk;
     double ra = 0.0, rb = 0.0;
-    for (int d = 0; d < nd; ++d) ra += sC[d * lang + tt] * A.cs[(size_t)d * mang + k];
+    for (int d = 0; d < nd; ++d) ra += sC[d * lang + tt] * A.cs[(size_t)d * nk + k];
     if (pol)
-      for (int d = 0; d < nd; ++d) rb += sC[nd * lang + d * lang + tt] * A.cs[(size_t)d * mang + k];
-    const double w = wp[tt];
+      for (int d = 0; d < nd; ++d) rb += sC[nd * lang + d * lang + tt] * A.cs[(size_t)d * nk + k];
+    const double w = wp[tt] * A.pw[k];
     double exc, va, vb = 0.0;
     if (pol)
       lda_point_pol(A.xf, A.cf, ra, rb, A.thr, exc, va, vb);
@@ -295,37 +396,37 @@ __global__ void __launch_bounds__(LP_NT) k_xc_point(XCArgs A) {
   ne = wave_sum(ne);
   if ((t & 63) == 0) {
     red[t >> 6] = ex;
-    red[LP_WAVES + (t >> 6)] = ne;
+    red[LP_MAX / 64 + (t >> 6)] = ne;
   }
   __syncthreads();
   if (t == 0) {
     double sx = 0.0, sn = 0.0;
-    for (int w = 0; w < LP_WAVES; ++w) {
+    for (int w = 0; w < nt / 64; ++w) {
       sx += red[w];
-      sn += red[LP_WAVES + w];
+      sn += red[LP_MAX / 64 + w];
     }
     A.part[3 * ((size_t)e * A.nrad + i)] = sx;
     A.part[3 * ((size_t)e * A.nrad + i) + 1] = sn;
     A.part[3 * ((size_t)e * A.nrad + i) + 2] = 0.0;
   }
-  __syncthreads();
-  for (int q = t; q < ns * nd * lang; q += LP_NT) {
+  for (int q = t; q < ns * nd * lang; q += nt) {
     const int sp = q / (nd * lang), qq = q - sp * nd * lang;
     const int d = qq / lang, tt = qq - d * lang;
-    const double *V = sV + sp * nang + tt * mang;
+    const double *V = sV + sp * nang + tt * nk;
     double s = 0.0;
-    for (int k = 0; k < mang; ++k) s += V[k] * A.cs[(size_t)d * mang + k];
+    for (int k = 0; k < nk; ++k) s += V[k] * A.cs[(size_t)d * nk + k];
     sC[q] = s;
   }
   __syncthreads();
   for (int sp = 0; sp < ns; ++sp) {
     double *Wout = sp == 0 ? A.W : A.Wb;
     const double *C = sC + sp * nd * lang;
-    for (int x = t; x < np; x += LP_NT) {
+    for (int x = t; x < np; x += nt) {
       const double *Cd = C + A.xd[x] * lang;
       double w = 0.0;
+#pragma unroll 4
       for (int tt = 0; tt < lang; ++tt) w += A.thx[(size_t)tt * np + x] * Cd[tt];
-      Wout[((size_t)e * np + x) * A.nrad + i] = w;  // [element][x][point]: rad_out reads runs of points
+      Wout[row + x] = w;
     }
   }
 }
@@ -335,49 +436,37 @@ __global__ void __launch_bounds__(LP_NT) k_xc_point(XCArgs A) {
 // and with tau F), then its point values (w vrho, c_1 U_1, c_2 U_2, c_3 U_3
 // and with tau w vtau/2); region B holds the class sums (C, G, T and with tau
 // the three tau sums), then the class transforms (V_d - d Vphi_d, Vr_d,
-// Vtheta_d and with tau S_d).  Any supported functional pair runs here
-// (vsigma = 0 without a GGA part, vtau = 0 without a meta-GGA part).
+// Vtheta_d and with tau S_d); region C the pieces of the class sums.  Any
+// supported functional pair runs here (vsigma = 0 without a GGA part, vtau = 0
+// without a meta-GGA part).
 template <int MODE> struct GgaShape {
   static constexpr int nin = MODE == 2 ? 3 : 2;  // radial contractions per spin
   static constexpr int ncs = MODE == 2 ? 6 : 3;  // class sums per spin
   static constexpr int npv = MODE == 2 ? 5 : 4;  // point arrays per spin
 };
 
-size_t xc_gga_point_lds(int np, int nd, int lang, int mang, int ns, bool tau) {
-  const int nin = tau ? 3 : 2, ncs = tau ? 6 : 3, npv = tau ? 5 : 4;
-  const size_t na = (size_t)std::max(nin * np, npv * lang * mang);
-  return sizeof(double) * ((size_t)ns * na + (size_t)ns * ncs * nd * lang);
-}
-
-// The GGA / meta-GGA point kernel holds one radial point's density and
-// potential tables in LDS (63 KB for PBE, 101 KB for TPSS on a 36 x 36
-// angular rule with 49 shells), so one or two workgroups fit a CU: it runs
-// XP_NT threads over the same tables to keep more waves resident (Xe:
-// 1024 threads take the PBE point kernel from 4.1 to 2.6 ms and TPSS from
-// 7.8 to 4.3 ms against 256).
-#ifndef HFG_XC_POINT_NT
-#define HFG_XC_POINT_NT 1024
-#endif
-constexpr int XP_NT = HFG_XC_POINT_NT, XP_WAVES = XP_NT / 64;
-static_assert(XP_NT % 64 == 0 && XP_NT <= 1024, "point kernel workgroup");
+// Threads: one per angular point, at least 256, at most 512 (the functional's
+// derivatives dominate: idle threads would hold registers for nothing).
+constexpr int XP_MAX = 256;
 
 template <int MODE>
-__global__ void __launch_bounds__(XP_NT) k_xc_point_gga(XCArgs A) {
+__global__ void __launch_bounds__(XP_MAX) k_xc_point_gga(XCArgs A) {
   typedef GgaShape<MODE> G;
   const int e = blockIdx.x / A.nrad, i = blockIdx.x - e * A.nrad;
-  const int t = threadIdx.x;
-  const int np = A.npair, nd = A.nd, lang = A.lang, mang = A.mang, nang = lang * mang, dmax = (nd - 1) / 2;
+  const int t = threadIdx.x, nt = blockDim.x;
+  const int np = A.npair, nd = A.nd, lang = A.lang, nk = A.nk, nang = lang * nk;
   const bool pol = A.Db != nullptr;
   const int ns = pol ? 2 : 1;
   const bool gga = xcf::is_gga(A.xf) || xcf::is_gga(A.cf);
   const bool tau = MODE == 2;
   const int na = max(G::nin * np, G::npv * nang), ncl = nd * lang;
   extern __shared__ double sm[];
-  double *sA = sm;            // [ns][na]
-  double *sB = sm + ns * na;  // [ns][ncs][nd][lang]
-  __shared__ double red[3 * XP_WAVES];
+  double *sA = sm;                         // [ns][na]
+  double *sB = sm + ns * na;               // [ncs][ns][nd][lang]
+  double *sP = sB + ns * G::ncs * ncl;     // [ns][pieces][lang]
+  __shared__ double red[3 * XP_MAX / 64];
   const size_t row = ((size_t)e * A.nrad + i) * np;
-  for (int x = t; x < np; x += XP_NT) {
+  for (int x = t; x < np; x += nt) {
     sA[x] = A.D[row + x];
     sA[np + x] = A.E[row + x];
     if (tau) sA[2 * np + x] = A.F[row + x];
@@ -390,36 +479,32 @@ __global__ void __launch_bounds__(XP_NT) k_xc_point_gga(XCArgs A) {
   __syncthreads();
   // class sums: 0 C (Theta Theta D), 1 G (Theta Theta E), 2 T ((Theta Theta)' D),
   // with tau 3 (Theta Theta F), 4 (Theta' Theta' D), 5 (m m Theta Theta D)
-  for (int q = t; q < ns * G::ncs * ncl; q += XP_NT) {
-    const int sp = q / (G::ncs * ncl), r1 = q - sp * G::ncs * ncl, c = r1 / ncl, r2 = r1 - c * ncl;
-    const int d = r2 / lang, tt = r2 - d * lang;
-    const double *src = sA + sp * na + (c == 1 ? np : c == 3 ? 2 * np : 0);
+  for (int c = 0; c < G::ncs; ++c) {
     const double *tab = c == 2 ? A.thdt : c == 4 ? A.thddt : c == 5 ? A.thmmt : A.thxt;
-    double acc = 0.0;
-    for (int x = A.dstart[d]; x < A.dstart[d + 1]; ++x) acc += tab[(size_t)x * lang + tt] * src[x];
-    sB[q] = acc;
+    const int off = c == 1 ? np : c == 3 ? 2 * np : 0;
+    class_sums(A, ns, [&](int) { return tab; }, [&](int sp) { return sA + sp * na + off; }, sP, sB + c * ns * ncl);
   }
-  __syncthreads();
   const double *wp = A.wpt + ((size_t)e * A.nrad + i) * lang;
   const double *gs = A.gsc + ((size_t)e * A.nrad + i) * lang * 3;
   double ex = 0.0, ne = 0.0, ek = 0.0;
-  for (int q = t; q < nang; q += XP_NT) {
-    const int tt = q / mang, k = q - tt * mang;
+  for (int q = t; q < nang; q += nt) {
+    const int tt = q / nk, k = q - tt * nk;
     const double c1 = gs[3 * tt], c2 = gs[3 * tt + 1], c3 = gs[3 * tt + 2];
     double rho[2] = {0.0, 0.0}, g[2][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}}, tk[2] = {0.0, 0.0};
     for (int sp = 0; sp < ns; ++sp) {
-      const double *C = sB + sp * G::ncs * ncl;
+      const double *C = sB + sp * ncl;
+      const int cst = ns * ncl;
       double r0 = 0.0, gr = 0.0, gt = 0.0, gp = 0.0, kf = 0.0, kt = 0.0, km = 0.0;
       for (int d = 0; d < nd; ++d) {
-        const double cc = A.cs[(size_t)d * mang + k], cd = C[d * lang + tt];
+        const double cc = A.cs[(size_t)d * nk + k], cd = C[d * lang + tt];
         r0 += cd * cc;
-        gr += C[ncl + d * lang + tt] * cc;
-        gt += C[2 * ncl + d * lang + tt] * cc;
-        gp += (double)(d - dmax) * cd * A.sn[(size_t)d * mang + k];
+        gr += C[cst + d * lang + tt] * cc;
+        gt += C[2 * cst + d * lang + tt] * cc;
+        gp += (double)d * cd * A.sn[(size_t)d * nk + k];
         if (tau) {
-          kf += C[3 * ncl + d * lang + tt] * cc;
-          kt += C[4 * ncl + d * lang + tt] * cc;
-          km += C[5 * ncl + d * lang + tt] * cc;
+          kf += C[3 * cst + d * lang + tt] * cc;
+          kt += C[4 * cst + d * lang + tt] * cc;
+          km += C[5 * cst + d * lang + tt] * cc;
         }
       }
       rho[sp] = r0;
@@ -428,7 +513,7 @@ __global__ void __launch_bounds__(XP_NT) k_xc_point_gga(XCArgs A) {
       g[sp][2] = -c3 * gp;
       if (tau) tk[sp] = 0.5 * (c1 * c1 * kf + c2 * c2 * kt + c3 * c3 * km);
     }
-    const double w = wp[tt];
+    const double w = wp[tt] * A.pw[k];
     double f, va, vb = 0.0, vta = 0.0, vtb = 0.0, u[2][3];
     if (pol) {
       const double x7[7] = {rho[0], rho[1], g[0][0] * g[0][0] + g[0][1] * g[0][1] + g[0][2] * g[0][2],
@@ -473,37 +558,35 @@ __global__ void __launch_bounds__(XP_NT) k_xc_point_gga(XCArgs A) {
   ek = wave_sum(ek);
   if ((t & 63) == 0) {
     red[t >> 6] = ex;
-    red[XP_WAVES + (t >> 6)] = ne;
-    red[2 * XP_WAVES + (t >> 6)] = ek;
+    red[XP_MAX / 64 + (t >> 6)] = ne;
+    red[2 * XP_MAX / 64 + (t >> 6)] = ek;
   }
   __syncthreads();
   if (t == 0) {
     double sx = 0.0, sn = 0.0, sk = 0.0;
-    for (int w = 0; w < XP_WAVES; ++w) {
+    for (int w = 0; w < nt / 64; ++w) {
       sx += red[w];
-      sn += red[XP_WAVES + w];
-      sk += red[2 * XP_WAVES + w];
+      sn += red[XP_MAX / 64 + w];
+      sk += red[2 * XP_MAX / 64 + w];
     }
     A.part[3 * ((size_t)e * A.nrad + i)] = sx;
     A.part[3 * ((size_t)e * A.nrad + i) + 1] = sn;
     A.part[3 * ((size_t)e * A.nrad + i) + 2] = sk;
   }
-  __syncthreads();
   // class transforms: 0 Q = V_d - d Vphi_d, 1 Vr_d, 2 Vtheta_d, with tau 3 S_d
   const int ntr = tau ? 4 : 3;
-  for (int q = t; q < ns * ntr * ncl; q += XP_NT) {
+  for (int q = t; q < ns * ntr * ncl; q += nt) {
     const int sp = q / (ntr * ncl), r1 = q - sp * ntr * ncl, c = r1 / ncl, r2 = r1 - c * ncl;
     const int d = r2 / lang, tt = r2 - d * lang;
-    const double *V = sA + sp * na + tt * mang;
-    const double *cs = A.cs + (size_t)d * mang, *snd = A.sn + (size_t)d * mang;
+    const double *V = sA + sp * na + tt * nk;
+    const double *cs = A.cs + (size_t)d * nk, *snd = A.sn + (size_t)d * nk;
     double acc = 0.0;
     if (c == 0) {
-      const double fphi = (double)(d - dmax);
       const double *Vp = V + 3 * nang;
-      for (int k = 0; k < mang; ++k) acc += V[k] * cs[k] - fphi * Vp[k] * snd[k];
+      for (int k = 0; k < nk; ++k) acc += V[k] * cs[k] - (double)d * Vp[k] * snd[k];
     } else {
       const double *Vc = V + (c == 1 ? 1 : c == 2 ? 2 : 4) * nang;
-      for (int k = 0; k < mang; ++k) acc += Vc[k] * cs[k];
+      for (int k = 0; k < nk; ++k) acc += Vc[k] * cs[k];
     }
     sB[sp * G::ncs * ncl + c * ncl + d * lang + tt] = acc;
   }
@@ -511,10 +594,11 @@ __global__ void __launch_bounds__(XP_NT) k_xc_point_gga(XCArgs A) {
   for (int sp = 0; sp < ns; ++sp) {
     double *Wout = sp == 0 ? A.W : A.Wb, *Yout = sp == 0 ? A.Y : A.Yb, *Zout = sp == 0 ? A.Z : A.Zb;
     const double *Q = sB + sp * G::ncs * ncl, *Vr = Q + ncl, *Vt = Vr + ncl, *S = Vt + ncl;
-    for (int x = t; x < np; x += XP_NT) {
+    for (int x = t; x < np; x += nt) {
       const int d = A.xd[x];
       const double *Qd = Q + d * lang, *Vrd = Vr + d * lang, *Vtd = Vt + d * lang, *Sd = S + d * lang;
       double w2 = 0.0, y = 0.0, z = 0.0;
+#pragma unroll 4
       for (int tt = 0; tt < lang; ++tt) {
         const double th = A.thx[(size_t)tt * np + x];
         w2 += th * Qd[tt] + A.thd[(size_t)tt * np + x] * Vtd[tt];
@@ -525,86 +609,136 @@ __global__ void __launch_bounds__(XP_NT) k_xc_point_gga(XCArgs A) {
           z += c1 * c1 * th * Sd[tt];
         }
       }
-      Wout[((size_t)e * np + x) * A.nrad + i] = w2;
-      Yout[((size_t)e * np + x) * A.nrad + i] = y;
-      if (tau) Zout[((size_t)e * np + x) * A.nrad + i] = z;
+      Wout[row + x] = w2;
+      Yout[row + x] = y;
+      if (tau) Zout[row + x] = z;
     }
   }
 }
 
-// Workgroups per row of the output kernel (below): the pairs of one row are
-// spread over this many, so the launch holds more waves for the latency of
-// its dependent radial loads (Xe, split 1 / 2 / 4 / 8: LDA 0.437 / 0.405 /
-// 0.392 / 0.401 ms, PBE 1.18 / 1.12 / 1.10 / 1.14 ms).
-#ifndef HFG_XC_OUT_SPLIT
-#define HFG_XC_OUT_SPLIT 4
-#endif
-constexpr int XO_SPLIT = HFG_XC_OUT_SPLIT;
-
-// One workgroup per (element, shell a); thread (r,s) of the element band,
-// looping over the pairs (a, b) of row a.  The corner shared with element
-// e+1 is written by e with both contributions; e > 0 skips its own (0,0).
+// H_ab = H_ba = sum_i R' diag(W) R of every pair (with GGA M + M', M = sum_i
+// (R W / 2 + dR Y)' R; with tau also dR' diag(Z) dR) on the FP64 matrix cores:
+// one wave per pair, 16 pairs per workgroup.  The corner entry shared with
+// element e+1 is written by e with both contributions (the wave sums e+1's over
+// its points); e > 0 skips its own (0,0).  blockIdx.y: spin.
+// Bound by the band writes and the W reads: Xe LDA 393 (FP64 vector sums, a
+// workgroup per ordered pair) -> 100 us, N2 68 -> 34, O polarized PBE 2 x 124 -> 30.
 template <int MODE>
-__global__ void __launch_bounds__(NT) k_xc_rad_out(XCArgs A) {
-  // XO_SPLIT workgroups share row a, taking its pairs (a, b) in turn; each
-  // pair's H block is written by one of them
-  const int blk = blockIdx.x / XO_SPLIT, part = blockIdx.x - blk * XO_SPLIT;
-  const int e = blk / A.Nang, a = blk - e * A.Nang;
-  const int t = threadIdx.x, r = t & 15, s = t >> 4;
+__global__ void __launch_bounds__(NT) k_xc_rad_out(XCArgs A, XCArgs B) {
+  if (blockIdx.y) A = B;
+  const int groups = (A.npair + XR_PAIRS - 1) / XR_PAIRS;
+  const int e = blockIdx.x / groups, x0 = (blockIdx.x - e * groups) * XR_PAIRS;
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6, g = lane >> 4, c = lane & 15;
   const int ni = A.ni[e], f0 = A.first[e];
-  extern __shared__ double sm[];
-  double *sR = sm;  // [nrad][TILE] of e, then column 0 of e+1; with GGA the same of d/dr R
-  double *sN = sm + A.nrad * TILE;
-  double *sdR = sN + A.nrad, *sdN = sdR + A.nrad * TILE;
-  for (int q = t; q < A.nrad * TILE; q += NT) {
-    sR[q] = A.R[(size_t)e * A.nrad * TILE + q];
-    if (MODE) sdR[q] = A.dR[(size_t)e * A.nrad * TILE + q];
-  }
+  const int np = min(XR_PAIRS, A.npair - x0);
   const bool has_next = e + 1 < A.Nel;
-  if (has_next)
-    for (int q = t; q < A.nrad; q += NT) {
-      sN[q] = A.R[((size_t)(e + 1) * A.nrad + q) * TILE];
-      if (MODE) sdN[q] = A.dR[((size_t)(e + 1) * A.nrad + q) * TILE];
+  constexpr int PW = XR_PAIRS / (NT / 64);
+  extern __shared__ double sm[];
+  double *sR = sm;                                    // [XR_PTS][XR_RS]
+  double *sdR = sR + XR_PTS * XR_RS;                  // with GGA
+  double *sW = sR + (MODE ? 2 : 1) * XR_PTS * XR_RS;  // [MODE + 1][XR_PTS][XR_WS]
+  v4d acc[PW];
+  double crn[PW];  // e+1's share of the corner entry, per lane
+#pragma unroll
+  for (int p = 0; p < PW; ++p) {
+    acc[p] = v4d{0.0, 0.0, 0.0, 0.0};
+    crn[p] = 0.0;
+  }
+  for (int i0 = 0; i0 < A.nrad; i0 += XR_PTS) {
+    const int nq = min(XR_PTS, A.nrad - i0), nq4 = (nq + 3) & ~3;
+    __syncthreads();
+    for (int q = t; q < nq4 * TILE; q += NT) {  // zeros up to a whole k-step
+      const bool in = (q >> 4) < nq;
+      sR[(q >> 4) * XR_RS + (q & 15)] = in ? A.R[((size_t)e * A.nrad + i0) * TILE + q] : 0.0;
+      if (MODE) sdR[(q >> 4) * XR_RS + (q & 15)] = in ? A.dR[((size_t)e * A.nrad + i0) * TILE + q] : 0.0;
     }
-  __syncthreads();
-  if (r >= ni || s >= ni) return;
-  if (e > 0 && r == 0 && s == 0) return;
-  const long long row = grid_row(A.skip, A.poff, a, f0 + r);
-  if (row < 0) return;
-  const bool corner = has_next && r == ni - 1 && s == ni - 1;
-  const size_t np = A.npair;
-  for (int q = A.rstart[a] + part; q < A.rstart[a + 1]; q += XO_SPLIT) {
-    const int b = A.rb[q], x = A.rx[q];
-    const long long col = grid_row(A.skip, A.poff, b, f0 + s);
-    if (col < 0) continue;
-    const double *Wp = A.W + ((size_t)e * np + x) * A.nrad;
-    double v = 0.0;
-    if (MODE) {
-      const int xT = A.rxT[q];
-      const double *Yp = A.Y + ((size_t)e * np + x) * A.nrad, *YT = A.Y + ((size_t)e * np + xT) * A.nrad;
-      const double *Zp = MODE == 2 ? A.Z + ((size_t)e * np + x) * A.nrad : nullptr;
-      for (int i = 0; i < A.nrad; ++i) {
-        const double Rr = sR[i * TILE + r], Rs = sR[i * TILE + s], Dr = sdR[i * TILE + r], Ds = sdR[i * TILE + s];
-        v += Rr * Rs * Wp[i] + Dr * Rs * Yp[i] + Rr * Ds * YT[i];
-        if (MODE == 2) v += Dr * Ds * Zp[i];
-      }
-      if (corner) {
-        const double *Wn = A.W + ((size_t)(e + 1) * np + x) * A.nrad;
-        const double *Yn = A.Y + ((size_t)(e + 1) * np + x) * A.nrad, *YTn = A.Y + ((size_t)(e + 1) * np + xT) * A.nrad;
-        for (int i = 0; i < A.nrad; ++i) v += sN[i] * (sN[i] * Wn[i] + sdN[i] * (Yn[i] + YTn[i]));
-        if (MODE == 2) {
-          const double *Zn = A.Z + ((size_t)(e + 1) * np + x) * A.nrad;
-          for (int i = 0; i < A.nrad; ++i) v += sdN[i] * sdN[i] * Zn[i];
+    for (int q = t; q < nq4 * XR_PAIRS; q += NT) {
+      const int i = q >> 4, x = q & 15;
+      const bool in = i < nq && x < np;
+      const size_t o = ((size_t)e * A.nrad + i0 + i) * A.npair + x0 + x;
+      sW[i * XR_WS + x] = in ? A.W[o] : 0.0;
+      if (MODE) sW[(XR_PTS + i) * XR_WS + x] = in ? A.Y[o] : 0.0;
+      if (MODE == 2) sW[(2 * XR_PTS + i) * XR_WS + x] = in ? A.Z[o] : 0.0;
+    }
+    __syncthreads();
+    for (int ks = 0; ks < nq4; ks += 4) {
+      const double r = sR[(ks + g) * XR_RS + c], dr = MODE ? sdR[(ks + g) * XR_RS + c] : 0.0;
+#pragma unroll
+      for (int p = 0; p < PW; ++p) {
+        const int x = wv * PW + p;
+        const double w = sW[(ks + g) * XR_WS + x];
+        if (MODE == 0) {
+          acc[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(w * r, r, acc[p], 0, 0, 0);
+        } else {
+          const double y = sW[(XR_PTS + ks + g) * XR_WS + x];
+          acc[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(0.5 * w * r + y * dr, r, acc[p], 0, 0, 0);
+          if (MODE == 2) {
+            // symmetric: half of it survives the M + M' below
+            const double z = sW[(2 * XR_PTS + ks + g) * XR_WS + x];
+            acc[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(0.5 * z * dr, dr, acc[p], 0, 0, 0);
+          }
         }
       }
-    } else {
-      for (int i = 0; i < A.nrad; ++i) v += sR[i * TILE + r] * sR[i * TILE + s] * Wp[i];
-      if (corner) {
-        const double *Wn = A.W + ((size_t)(e + 1) * np + x) * A.nrad;
-        for (int i = 0; i < A.nrad; ++i) v += sN[i] * sN[i] * Wn[i];
+    }
+    if (has_next)
+#pragma unroll
+      for (int p = 0; p < PW; ++p) {
+        const int x = wv * PW + p;
+        if (x >= np) continue;
+        for (int i = lane; i < nq; i += 64) {
+          const size_t n = (size_t)(e + 1) * A.nrad + i0 + i, o = n * A.npair + x0 + x;
+          const double r = A.R[n * TILE];
+          double v = r * r * A.W[o];
+          if (MODE) {
+            const double dr = A.dR[n * TILE];
+            v += 2.0 * r * dr * A.Y[o];
+            if (MODE == 2) v += dr * dr * A.Z[o];
+          }
+          crn[p] += v;
+        }
+      }
+  }
+  double *sT = sW;  // transposes, one 16 x 17 tile per wave
+  if (MODE) __syncthreads();
+#pragma unroll
+  for (int p = 0; p < PW; ++p) {
+    const int x = wv * PW + p;
+    if (x >= np) continue;
+    v4d v = acc[p];  // lane (g,c): entry (g + 4 s, c)
+    if (MODE) {
+      double *T = sT + wv * TILE * XR_RS;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) T[(g + 4 * s) * XR_RS + c] = v[s];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int s = 0; s < 4; ++s) v[s] += T[c * XR_RS + g + 4 * s];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    double corner = 0.0;
+    if (has_next) {
+      corner = wave_sum(crn[p]);
+      corner = __shfl(corner, 0, 64);
+    }
+    const int2 ab = A.pab[x0 + x];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      // the tile is symmetric: entry (c, col), so that lanes of one column
+      // write consecutive rows
+      const int cl = g + 4 * s;
+      if (c >= ni || cl >= ni || (e > 0 && c == 0 && cl == 0)) continue;
+      double h = v[s];
+      if (has_next && c == ni - 1 && cl == ni - 1) h += corner;
+      const long long ra = grid_row(A.skip, A.poff, ab.x, f0 + c), cb = grid_row(A.skip, A.poff, ab.y, f0 + cl);
+      if (ra >= 0 && cb >= 0) A.H[ra + cb * A.ldh] = h;
+      if (ab.x != ab.y) {
+        const long long rb = grid_row(A.skip, A.poff, ab.y, f0 + c), ca = grid_row(A.skip, A.poff, ab.x, f0 + cl);
+        if (rb >= 0 && ca >= 0) A.H[rb + ca * A.ldh] = h;
       }
     }
-    A.H[row + col * A.ldh] = v;
   }
 }
 
@@ -613,39 +747,74 @@ __global__ void __launch_bounds__(NT) k_xc_rad_out(XCArgs A) {
 bool xc_generic(int xf, int cf) { return !((xf == 0 || xf == 1) && (cf == 0 || cf == 7)); }
 bool xc_tau(int xf, int cf) { return xcf::is_mgga(xf) || xcf::is_mgga(cf); }
 
-size_t xc_point_lds(const XCGridDevice &g, int xf, int cf, bool pol) {
+size_t xc_gga_limit_lds(const XCGridDevice &g, int ns, bool tau) {
+  const int nin = tau ? 3 : 2, ncs = tau ? 6 : 3, npv = tau ? 5 : 4;
+  const size_t na = (size_t)std::max(nin * g.npair_all, npv * g.lang * g.mang);
+  return sizeof(double) * ns * (na + (size_t)ncs * (2 * g.dmax + 1) * g.lang);
+}
+
+size_t xc_gga_point_lds(const XCGridDevice &g, int ns, bool tau) {
+  const int nin = tau ? 3 : 2, ncs = tau ? 6 : 3, npv = tau ? 5 : 4;
+  const size_t na = (size_t)std::max(nin * g.npair, npv * g.lang * g.nk);
+  const size_t pieces = g.npiece == 1 && g.dmax == 0 ? 0 : (size_t)g.npiece * g.lang;
+  return sizeof(double) * ns * (na + (size_t)ncs * (g.dmax + 1) * g.lang + pieces);
+}
+
+size_t xc_limit_lds(const XCGridDevice &g, int xf, int cf, bool pol) {
   const int ns = pol ? 2 : 1, nd = 2 * g.dmax + 1;
-  if (xc_generic(xf, cf)) return xc_gga_point_lds(g.npair, nd, g.lang, g.mang, ns, xc_tau(xf, cf));
-  return sizeof(double) * ns * ((size_t)g.npair + (size_t)g.lang * nd + (size_t)g.lang * g.mang);
+  if (xc_generic(xf, cf)) return xc_gga_limit_lds(g, ns, xc_tau(xf, cf));
+  return sizeof(double) * ns * ((size_t)g.npair_all + (size_t)g.lang * nd + (size_t)g.lang * g.mang);
 }
 
 namespace {
+template <typename F>
+void allow_lds(F f, size_t bytes, const char *what) {
+  if (bytes > 64 * 1024)
+    hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(f), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)bytes),
+              what);
+}
+
 template <int MODE>
-void launch_general(const XCGridDevice &g, const XCArgs &a, const XCArgs &b, bool pol, size_t sh_in, size_t sh_pt,
-                    size_t sh_out, hipStream_t s, KernelTimer *timer) {
+void launch_general(const XCGridDevice &g, const XCArgs &a, const XCArgs &b, bool pol, hipStream_t s,
+                    KernelTimer *timer) {
+  const int ns = pol ? 2 : 1, nd = g.dmax + 1;
+  const unsigned groups = (unsigned)((g.npair + XR_PAIRS - 1) / XR_PAIRS) * g.Nel;
+  const size_t radial = sizeof(double) * (MODE ? 2 : 1) * XR_PTS * XR_RS;
+  const size_t vals = sizeof(double) * (MODE + 1) * XR_PTS * XR_WS;
   {
     TimedLaunch tl(timer, "xc_rad_in", s);
-    hipLaunchKernelGGL(k_xc_rad_in<MODE>, dim3(g.Nel * g.Nang), dim3(NT), sh_in, s, a);
-    if (pol) hipLaunchKernelGGL(k_xc_rad_in<MODE>, dim3(g.Nel * g.Nang), dim3(NT), sh_in, s, b);
+    const size_t lds =
+        radial + sizeof(double) * ((MODE ? 2 : 1) * XI_J * TILE2 + (MODE + 1) * XR_PTS * XI_WS);
+    const int per = (size_t)g.npair * g.Nel * ns >= 512 * XI_PAIRS ? XI_PAIRS : XI_J;
+    allow_lds(&k_xc_rad_in<MODE>, lds, "xc_rad_in LDS size");
+    hipLaunchKernelGGL(k_xc_rad_in<MODE>, dim3((unsigned)((g.npair + per - 1) / per) * g.Nel, ns), dim3(NT), lds, s, a,
+                       b, per);
     hip_check(hipGetLastError(), "xc_rad_in");
   }
   {
     TimedLaunch tl(timer, "xc_point", s);
-    if (MODE == 0) {
-      hipLaunchKernelGGL(k_xc_point, dim3(g.Nel * g.nrad), dim3(LP_NT), sh_pt, s, a);
+    const unsigned points = (unsigned)(g.Nel * g.nrad);
+    if constexpr (MODE == 0) {
+      const size_t lds = sizeof(double) * ns *
+                         ((size_t)g.npair + (size_t)g.lang * nd + (size_t)g.lang * std::max(g.nk, g.npiece));
+      // few points per CU: more threads on each
+      const int threads = points >= 1024 ? 256 : 512;
+      allow_lds(&k_xc_point, lds, "xc_point LDS size");
+      hipLaunchKernelGGL(k_xc_point, dim3(points), dim3(threads), lds, s, a);
     } else {
-      if (sh_pt > 64 * 1024)
-        hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_xc_point_gga<MODE>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh_pt),
-                  "xc_point_gga LDS size");
-      hipLaunchKernelGGL(k_xc_point_gga<MODE>, dim3(g.Nel * g.nrad), dim3(XP_NT), sh_pt, s, a);
+      const size_t lds = xc_gga_point_lds(g, ns, MODE == 2);
+      const int threads = std::min(XP_MAX, std::max(256, (g.lang * g.nk + 63) / 64 * 64));
+      allow_lds(&k_xc_point_gga<MODE>, lds, "xc_point_gga LDS size");
+      hipLaunchKernelGGL(k_xc_point_gga<MODE>, dim3(points), dim3(threads), lds, s, a);
     }
     hip_check(hipGetLastError(), "xc_point");
   }
   {
     TimedLaunch tl(timer, "xc_rad_out", s);
-    hipLaunchKernelGGL(k_xc_rad_out<MODE>, dim3(g.Nel * g.Nang * XO_SPLIT), dim3(NT), sh_out, s, a);
-    if (pol) hipLaunchKernelGGL(k_xc_rad_out<MODE>, dim3(g.Nel * g.Nang * XO_SPLIT), dim3(NT), sh_out, s, b);
+    const size_t lds = radial + std::max(vals, sizeof(double) * (NT / 64) * TILE * XR_RS);
+    allow_lds(&k_xc_rad_out<MODE>, lds, "xc_rad_out LDS size");
+    hipLaunchKernelGGL(k_xc_rad_out<MODE>, dim3(groups, ns), dim3(NT), lds, s, a, b);
     hip_check(hipGetLastError(), "xc_rad_out");
   }
 }
@@ -658,11 +827,10 @@ void xc_grid_launch(XCGridDevice &g, int xf, int cf, double thr, const double *P
   const int mode = xc_tau(xf, cf) ? 2 : xc_generic(xf, cf) ? 1 : 0;
   fill_zero_launch(Ha, g.Nbf, g.Nbf, ldha, s);
   if (pol) fill_zero_launch(Hb, g.Nbf, g.Nbf, ldhb, s);
-  const int nd = 2 * g.dmax + 1;
-  XCArgs a{Pa, ldpa, Ha, ldha, g.Nel, g.Nang, g.nrad, g.lang, g.mang, nd, xf, cf, g.npair, thr,
-           g.first.p, g.ni.p, g.skip.p, g.poff.p, g.rstart.p, g.rb.p, g.rx.p, g.dstart.p, g.xd.p,
-           g.R.p, g.wpt.p, g.thx.p, g.thxt.p, g.cs.p, g.D.p, g.W.p, g.part.p, pol ? g.Db.p : nullptr,
-           pol ? g.Wb.p : nullptr, g.dR.p, g.gsc.p, g.sn.p, g.thd.p, g.thdt.p, g.rxT.p,
+  XCArgs a{Pa, ldpa, Ha, ldha, g.Nel, g.Nang, g.nrad, g.lang, g.nk, g.dmax + 1, g.npiece, xf, cf, g.npair, thr,
+           g.first.p, g.ni.p, g.skip.p, g.poff.p, g.pab.p, g.xd.p, g.pstart.p, g.piece.p,
+           g.R.p, g.wpt.p, g.thx.p, g.thxt.p, g.cs.p, g.pw.p, g.D.p, g.W.p, g.part.p, pol ? g.Db.p : nullptr,
+           pol ? g.Wb.p : nullptr, g.dR.p, g.gsc.p, g.sn.p, g.thd.p, g.thdt.p,
            g.E.p, g.Y.p, pol ? g.Eb.p : nullptr, pol ? g.Yb.p : nullptr,
            g.thdd.p, g.thddt.p, g.thmm.p, g.thmmt.p, g.F.p, g.Z.p, pol ? g.Fb.p : nullptr, pol ? g.Zb.p : nullptr};
   XCArgs b = a;  // second spin: its density in, its matrix out
@@ -678,17 +846,12 @@ void xc_grid_launch(XCGridDevice &g, int xf, int cf, double thr, const double *P
     b.F = g.Fb.p;
     b.Z = g.Zb.p;
   }
-  const int rf = mode ? 2 : 1;
-  const size_t sh_in =
-      sizeof(double) * ((size_t)rf * g.nrad * XC_RS + (size_t)xc_pairs_per_group(g.nrad) * TILE2);
-  const size_t sh_pt = xc_point_lds(g, xf, cf, pol);
-  const size_t sh_out = sizeof(double) * rf * ((size_t)g.nrad * TILE + g.nrad);
   if (mode == 2)
-    launch_general<2>(g, a, b, pol, sh_in, sh_pt, sh_out, s, timer);
+    launch_general<2>(g, a, b, pol, s, timer);
   else if (mode == 1)
-    launch_general<1>(g, a, b, pol, sh_in, sh_pt, sh_out, s, timer);
+    launch_general<1>(g, a, b, pol, s, timer);
   else
-    launch_general<0>(g, a, b, pol, sh_in, sh_pt, sh_out, s, timer);
+    launch_general<0>(g, a, b, pol, s, timer);
 }
 
 }  // namespace hfg
