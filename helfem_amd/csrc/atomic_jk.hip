@@ -76,26 +76,27 @@ struct JArgs {
   const int *lm_L, *lm_pstart, *pair_kl;
   const double *pair_c;
   double *Jin, *jsm, *jbg;
+  int n_lm;
 };
 
-// One workgroup per ((L,M), element): blk = lm * Nel + e.
+// One workgroup per ((L,M), element), items e n_lm + lm in shares per XCD: the L of
+// one M read the same tiles of P.  The waves deal the pairs: a chain of dependent
+// loads a quarter as long (Xe 167 -> 125 us).
 __device__ inline void j_gather_body(const JArgs &A, int blk) {
-  const int lm = blk / A.Nel, e = blk - lm * A.Nel;
+  const int item = xcd_item(blk, A.n_lm * A.Nel);
+  if (item < 0) return;
+  const int e = item / A.n_lm, lm = item - e * A.n_lm;
   const int t = threadIdx.x, a = t & 15, b = t >> 4;
   const int ni = A.ni[e], f0 = A.first[e], L = A.lm_L[lm];
+  __shared__ double part[4 * TILE2];
   __shared__ double sP[TILE2];
   __shared__ double sS[TILE2];
   __shared__ double red[8];
-  double v = 0.0;
-  if (a < ni && b < ni) {
-    const int p0 = A.lm_pstart[lm], p1 = A.lm_pstart[lm + 1];
-    for (int p = p0; p < p1; ++p) {
-      const int kl = A.pair_kl[p];
-      const int k = kl / A.Nang, l = kl - k * A.Nang;
-      v += A.pair_c[p] * A.P[(int64_t)(k * A.Nrad + f0 + a) + (int64_t)(l * A.Nrad + f0 + b) * A.ldp];
-    }
-  }
-  sP[t] = v;
+  auto at = [&](int kl, int r, int c) {
+    const int k = kl / A.Nang, l = kl - k * A.Nang;
+    return r < ni && c < ni ? A.P[(int64_t)(k * A.Nrad + f0 + r) + (int64_t)(l * A.Nrad + f0 + c) * A.ldp] : 0.0;
+  };
+  j_pair_sums<1>(A.pair_kl, A.pair_c, A.lm_pstart[lm], A.lm_pstart[lm + 1], at, part, &sP[t]);
   __syncthreads();
   // tr(r_small P) and tr(r_big P): sum_ab r(a,b) P(b,a)
   const size_t tile = ((size_t)L * A.Nel + e) * TILE2;
@@ -120,73 +121,76 @@ __device__ inline void j_gather_body(const JArgs &A, int blk) {
   }
   __syncthreads();
   double jin = 0.0;
+#pragma unroll 4
   for (int p = 0; p < rank; ++p) jin += M[(size_t)p * TILE2 + t] * sS[p];
   A.Jin[((size_t)lm * A.Nel + e) * TILE2 + t] = jin;
 }
 
 __global__ void __launch_bounds__(NT) k_atomic_j_gather(JArgs A) { j_gather_body(A, blockIdx.x); }
 
-// Cross-element weights: pre_a(lm,e) = sum_{j>e} jbig(j), pre_b = sum_{j<e} jsmall(j)
-__device__ inline void j_prefix_body(int lm, int n_lm, int Nel, const double *jsm, const double *jbg,
-                                     double *preA, double *preB) {
-  if (lm >= n_lm) return;
-  const double *s = jsm + (size_t)lm * Nel;
-  const double *g = jbg + (size_t)lm * Nel;
-  double acc = 0.0;
-  for (int e = 0; e < Nel; ++e) {
-    preB[(size_t)lm * Nel + e] = acc;
-    acc += s[e];
-  }
-  acc = 0.0;
-  for (int e = Nel - 1; e >= 0; --e) {
-    preA[(size_t)lm * Nel + e] = acc;
-    acc += g[e];
-  }
+struct JBandArgs {
+  int n_lm, Nel;
+  const int *lm_L;
+  const double *rs, *rb, *jsm, *jbg;
+  double *Jin;
+};
+
+// The whole potential of (L,M) in element e, in place: Jin + (sum_{j>e} jbig(j))
+// r_small + (sum_{j<e} jsmall(j)) r_big; blk = lm * Nel + e.  Formed once here, an
+// output block reads one tile per L instead of three.
+__device__ inline void j_band_body(const JBandArgs &A, int blk) {
+  if (blk >= A.n_lm * A.Nel) return;  // the batch rounds its grids up
+  const int lm = blk / A.Nel, e = blk - lm * A.Nel, t = threadIdx.x;
+  const double *s = A.jsm + (size_t)lm * A.Nel, *g = A.jbg + (size_t)lm * A.Nel;
+  double pa = 0.0, pb = 0.0;
+  for (int j = A.Nel - 1; j > e; --j) pa += g[j];
+  for (int j = 0; j < e; ++j) pb += s[j];
+  const size_t tile = ((size_t)A.lm_L[lm] * A.Nel + e) * TILE2;
+  double v = A.Jin[(size_t)blk * TILE2 + t] + pa * A.rs[tile + t];
+  if (e > 0) v += pb * A.rb[tile + t];
+  A.Jin[(size_t)blk * TILE2 + t] = v;
 }
 
-__global__ void k_atomic_j_prefix(int n_lm, int Nel, const double *jsm, const double *jbg, double *preA,
-                                  double *preB) {
-  j_prefix_body(blockIdx.x * blockDim.x + threadIdx.x, n_lm, Nel, jsm, jbg, preA, preB);
-}
+__global__ void __launch_bounds__(NT) k_atomic_j_band(JBandArgs A) { j_band_body(A, blockIdx.x); }
 
 struct JOutArgs {
   double *J;
   int64_t ldj;
   int Nel, Nrad, Nang;
-  const int *first, *ni, *lm_L;
-  const double *rs, *rb, *Jin, *preA, *preB;
+  const int *first, *ni;
+  const double *Jin;
   const int *out_start, *out_lm;
   const double *out_c;
 };
 
-__device__ inline double jband(const JOutArgs &A, int lm, int e, int t) {
-  const int L = A.lm_L[lm];
-  const size_t tile = ((size_t)L * A.Nel + e) * TILE2;
-  const size_t q = (size_t)lm * A.Nel + e;
-  double v = A.Jin[q * TILE2 + t] + A.preA[q] * A.rs[tile + t];
-  if (e > 0) v += A.preB[q] * A.rb[tile + t];
-  return v;
-}
-
-// One workgroup per (angular output block (i,j), element): blk = ij * Nel + e.
+// One workgroup per (angular output block (i,j), element): the element's columns of the block from top to bottom, zeros included, so that
+// J is written in one pass of whole columns instead of a fill and strided tiles
+// on top of it.  A column shared with element e-1 is e-1's.  The blocks i of one
+// column run on one XCD, whose L2 joins their partial lines.  Bound by the writes:
+// fill + prefix + expand of Xe (2.3 GB) 390 + 13 + 145 -> 424 us (and 12 for the band tiles).
 __device__ inline void j_expand_body(const JOutArgs &A, int blk) {
-  const int ij = blk / A.Nel, e = blk - ij * A.Nel;
+  const int item = xcd_item(blk, A.Nang * A.Nang * A.Nel);
+  if (item < 0) return;
+  const int je = item / A.Nang, i = item - je * A.Nang, j = je / A.Nel, e = je - j * A.Nel, ij = i * A.Nang + j;
   const int q0 = A.out_start[ij], q1 = A.out_start[ij + 1];
-  if (q0 == q1) return;
   const int t = threadIdx.x, a = t & 15, b = t >> 4;
-  const int ni = A.ni[e], f0 = A.first[e];
-  if (a >= ni || b >= ni) return;
-  if (e > 0 && a == 0 && b == 0) return;  // shared corner, written by e-1
-  const bool corner = (a == ni - 1 && b == ni - 1 && e + 1 < A.Nel);
-  double v = 0.0;
-  for (int q = q0; q < q1; ++q) {
-    const int lm = A.out_lm[q];
-    double x = jband(A, lm, e, t);
-    if (corner) x += jband(A, lm, e + 1, 0);
-    v += A.out_c[q] * x;
+  const int ni = A.ni[e], f0 = A.first[e], nn = e + 1 < A.Nel ? A.ni[e + 1] : 0;
+  __shared__ double sT[TILE2], sN[TILE];
+  {
+    double v = 0.0, w = 0.0;
+#pragma unroll 4
+    for (int q = q0; q < q1; ++q) v += A.out_c[q] * A.Jin[((size_t)A.out_lm[q] * A.Nel + e) * TILE2 + t];
+    if (nn && t < TILE)
+#pragma unroll 4
+      for (int q = q0; q < q1; ++q) w += A.out_c[q] * A.Jin[((size_t)A.out_lm[q] * A.Nel + e + 1) * TILE2 + t];
+    if (t < TILE) sN[t] = w;
+    sT[t] = v;
+    __syncthreads();
+    if (nn && a == ni - 1 && b == ni - 1) sT[t] = v + sN[0];
+    __syncthreads();
   }
-  const int i = ij / A.Nang, j = ij - i * A.Nang;
-  A.J[(int64_t)(i * A.Nrad + f0 + a) + (int64_t)(j * A.Nrad + f0 + b) * A.ldj] = v;
+  double *J = A.J + (int64_t)i * A.Nrad + (int64_t)j * A.Nrad * A.ldj;
+  j_store_columns(J, A.ldj, A.Nrad, 0, 0, f0, ni, nn, e > 0, sT, sN);
 }
 
 __global__ void __launch_bounds__(NT) k_atomic_j_expand(JOutArgs A) { j_expand_body(A, blockIdx.x); }
@@ -1078,31 +1082,30 @@ size_t atomic_coulomb_work_doubles(const AtomicDevice &d) {
 void atomic_coulomb_launch(const AtomicDevice &d, const double *P, int64_t ldp, double *J, int64_t ldj,
                            hipStream_t s, KernelTimer *timer, double *work) {
   const int64_t nbf = (int64_t)d.Nrad * d.Nang;
-  fill_zero_launch(J, nbf, nbf, ldj, s);
-  if (d.n_lm == 0) return;
+  if (d.n_lm == 0) {
+    fill_zero_launch(J, nbf, nbf, ldj, s);
+    return;
+  }
   // work space: the handle's buffers, or one caller-given block laid out as
-  // Jin [n_lm][Nel][TILE2], then jsm, jbg, preA, preB [n_lm][Nel] each
+  // Jin [n_lm][Nel][TILE2], then jsm, jbg [n_lm][Nel] each
   const size_t nq = (size_t)d.n_lm * d.Nel;
   double *Jin = work ? work : d.Jin.p;
   double *jsm = work ? work + nq * TILE2 : d.jsm.p;
   double *jbg = work ? jsm + nq : d.jbg.p;
-  double *preA = work ? jbg + nq : d.preA.p;
-  double *preB = work ? preA + nq : d.preB.p;
   JArgs a{P, ldp, d.Nel, d.Nrad, d.Nang, d.first.p, d.ni.p, d.rs.p, d.rb.p, d.chol.p, d.chol_off.p,
-          d.chol_rank.p, d.lm_L.p, d.lm_pstart.p, d.pair_kl.p, d.pair_c.p, Jin, jsm, jbg};
+          d.chol_rank.p, d.lm_L.p, d.lm_pstart.p, d.pair_kl.p, d.pair_c.p, Jin, jsm, jbg, d.n_lm};
   {
     TimedLaunch tl(timer, "atomic_j_gather", s);
-    hipLaunchKernelGGL(k_atomic_j_gather, dim3(d.n_lm * d.Nel), dim3(NT), 0, s, a);
+    hipLaunchKernelGGL(k_atomic_j_gather, dim3(8 * xcd_share(d.n_lm * d.Nel)), dim3(NT), 0, s, a);
     hip_check(hipGetLastError(), "atomic_j_gather");
   }
-  hipLaunchKernelGGL(k_atomic_j_prefix, dim3((d.n_lm + 63) / 64), dim3(64), 0, s, d.n_lm, d.Nel, jsm, jbg,
-                     preA, preB);
-  hip_check(hipGetLastError(), "atomic_j_prefix");
-  JOutArgs o{J, ldj, d.Nel, d.Nrad, d.Nang, d.first.p, d.ni.p, d.lm_L.p, d.rs.p, d.rb.p, Jin,
-             preA, preB, d.out_start.p, d.out_lm.p, d.out_c.p};
+  JBandArgs w{d.n_lm, d.Nel, d.lm_L.p, d.rs.p, d.rb.p, jsm, jbg, Jin};
+  hipLaunchKernelGGL(k_atomic_j_band, dim3(d.n_lm * d.Nel), dim3(NT), 0, s, w);
+  hip_check(hipGetLastError(), "atomic_j_band");
+  JOutArgs o{J, ldj, d.Nel, d.Nrad, d.Nang, d.first.p, d.ni.p, Jin, d.out_start.p, d.out_lm.p, d.out_c.p};
   {
     TimedLaunch tl(timer, "atomic_j_expand", s);
-    hipLaunchKernelGGL(k_atomic_j_expand, dim3(d.Nang * d.Nang * d.Nel), dim3(NT), 0, s, o);
+    hipLaunchKernelGGL(k_atomic_j_expand, dim3(8 * xcd_share(d.Nang * d.Nang * d.Nel)), dim3(NT), 0, s, o);
     hip_check(hipGetLastError(), "atomic_j_expand");
   }
 }
@@ -1636,12 +1639,6 @@ struct FillArgs {
   int nblk;
 };
 
-struct PrefixArgs {
-  int n_lm, Nel;
-  const double *jsm, *jbg;
-  double *preA, *preB;
-};
-
 template <typename T>
 struct PtileArgs {
   const double *P;
@@ -1662,10 +1659,9 @@ __global__ void __launch_bounds__(NT) k_atomic_j_gather_batch(const JArgs *args,
   j_gather_body(args[s], blockIdx.x - start[s]);
 }
 
-__global__ void __launch_bounds__(64) k_atomic_j_prefix_batch(const PrefixArgs *args, const int *start, int n) {
+__global__ void __launch_bounds__(NT) k_atomic_j_band_batch(const JBandArgs *args, const int *start, int n) {
   const int s = batch_find(start, n, blockIdx.x);
-  const PrefixArgs &a = args[s];
-  j_prefix_body((blockIdx.x - start[s]) * 64 + threadIdx.x, a.n_lm, a.Nel, a.jsm, a.jbg, a.preA, a.preB);
+  j_band_body(args[s], blockIdx.x - start[s]);
 }
 
 __global__ void __launch_bounds__(NT) k_atomic_j_expand_batch(const JOutArgs *args, const int *start, int n) {
@@ -1831,44 +1827,44 @@ void atomic_batch_coulomb(AtomicBatch &b, const double *const *P, const int64_t 
   const int n = (int)b.sys.size();
   std::vector<FillArgs> fills(n);
   std::vector<JArgs> gat(n);
-  std::vector<PrefixArgs> pre(n);
+  std::vector<JBandArgs> band(n);
   std::vector<JOutArgs> outs(n);
-  std::vector<int> sF(n + 1, 0), sG(n + 1, 0), sP(n + 1, 0), sE(n + 1, 0);
+  std::vector<int> sF(n + 1, 0), sG(n + 1, 0), sE(n + 1, 0);
   for (int i = 0; i < n; ++i) {
     AtomicDevice &d = *b.sys[i];
     const int64_t nbf = (int64_t)d.Nrad * d.Nang;
-    fills[i] = FillArgs{J[i], nbf, nbf, ldj[i], fill_blocks(nbf, nbf)};
+    const bool any = d.n_lm > 0;
+    fills[i] = FillArgs{J[i], nbf, nbf, ldj[i], any ? 0 : fill_blocks(nbf, nbf)};
     sF[i + 1] = sF[i] + fills[i].nblk;
     gat[i] = JArgs{P[i], ldp[i], d.Nel, d.Nrad, d.Nang, d.first.p, d.ni.p, d.rs.p, d.rb.p, d.chol.p,
                    d.chol_off.p, d.chol_rank.p, d.lm_L.p, d.lm_pstart.p, d.pair_kl.p, d.pair_c.p,
-                   d.Jin.p, d.jsm.p, d.jbg.p};
-    pre[i] = PrefixArgs{d.n_lm, d.Nel, d.jsm.p, d.jbg.p, d.preA.p, d.preB.p};
-    outs[i] = JOutArgs{J[i], ldj[i], d.Nel, d.Nrad, d.Nang, d.first.p, d.ni.p, d.lm_L.p, d.rs.p, d.rb.p,
-                       d.Jin.p, d.preA.p, d.preB.p, d.out_start.p, d.out_lm.p, d.out_c.p};
-    const bool any = d.n_lm > 0;
-    sG[i + 1] = sG[i] + (any ? d.n_lm * d.Nel : 0);
-    sP[i + 1] = sP[i] + (any ? (d.n_lm + 63) / 64 : 0);
-    sE[i + 1] = sE[i] + (any ? d.Nang * d.Nang * d.Nel : 0);
+                   d.Jin.p, d.jsm.p, d.jbg.p, d.n_lm};
+    band[i] = JBandArgs{d.n_lm, d.Nel, d.lm_L.p, d.rs.p, d.rb.p, d.jsm.p, d.jbg.p, d.Jin.p};
+    outs[i] = JOutArgs{J[i], ldj[i], d.Nel, d.Nrad, d.Nang, d.first.p, d.ni.p, d.Jin.p, d.out_start.p, d.out_lm.p,
+                       d.out_c.p};
+    sG[i + 1] = sG[i] + (any ? 8 * xcd_share(d.n_lm * d.Nel) : 0);
+    sE[i + 1] = sE[i] + (any ? 8 * xcd_share(d.Nang * d.Nang * d.Nel) : 0);
   }
   TabImage img;
-  const size_t oF = img.add(fills), oG = img.add(gat), oP = img.add(pre), oE = img.add(outs);
-  const size_t osF = img.add(sF), osG = img.add(sG), osP = img.add(sP), osE = img.add(sE);
+  const size_t oF = img.add(fills), oG = img.add(gat), oB = img.add(band), oE = img.add(outs);
+  const size_t osF = img.add(sF), osG = img.add(sG), osE = img.add(sE);
   char *base = upload_table(img, b.dtab_j, b.htab_j, b.ev_j, s);
-  const std::vector<long long> sig{sF[n], sG[n], sP[n], sE[n]};
+  const std::vector<long long> sig{sF[n], sG[n], sE[n]};
   auto launches = [&](KernelTimer *t) {
     const int *dsF = (const int *)(base + osF), *dsG = (const int *)(base + osG);
-    const int *dsP = (const int *)(base + osP), *dsE = (const int *)(base + osE);
-    hipLaunchKernelGGL(k_fill_zero_batch, dim3(sF[n]), dim3(NT), 0, s, (const FillArgs *)(base + oF), dsF, n);
-    hip_check(hipGetLastError(), "fill_zero_batch");
+    const int *dsE = (const int *)(base + osE);
+    if (sF[n] > 0) {
+      hipLaunchKernelGGL(k_fill_zero_batch, dim3(sF[n]), dim3(NT), 0, s, (const FillArgs *)(base + oF), dsF, n);
+      hip_check(hipGetLastError(), "fill_zero_batch");
+    }
     if (sG[n] == 0) return;
     {
       TimedLaunch tl(t, "batch_j_gather", s);
       hipLaunchKernelGGL(k_atomic_j_gather_batch, dim3(sG[n]), dim3(NT), 0, s, (const JArgs *)(base + oG), dsG, n);
       hip_check(hipGetLastError(), "atomic_j_gather_batch");
     }
-    hipLaunchKernelGGL(k_atomic_j_prefix_batch, dim3(sP[n]), dim3(64), 0, s, (const PrefixArgs *)(base + oP), dsP,
-                       n);
-    hip_check(hipGetLastError(), "atomic_j_prefix_batch");
+    hipLaunchKernelGGL(k_atomic_j_band_batch, dim3(sG[n]), dim3(NT), 0, s, (const JBandArgs *)(base + oB), dsG, n);
+    hip_check(hipGetLastError(), "atomic_j_band_batch");
     {
       TimedLaunch tl(t, "batch_j_expand", s);
       hipLaunchKernelGGL(k_atomic_j_expand_batch, dim3(sE[n]), dim3(NT), 0, s, (const JOutArgs *)(base + oE), dsE,

@@ -265,8 +265,6 @@ void atomic_upload(hf_atomic *h) {
   d.Jin.alloc((size_t)std::max(nlm, 1) * Nel * TILE2);
   d.jsm.alloc((size_t)std::max(nlm, 1) * Nel);
   d.jbg.alloc((size_t)std::max(nlm, 1) * Nel);
-  d.preA.alloc((size_t)std::max(nlm, 1) * Nel);
-  d.preB.alloc((size_t)std::max(nlm, 1) * Nel);
 
   hip_check(hipStreamSynchronize(s), "upload sync");
   atomic_build_operator(S, d, s);

@@ -301,8 +301,6 @@ void diatomic_upload(hf_diatomic *h) {
   d.Jin.alloc((size_t)std::max(nLM, 1) * Nel * 2 * TILE2);
   d.ds.alloc((size_t)std::max(nLM, 1) * Nel);
   d.db.alloc((size_t)std::max(nLM, 1) * Nel);
-  d.preA.alloc((size_t)std::max(nLM, 1) * Nel);
-  d.preB.alloc((size_t)std::max(nLM, 1) * Nel);
   hip_check(hipStreamSynchronize(s), "upload sync");
   diatomic_build_operator(S, d, s);
   d.op_ready = false;

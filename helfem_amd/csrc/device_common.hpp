@@ -103,5 +103,88 @@ __device__ inline int batch_find(const int *start, int n, int b) {
   return __builtin_amdgcn_readfirstlane(lo);
 }
 
+// Whole columns b0 .. ni-1 of one element of a Coulomb shell block, zeros
+// included: tile T(a,b) = T[a + 16 b] in rows f0 + a, and in the last column the
+// next element's first column N[0 .. nn) (nn = 0 without one; N[0] is in T).
+// Block rows start at J, its first column at J; the shells leave out their first
+// roff and coff functions.  A wave per column, lanes along rows in 16-byte pairs
+// from the first aligned address on.
+__device__ inline void j_store_columns(double *J, int64_t ldj, int nrow, int roff, int coff, int f0, int ni, int nn,
+                                       int b0, const double *T, const double *N) {
+  const int lane = threadIdx.x & 63;
+  for (int b = b0 + (int)(threadIdx.x >> 6); b < ni; b += (int)(blockDim.x >> 6)) {
+    const int c = f0 + b - coff;
+    if (c < 0) continue;
+    double *col = J + (int64_t)c * ldj;
+    const int nx = b == ni - 1 ? nn : 0;
+    auto at = [&](int r) {
+      const int a = r + roff - f0;
+      if (a >= 0 && a < ni) return T[a + TILE * b];
+      return a >= ni && a - (ni - 1) < nx ? N[a - (ni - 1)] : 0.0;
+    };
+    const int odd = (int)((reinterpret_cast<uintptr_t>(col) >> 3) & 1);
+    for (int r = 2 * lane - odd; r < nrow; r += 128) {
+      if (r >= 0 && r + 1 < nrow)
+        *reinterpret_cast<double2 *>(col + r) = make_double2(at(r), at(r + 1));
+      else if (r >= 0)
+        col[r] = at(r);
+      else
+        col[0] = at(0);  // r = -1: nrow >= 1
+    }
+  }
+}
+
+// Workgroup w of a grid of 8 * xcd_share(n) places -> work item: each XCD (w & 7)
+// takes a contiguous share, so that neighbours meet in one L2; items from n on are
+// empty.
+__host__ __device__ inline int xcd_share(int n) { return (n + 7) / 8; }
+__device__ inline int xcd_item(int w, int n) {
+  const int i = (w & 7) * xcd_share(n) + (w >> 3);
+  return i < n ? i : -1;
+}
+
+// v[k] = sum_p pair_c[nc p + k] P-tile(pair p) over the pair list [p0, p1): the
+// waves deal the pairs in runs of JG_RUN, a lane holds entries lane + 64 u, and the
+// waves' sums meet in part [4][NC][TILE2].  at(kl, a, b) is the entry of P.
+constexpr int JG_RUN = 4;
+template <int NC, typename At>
+__device__ inline void j_pair_sums(const int *pair_kl, const double *pair_c, int p0, int p1, At at, double *part,
+                                   double *out) {
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6, a = lane & 15, b = lane >> 4;
+  double v[NC][4];
+#pragma unroll
+  for (int k = 0; k < NC; ++k)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[k][u] = 0.0;
+  const int w0 = __builtin_amdgcn_readfirstlane(w);
+  for (int p = p0 + w0 * JG_RUN; p < p1; p += 4 * JG_RUN) {
+    double x[JG_RUN][4];
+#pragma unroll
+    for (int i = 0; i < JG_RUN; ++i) {
+      const int kl = pair_kl[min(p + i, p1 - 1)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[i][u] = at(kl, a, b + 4 * u);
+    }
+#pragma unroll
+    for (int i = 0; i < JG_RUN; ++i)
+      if (p + i < p1)
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+          const double c = pair_c[NC * (p + i) + k];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[k][u] += c * x[i][u];
+        }
+  }
+#pragma unroll
+  for (int k = 0; k < NC; ++k)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) part[(w * NC + k) * TILE2 + lane + 64 * u] = v[k][u];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NC; ++k)
+    out[k] = part[k * TILE2 + t] + part[(NC + k) * TILE2 + t] + part[(2 * NC + k) * TILE2 + t] +
+             part[(3 * NC + k) * TILE2 + t];
+}
+
 }  // namespace dev
 }  // namespace hfg

@@ -63,30 +63,32 @@ struct DJArgs {
   const int *pstart, *pair_kl;
   const double *pair_c;
   double *Jin, *ds, *db;
+  int n_LM;
 };
 
-// One workgroup per ((L,M), element).
+// One workgroup per ((L,M), element), items e n_LM + q in shares per XCD: the L of
+// one M read the same tiles of P.  The waves deal the pairs: a chain of dependent
+// loads a quarter as long (N2, 16 shells per |m| <= 2: 410 -> 269 us).
 __global__ void __launch_bounds__(NT) k_dia_j_gather(DJArgs A) {
-  const int q = blockIdx.x / A.Nel, e = blockIdx.x - q * A.Nel;
+  const int item = xcd_item(blockIdx.x, A.n_LM * A.Nel);
+  if (item < 0) return;
+  const int e = item / A.n_LM, q = item - e * A.n_LM;
   const int t = threadIdx.x, a = t & 15, b = t >> 4;
   const int ni = A.ni[e], f0 = A.first[e], ilm = A.LM_ilm[q];
   const double fac = A.LM_fac[q];
+  __shared__ double part[8 * TILE2];
   __shared__ double s0[TILE2], s2[TILE2];
-  __shared__ double sc[2 * TILE2];
   __shared__ double red[8];
-  double v0 = 0.0, v2 = 0.0;
-  if (a < ni && b < ni) {
-    for (int p = A.pstart[q]; p < A.pstart[q + 1]; ++p) {
-      const int kl = A.pair_kl[p], k = kl / A.Nang, l = kl - k * A.Nang;
-      const long long r = pure_row(A.skip, A.poff, k, f0 + a), c = pure_row(A.skip, A.poff, l, f0 + b);
-      if (r < 0 || c < 0) continue;
-      const double x = A.P[r + c * A.ldp];
-      v0 += A.pair_c[2 * p] * x;
-      v2 += A.pair_c[2 * p + 1] * x;
-    }
-  }
-  s0[t] = v0;
-  s2[t] = v2;
+  double *sc = part;  // 2 TILE2 channel weights, once the partial sums are added
+  auto at = [&](int kl, int i, int j) {
+    const int k = kl / A.Nang, l = kl - k * A.Nang;
+    const long long r = pure_row(A.skip, A.poff, k, f0 + i), c = pure_row(A.skip, A.poff, l, f0 + j);
+    return i < ni && j < ni && r >= 0 && c >= 0 ? A.P[r + c * A.ldp] : 0.0;
+  };
+  double v[2];
+  j_pair_sums<2>(A.pair_kl, A.pair_c, A.pstart[q], A.pstart[q + 1], at, part, v);
+  s0[t] = v[0];
+  s2[t] = v[1];
   __syncthreads();
   // traces tr(X s) = sum_ab X(a,b) s(b,a)
   const size_t tb = ((size_t)ilm * A.Nel + e) * 4 * TILE2;
@@ -112,6 +114,7 @@ __global__ void __launch_bounds__(NT) k_dia_j_gather(DJArgs A) {
   }
   __syncthreads();
   double j0 = 0.0, j2 = 0.0;
+#pragma unroll 4
   for (int p = 0; p < rank; ++p) {
     const double cp = sc[p];
     j0 += M[(size_t)p * 2 * TILE2 + t] * cp;
@@ -122,20 +125,27 @@ __global__ void __launch_bounds__(NT) k_dia_j_gather(DJArgs A) {
   out[TILE2 + t] = j2 * fac;
 }
 
-// preA(q,e) = sum_{j>e} db(q,j), preB(q,e) = sum_{j<e} ds(q,j)
-__global__ void k_dia_j_prefix(int n_q, int Nel, const double *ds, const double *db, double *preA, double *preB) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n_q) return;
-  double acc = 0.0;
-  for (int e = 0; e < Nel; ++e) {
-    preB[(size_t)q * Nel + e] = acc;
-    acc += ds[(size_t)q * Nel + e];
-  }
-  acc = 0.0;
-  for (int e = Nel - 1; e >= 0; --e) {
-    preA[(size_t)q * Nel + e] = acc;
-    acc += db[(size_t)q * Nel + e];
-  }
+struct DJBandArgs {
+  int Nel;
+  const int *LM_ilm;
+  const double *pq, *ds, *db;
+  double *Jin;
+};
+
+// The whole potential of (L,M) in element e, in place, one workgroup per (q, e):
+// Ja0 = Jin0 + preA P0 + preB Q0, Ja2 = Jin2 - preA P2 - preB Q2 with preA =
+// sum_{j>e} db(q,j), preB = sum_{j<e} ds(q,j).  Formed once here, an output block
+// reads two tiles per (L,M) instead of six.
+__global__ void __launch_bounds__(NT) k_dia_j_band(DJBandArgs A) {
+  const int q = blockIdx.x / A.Nel, e = blockIdx.x - q * A.Nel, t = threadIdx.x;
+  const double *ds = A.ds + (size_t)q * A.Nel, *db = A.db + (size_t)q * A.Nel;
+  double pa = 0.0, pb = 0.0;
+  for (int j = A.Nel - 1; j > e; --j) pa += db[j];
+  for (int j = 0; j < e; ++j) pb += ds[j];
+  const double *pq = A.pq + ((size_t)A.LM_ilm[q] * A.Nel + e) * 4 * TILE2;
+  double *jin = A.Jin + (size_t)blockIdx.x * 2 * TILE2;
+  jin[t] = jin[t] + pa * pq[t] + pb * pq[2 * TILE2 + t];
+  jin[TILE2 + t] = jin[TILE2 + t] - pa * pq[TILE2 + t] - pb * pq[3 * TILE2 + t];
 }
 
 struct DJOutArgs {
@@ -144,48 +154,44 @@ struct DJOutArgs {
   int Nel, Nang;
   const int *first, *ni, *skip;
   const long long *poff;
-  const double *pq, *Jin, *preA, *preB;
-  const int *LM_ilm, *out_start, *out_q;
+  const double *Jin;
+  const int *out_start, *out_q;
   const double *out_c;
 };
 
-// Ja0 = Jin0 + preA P0 + preB Q0, Ja2 = Jin2 - preA P2 - preB Q2 at entry t
-__device__ inline void dia_band(const DJOutArgs &A, int q, int e, int t, double &x0, double &x2) {
-  const size_t tb = ((size_t)A.LM_ilm[q] * A.Nel + e) * 4 * TILE2;
-  const size_t qe = (size_t)q * A.Nel + e;
-  const double pa = A.preA[qe], pb = A.preB[qe];
-  const double *jin = A.Jin + qe * 2 * TILE2;
-  x0 = jin[t] + pa * A.pq[tb + t] + pb * A.pq[tb + 2 * TILE2 + t];
-  x2 = jin[TILE2 + t] - pa * A.pq[tb + TILE2 + t] - pb * A.pq[tb + 3 * TILE2 + t];
-}
-
-// One workgroup per (output shell block (i,j), element).
+// One workgroup per (output shell block (i,j), element): the element's columns of
+// the block from top to bottom, zeros included, so that J is written in one pass
+// of whole columns.  A column shared with element e-1 is e-1's.  The blocks i of
+// one column run on one XCD, whose L2 joins their partial lines.  Bound by the
+// latency of the tile reads: fill + expand of N2 (16 shells per |m| <= 2) 72 + 276
+// -> 197 us (and 8 for the band tiles).
 __global__ void __launch_bounds__(NT) k_dia_j_expand(DJOutArgs A) {
-  const int ij = blockIdx.x / A.Nel, e = blockIdx.x - ij * A.Nel;
+  const int item = xcd_item(blockIdx.x, A.Nang * A.Nang * A.Nel);
+  if (item < 0) return;
+  const int je = item / A.Nang, i = item - je * A.Nang, j = je / A.Nel, e = je - j * A.Nel, ij = i * A.Nang + j;
   const int o0 = A.out_start[ij], o1 = A.out_start[ij + 1];
-  if (o0 == o1) return;
   const int t = threadIdx.x, a = t & 15, b = t >> 4;
-  const int ni = A.ni[e], f0 = A.first[e];
-  if (a >= ni || b >= ni) return;
-  if (e > 0 && a == 0 && b == 0) return;  // shared corner, written by element e-1
-  const int i = ij / A.Nang, j = ij - i * A.Nang;
-  const long long row = pure_row(A.skip, A.poff, i, f0 + a), col = pure_row(A.skip, A.poff, j, f0 + b);
-  if (row < 0 || col < 0) return;
-  const bool corner = (a == ni - 1 && b == ni - 1 && e + 1 < A.Nel);
-  double v = 0.0;
+  const int ni = A.ni[e], f0 = A.first[e], nn = e + 1 < A.Nel ? A.ni[e + 1] : 0;
+  __shared__ double sT[TILE2], sN[TILE];
+  double v = 0.0, w = 0.0;
+#pragma unroll 4
   for (int o = o0; o < o1; ++o) {
-    const int q = A.out_q[o];
-    double x0, x2;
-    dia_band(A, q, e, t, x0, x2);
-    if (corner) {
-      double y0, y2;
-      dia_band(A, q, e + 1, 0, y0, y2);
-      x0 += y0;
-      x2 += y2;
-    }
-    v += A.out_c[2 * o] * x0 + A.out_c[2 * o + 1] * x2;
+    const double *x = A.Jin + ((size_t)A.out_q[o] * A.Nel + e) * 2 * TILE2;
+    v += A.out_c[2 * o] * x[t] + A.out_c[2 * o + 1] * x[TILE2 + t];
   }
-  A.J[row + col * A.ldj] = v;
+  if (nn && t < TILE)
+#pragma unroll 4
+    for (int o = o0; o < o1; ++o) {
+      const double *x = A.Jin + ((size_t)A.out_q[o] * A.Nel + e + 1) * 2 * TILE2;
+      w += A.out_c[2 * o] * x[t] + A.out_c[2 * o + 1] * x[TILE2 + t];
+    }
+  if (t < TILE) sN[t] = w;
+  sT[t] = v;
+  __syncthreads();
+  if (nn && a == ni - 1 && b == ni - 1) sT[t] = v + sN[0];
+  __syncthreads();
+  double *J = A.J + A.poff[i] + A.poff[j] * A.ldj;
+  j_store_columns(J, A.ldj, (int)(A.poff[i + 1] - A.poff[i]), A.skip[i], A.skip[j], f0, ni, nn, e > 0, sT, sN);
 }
 
 // --- Exchange ----------------------------------------------------------------
@@ -1611,24 +1617,26 @@ void diatomic_op_build(DiatomicDevice &d, const std::vector<int> &ni, hipStream_
 
 void diatomic_coulomb_launch(const DiatomicDevice &d, const double *P, int64_t ldp, double *J, int64_t ldj,
                              hipStream_t s, KernelTimer *timer) {
-  fill_zero_launch(J, d.Nbf, d.Nbf, ldj, s);
-  if (d.n_LM == 0) return;
+  if (d.n_LM == 0) {
+    fill_zero_launch(J, d.Nbf, d.Nbf, ldj, s);
+    return;
+  }
   DJArgs a{P, ldp, d.Nel, d.Nang, d.first.p, d.ni.p, d.skip.p, d.poff.p, d.pq.p, d.chol.p, d.sigma.p,
            d.chol_off.p, d.chol_rank.p, d.LM_ilm.p, d.LM_fac.p, d.pstart.p, d.pair_kl.p, d.pair_c.p,
-           d.Jin.p, d.ds.p, d.db.p};
+           d.Jin.p, d.ds.p, d.db.p, d.n_LM};
   {
     TimedLaunch tl(timer, "diatomic_j_gather", s);
-    hipLaunchKernelGGL(k_dia_j_gather, dim3(d.n_LM * d.Nel), dim3(NT), 0, s, a);
+    hipLaunchKernelGGL(k_dia_j_gather, dim3(8 * xcd_share(d.n_LM * d.Nel)), dim3(NT), 0, s, a);
     hip_check(hipGetLastError(), "diatomic_j_gather");
   }
-  hipLaunchKernelGGL(k_dia_j_prefix, dim3((d.n_LM + 63) / 64), dim3(64), 0, s, d.n_LM, d.Nel, d.ds.p, d.db.p,
-                     d.preA.p, d.preB.p);
-  hip_check(hipGetLastError(), "diatomic_j_prefix");
-  DJOutArgs o{J, ldj, d.Nel, d.Nang, d.first.p, d.ni.p, d.skip.p, d.poff.p, d.pq.p, d.Jin.p, d.preA.p,
-              d.preB.p, d.LM_ilm.p, d.out_start.p, d.out_q.p, d.out_c.p};
+  DJBandArgs w{d.Nel, d.LM_ilm.p, d.pq.p, d.ds.p, d.db.p, d.Jin.p};
+  hipLaunchKernelGGL(k_dia_j_band, dim3(d.n_LM * d.Nel), dim3(NT), 0, s, w);
+  hip_check(hipGetLastError(), "diatomic_j_band");
+  DJOutArgs o{J, ldj, d.Nel, d.Nang, d.first.p, d.ni.p, d.skip.p, d.poff.p, d.Jin.p, d.out_start.p, d.out_q.p,
+              d.out_c.p};
   {
     TimedLaunch tl(timer, "diatomic_j_expand", s);
-    hipLaunchKernelGGL(k_dia_j_expand, dim3(d.Nang * d.Nang * d.Nel), dim3(NT), 0, s, o);
+    hipLaunchKernelGGL(k_dia_j_expand, dim3(8 * xcd_share(d.Nang * d.Nang * d.Nel)), dim3(NT), 0, s, o);
     hip_check(hipGetLastError(), "diatomic_j_expand");
   }
 }

@@ -220,7 +220,7 @@ struct AtomicDevice {
   DevArray<double> term_c;                // 4pi/(2L+1) * G_j * G_k
   PinnedArray<double> h_bnorm;
   // work buffers
-  DevArray<double> Jin, jsm, jbg, preA, preB;
+  DevArray<double> Jin, jsm, jbg;
   DevArray<double> hostP, hostOut;        // staging for host-pointer entry points
   int max_rank = 0;
   int64_t n_terms = 0, n_pairs = 0;
@@ -321,7 +321,7 @@ struct DiatomicDevice {
   DevArray<int> mirror;                   // absm: pairs (dst jk, src jk)
   int n_mirror = 0;
   PinnedArray<double> h_bnorm;
-  DevArray<double> Jin, ds, db, preA, preB;
+  DevArray<double> Jin, ds, db;
   DevArray<double> hostP, hostOut;
   int64_t n_terms = 0, n_runs = 0, n_pairs = 0;
   double flops_k_radial = 0.0, flops_k_angular = 0.0;
