@@ -25,9 +25,8 @@
 //
 // Each functional is one energy density per volume f(rho_a, rho_b, sigma_aa,
 // sigma_ab, sigma_bb, tau_a, tau_b) written once over a scalar type; the
-// potentials come from forward-mode differentiation (a value and one
-// directional derivative, one pass per input), so the derivative formulas
-// are never written by hand.
+// potentials come from forward-mode differentiation (a value and its derivatives
+// along all inputs), so the derivative formulas are never written by hand.
 #pragma once
 #include <cfloat>
 #include <cmath>
@@ -35,51 +34,88 @@
 namespace hfg {
 namespace xcf {
 
-// value and derivative along one input
-struct Dl {
-  double v, d;
+// value and derivatives along N inputs: the transcendental functions are evaluated
+// once for all of them
+template <int N> struct Dl {
+  double v, d[N];
 };
-__host__ __device__ inline Dl mk(double v, double d = 0.0) { return Dl{v, d}; }
-__host__ __device__ inline Dl operator+(Dl a, Dl b) { return {a.v + b.v, a.d + b.d}; }
-__host__ __device__ inline Dl operator-(Dl a, Dl b) { return {a.v - b.v, a.d - b.d}; }
-__host__ __device__ inline Dl operator-(Dl a) { return {-a.v, -a.d}; }
-__host__ __device__ inline Dl operator*(Dl a, Dl b) { return {a.v * b.v, a.d * b.v + a.v * b.d}; }
-__host__ __device__ inline Dl operator/(Dl a, Dl b) {
-  const double q = a.v / b.v;
-  return {q, (a.d - q * b.d) / b.v};
+#define HFG_DL template <int N> __host__ __device__ inline
+HFG_DL Dl<N> chain(double v, double s, const Dl<N> &a) {  // (v, s a')
+  Dl<N> r;
+  r.v = v;
+#pragma unroll
+  for (int k = 0; k < N; ++k) r.d[k] = s * a.d[k];
+  return r;
 }
-__host__ __device__ inline Dl operator+(Dl a, double b) { return {a.v + b, a.d}; }
-__host__ __device__ inline Dl operator+(double a, Dl b) { return {a + b.v, b.d}; }
-__host__ __device__ inline Dl operator-(Dl a, double b) { return {a.v - b, a.d}; }
-__host__ __device__ inline Dl operator-(double a, Dl b) { return {a - b.v, -b.d}; }
-__host__ __device__ inline Dl operator*(Dl a, double b) { return {a.v * b, a.d * b}; }
-__host__ __device__ inline Dl operator*(double a, Dl b) { return {a * b.v, a * b.d}; }
-__host__ __device__ inline Dl operator/(Dl a, double b) { return {a.v / b, a.d / b}; }
-__host__ __device__ inline Dl operator/(double a, Dl b) {
+HFG_DL Dl<N> operator+(const Dl<N> &a, const Dl<N> &b) {
+  Dl<N> r;
+  r.v = a.v + b.v;
+#pragma unroll
+  for (int k = 0; k < N; ++k) r.d[k] = a.d[k] + b.d[k];
+  return r;
+}
+HFG_DL Dl<N> operator-(const Dl<N> &a, const Dl<N> &b) {
+  Dl<N> r;
+  r.v = a.v - b.v;
+#pragma unroll
+  for (int k = 0; k < N; ++k) r.d[k] = a.d[k] - b.d[k];
+  return r;
+}
+HFG_DL Dl<N> operator-(const Dl<N> &a) { return chain(-a.v, -1.0, a); }
+HFG_DL Dl<N> operator*(const Dl<N> &a, const Dl<N> &b) {
+  Dl<N> r;
+  r.v = a.v * b.v;
+#pragma unroll
+  for (int k = 0; k < N; ++k) r.d[k] = a.d[k] * b.v + a.v * b.d[k];
+  return r;
+}
+HFG_DL Dl<N> operator/(const Dl<N> &a, const Dl<N> &b) {
+  const double i = 1.0 / b.v, q = a.v / b.v;
+  Dl<N> r;
+  r.v = q;
+#pragma unroll
+  for (int k = 0; k < N; ++k) r.d[k] = (a.d[k] - q * b.d[k]) * i;
+  return r;
+}
+HFG_DL Dl<N> operator+(const Dl<N> &a, double b) {
+  Dl<N> r = a;
+  r.v = a.v + b;
+  return r;
+}
+HFG_DL Dl<N> operator+(double a, const Dl<N> &b) { return b + a; }
+HFG_DL Dl<N> operator-(const Dl<N> &a, double b) { return a + -b; }
+HFG_DL Dl<N> operator-(double a, const Dl<N> &b) { return chain(a - b.v, -1.0, b); }
+HFG_DL Dl<N> operator*(const Dl<N> &a, double b) { return chain(a.v * b, b, a); }
+HFG_DL Dl<N> operator*(double a, const Dl<N> &b) { return chain(a * b.v, a, b); }
+HFG_DL Dl<N> operator/(const Dl<N> &a, double b) { return chain(a.v / b, 1.0 / b, a); }
+HFG_DL Dl<N> operator/(double a, const Dl<N> &b) {
   const double q = a / b.v;
-  return {q, -q * b.d / b.v};
+  return chain(q, -q / b.v, b);
 }
-__host__ __device__ inline Dl sqrt(Dl a) {
+HFG_DL Dl<N> sqrt(const Dl<N> &a) {
   const double s = ::sqrt(a.v);
-  return {s, 0.5 * a.d / s};
+  return chain(s, 0.5 / s, a);
 }
-__host__ __device__ inline Dl cbrt(Dl a) {
+HFG_DL Dl<N> cbrt(const Dl<N> &a) {
   const double c = ::cbrt(a.v);
-  return {c, a.d / (3.0 * c * c)};
+  return chain(c, 1.0 / (3.0 * c * c), a);
 }
-__host__ __device__ inline Dl log(Dl a) { return {::log(a.v), a.d / a.v}; }
-__host__ __device__ inline Dl exp(Dl a) {
+HFG_DL Dl<N> log(const Dl<N> &a) { return chain(::log(a.v), 1.0 / a.v, a); }
+HFG_DL Dl<N> exp(const Dl<N> &a) {
   const double e = ::exp(a.v);
-  return {e, e * a.d};
+  return chain(e, e, a);
 }
-__host__ __device__ inline Dl atan(Dl a) { return {::atan(a.v), a.d / (1.0 + a.v * a.v)}; }
-__host__ __device__ inline Dl asinh(Dl a) { return {::asinh(a.v), a.d / ::sqrt(1.0 + a.v * a.v)}; }
-__host__ __device__ inline Dl erf(Dl a) { return {::erf(a.v), a.d * 1.1283791670955126 * ::exp(-a.v * a.v)}; }
-__host__ __device__ inline double val(Dl a) { return a.v; }
+HFG_DL Dl<N> atan(const Dl<N> &a) { return chain(::atan(a.v), 1.0 / (1.0 + a.v * a.v), a); }
+HFG_DL Dl<N> asinh(const Dl<N> &a) { return chain(::asinh(a.v), 1.0 / ::sqrt(1.0 + a.v * a.v), a); }
+HFG_DL Dl<N> erf(const Dl<N> &a) { return chain(::erf(a.v), 1.1283791670955126 * ::exp(-a.v * a.v), a); }
+HFG_DL double val(const Dl<N> &a) { return a.v; }
+#undef HFG_DL
 __host__ __device__ inline double val(double a) { return a; }
 
 template <class T> __host__ __device__ inline T floor_at(T x, double lo) { return val(x) < lo ? T(x * 0.0 + lo) : x; }
-__host__ __device__ inline Dl floor_at(Dl x, double lo) { return x.v < lo ? mk(lo) : x; }
+template <int N> __host__ __device__ inline Dl<N> floor_at(Dl<N> x, double lo) {
+  return x.v < lo ? chain(lo, 0.0, Dl<N>{}) : x;
+}
 
 constexpr double kPi = 3.14159265358979323846;
 
@@ -351,18 +387,20 @@ template <class T> __host__ __device__ inline T lyp_c(T rho, T opz, T omz, T saa
          a * b * omega * (br - r2 * sig + (r2 - ra * ra) * sbb + (r2 - rb * rb) * saa);
 }
 
-// energy per volume of functional `id` (0: none)
-template <class T>
+// energy per volume of functional `id` (0: none; the meta-GGAs with MGGA)
+template <bool MGGA, class T>
 __host__ __device__ inline T energy(int id, T ra, T rb, T saa, T sab, T sbb, T ta, T tb, double thr, bool pol) {
   if (id == 0) return ra * 0.0;
   if (id == 106) return b88_pair(ra, rb, saa, sbb, thr, pol);
-  if (id == 202) {
-    T e = ra * 0.0;
-    if (!pol || val(ra) >= thr) e = e + 0.5 * tpss_x(2.0 * ra, 4.0 * floor_at(saa, 1e-40), 2.0 * ta);
-    if (!pol || val(rb) >= thr) e = e + 0.5 * tpss_x(2.0 * rb, 4.0 * floor_at(sbb, 1e-40), 2.0 * tb);
-    return e;
+  if constexpr (MGGA) {
+    if (id == 202) {
+      T e = ra * 0.0;
+      if (!pol || val(ra) >= thr) e = e + 0.5 * tpss_x(2.0 * ra, 4.0 * floor_at(saa, 1e-40), 2.0 * ta);
+      if (!pol || val(rb) >= thr) e = e + 0.5 * tpss_x(2.0 * rb, 4.0 * floor_at(sbb, 1e-40), 2.0 * tb);
+      return e;
+    }
+    if (id == 231) return tpss_c(ra, rb, saa, sab, sbb, ta, tb, thr);
   }
-  if (id == 231) return tpss_c(ra, rb, saa, sab, sbb, ta, tb, thr);
   if (id == 1) return slater_x(ra, rb);
   if (id == 101) return pbe_x_pair(ra, rb, saa, sbb, thr, pol);
   if (id == 406) return 0.75 * pbe_x_pair(ra, rb, saa, sbb, thr, pol) + pbe_c(ra, rb, saa, sab, sbb);
@@ -409,41 +447,52 @@ __host__ __device__ inline void exact_exchange(int id, double &kfrac, double &ks
   kernel = id == 433 ? 1 : id == 470 ? 2 : 0;
 }
 
-template <class T>
+template <bool MGGA, class T>
 __host__ __device__ inline T total(int xf, int cf, T ra, T rb, T saa, T sab, T sbb, T ta, T tb, double thr,
                                    bool pol) {
-  return energy(xf, ra, rb, saa, sab, sbb, ta, tb, thr, pol) + energy(cf, ra, rb, saa, sab, sbb, ta, tb, thr, pol);
+  return energy<MGGA>(xf, ra, rb, saa, sab, sbb, ta, tb, thr, pol) +
+         energy<MGGA>(cf, ra, rb, saa, sab, sbb, ta, tb, thr, pol);
 }
 
 // Unpolarized: x = (rho, sigma = |grad rho|^2, tau) -> energy per volume f and
-// v[k] = df/dx_k (sigma only with gga, tau only with mgga).
-__host__ __device__ inline void eval_unpol(int xf, int cf, const double x[3], double thr, bool gga, bool mgga, double &f,
-                                           double v[3]) {
+// v[k] = df/dx_k (tau only with MGGA; sigma's is zero without a gradient term).
+template <bool MGGA>
+__host__ __device__ inline void eval_unpol(int xf, int cf, const double x[3], double thr, double &f, double v[3]) {
+  constexpr int N = MGGA ? 3 : 2;
   f = v[0] = v[1] = v[2] = 0.0;
   if (!(x[0] >= thr)) return;
-  const int nk = mgga ? 3 : gga ? 2 : 1;
-  for (int k = 0; k < nk; ++k) {
-    const Dl r = mk(x[0], k == 0 ? 1.0 : 0.0), s = mk(x[1], k == 1 ? 1.0 : 0.0), t = mk(x[2], k == 2 ? 1.0 : 0.0);
-    const Dl e = total(xf, cf, 0.5 * r, 0.5 * r, 0.25 * s, 0.25 * s, 0.25 * s, 0.5 * t, 0.5 * t, thr, false);
-    f = e.v;
-    v[k] = e.d;
+  Dl<N> y[3];
+  for (int j = 0; j < 3; ++j) {
+    y[j] = chain(x[j], 0.0, Dl<N>{});
+    if (j < N) y[j].d[j] = 1.0;
   }
+  const Dl<N> r = 0.5 * y[0], s = 0.25 * y[1], t = 0.5 * y[2];
+  const Dl<N> e = total<MGGA>(xf, cf, r, r, s, s, s, t, t, thr, false);
+  f = e.v;
+  for (int k = 0; k < N; ++k) v[k] = e.d[k];
 }
 
 // Polarized: x = (rho_a, rho_b, sigma_aa, sigma_ab, sigma_bb, tau_a, tau_b)
-// -> f and v[k] = df/dx_k (the sigma derivatives only with gga, tau with mgga).
-__host__ __device__ inline void eval_pol(int xf, int cf, const double x[7], double thr, bool gga, bool mgga,
-                                         double &f, double v[7]) {
+// -> f and v[k] = df/dx_k.  Five inputs in one pass; the seven of a meta-GGA in
+// two, whose registers one pass would spill.
+template <bool MGGA>
+__host__ __device__ inline void eval_pol(int xf, int cf, const double x[7], double thr, double &f, double v[7]) {
+  constexpr int N = MGGA ? 4 : 5, M = MGGA ? 7 : 5;
   f = 0.0;
   for (int k = 0; k < 7; ++k) v[k] = 0.0;
   if (!(x[0] + x[1] >= thr)) return;
-  const int nk = mgga ? 7 : gga ? 5 : 2;
-  for (int k = 0; k < nk; ++k) {
-    Dl y[7];
-    for (int j = 0; j < 7; ++j) y[j] = mk(x[j], j == k ? 1.0 : 0.0);
-    const Dl e = total(xf, cf, y[0], y[1], y[2], y[3], y[4], y[5], y[6], thr, true);
+#pragma unroll 1
+  for (int k0 = 0; k0 < M; k0 += N) {
+    Dl<N> y[7];
+    for (int j = 0; j < 7; ++j) {
+      y[j].v = x[j];
+      for (int k = 0; k < N; ++k) y[j].d[k] = j == k0 + k ? 1.0 : 0.0;
+    }
+    const Dl<N> e = total<MGGA>(xf, cf, y[0], y[1], y[2], y[3], y[4], y[5], y[6], thr, true);
     f = e.v;
-    v[k] = e.d;
+    for (int j = 0; j < M; ++j)
+      for (int k = 0; k < N; ++k)
+        if (j == k0 + k) v[j] = e.d[k];
   }
 }
 

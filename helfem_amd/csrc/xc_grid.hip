@@ -445,9 +445,12 @@ template <int MODE> struct GgaShape {
   static constexpr int npv = MODE == 2 ? 5 : 4;  // point arrays per spin
 };
 
-// Threads: one per angular point, at least 256, at most 512 (the functional's
-// derivatives dominate: idle threads would hold registers for nothing).
-constexpr int XP_MAX = 256;
+// Threads: one per angular point, at least 256, at most 512.  Bound by the
+// functional's FP64 arithmetic and its register spills at 256 registers: O polarized
+// PBE 459 (ordered pairs, all phi points, 1024 threads) -> 236 (folded) -> 181 us
+// (all derivatives in one pass over the functional instead of one pass each).  256
+// threads: 169 us there, but TPSS and CAM-B3LYP of Xe 4 to 5% slower.
+constexpr int XP_MAX = 512;
 
 template <int MODE>
 __global__ void __launch_bounds__(XP_MAX) k_xc_point_gga(XCArgs A) {
@@ -457,8 +460,7 @@ __global__ void __launch_bounds__(XP_MAX) k_xc_point_gga(XCArgs A) {
   const int np = A.npair, nd = A.nd, lang = A.lang, nk = A.nk, nang = lang * nk;
   const bool pol = A.Db != nullptr;
   const int ns = pol ? 2 : 1;
-  const bool gga = xcf::is_gga(A.xf) || xcf::is_gga(A.cf);
-  const bool tau = MODE == 2;
+  constexpr bool tau = MODE == 2;
   const int na = max(G::nin * np, G::npv * nang), ncl = nd * lang;
   extern __shared__ double sm[];
   double *sA = sm;                         // [ns][na]
@@ -520,7 +522,7 @@ __global__ void __launch_bounds__(XP_MAX) k_xc_point_gga(XCArgs A) {
                             g[0][0] * g[1][0] + g[0][1] * g[1][1] + g[0][2] * g[1][2],
                             g[1][0] * g[1][0] + g[1][1] * g[1][1] + g[1][2] * g[1][2], tk[0], tk[1]};
       double v[7];
-      xcf::eval_pol(A.xf, A.cf, x7, A.thr, gga, tau, f, v);
+      xcf::eval_pol<tau>(A.xf, A.cf, x7, A.thr, f, v);
       va = v[0];
       vb = v[1];
       vta = v[5];
@@ -532,7 +534,7 @@ __global__ void __launch_bounds__(XP_MAX) k_xc_point_gga(XCArgs A) {
     } else {
       const double x3[3] = {rho[0], g[0][0] * g[0][0] + g[0][1] * g[0][1] + g[0][2] * g[0][2], tk[0]};
       double v[3];
-      xcf::eval_unpol(A.xf, A.cf, x3, A.thr, gga, tau, f, v);
+      xcf::eval_unpol<tau>(A.xf, A.cf, x3, A.thr, f, v);
       va = v[0];
       vta = v[2];
       for (int c = 0; c < 3; ++c) u[0][c] = 2.0 * w * v[1] * g[0][c];
