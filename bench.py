@@ -166,19 +166,20 @@ def kernel_stats(ctx, names):
 
 def xc_flops(hb, lang, mang):
     """FP64 operations of one exchange-correlation evaluation on the atomic
-    grid (the three kernels' sums with the element sizes, LDA point formulas
-    not counted): radial contraction 2 (Ni^2 + Ni) per (pair, point), the
-    pair-class and cos(d phi) transforms both ways per radial point, the
-    band assembly 3 Ni^2 per (pair, point)."""
+    grid as the three kernels execute them (element sizes, LDA point formulas
+    not counted): shell pairs once each, phi points 0 .. mang / 2.  Radial
+    contraction Ni^2 + 3 Ni per (pair, point), the pair-class and cos(d phi)
+    transforms both ways per radial point, the band assembly 2 Ni^2 + Ni per
+    (pair, point)."""
     mval = np.asarray(hb.mval)
     dmax = 2 * int(np.max(np.abs(mval)))
-    npair = int(np.sum(np.abs(mval[:, None] - mval[None, :]) <= dmax))
-    nd = 2 * dmax + 1
+    npair = len(mval) * (len(mval) + 1) // 2
+    nd, nk = dmax + 1, mang // 2 + 1
     nrad = 5 * 15
     ni = np.asarray(hb.nprim, dtype=float)
-    rad_in = npair * nrad * float(np.sum(2.0 * (ni * ni + ni)))
-    point = hb.Nel * nrad * (4.0 * lang * npair + 4.0 * lang * mang * nd)
-    rad_out = npair * nrad * float(np.sum(3.0 * ni * ni))
+    rad_in = npair * nrad * float(np.sum(ni * ni + 3.0 * ni))
+    point = hb.Nel * nrad * (4.0 * lang * npair + 4.0 * lang * nk * nd)
+    rad_out = npair * nrad * float(np.sum(2.0 * ni * ni + ni))
     return rad_in + point + rad_out
 
 
@@ -287,8 +288,8 @@ def fock_bench(H, cfg, ctx, steps, warmup, hb=None, P=None):
         out["energies"]["exchange"] = float(torch.sum(Pa * K))
         out["kernels_tflops"] = {k: (v[2] / max(v[1], 1e-30) / 1e9) for k, v in stats.items() if v[2] > 0}
         out["exchange_work"] = hb.work()
-        out["roofline"] = {"bound": "mfma", "kernel": {"atomic": "k_atomic_k_off_f64 + k_atomic_k_in_f64",
-                                                       "diatomic": "k_dia_k2_off<double> + k_dia_kin_lds<double>"}[kind] +
+        out["roofline"] = {"bound": "mfma", "kernel": {"atomic": "k_atomic_kc_off<double> + k_atomic_k_in_f64",
+                                                       "diatomic": "k_dia_k2_off<double> + k_dia_kin_fold<double>"}[kind] +
                                                       " (exchange: cross- and in-element launches of one build)",
                            "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                            "frac": achieved / FP64_PEAK_TFLOPS, "traffic": None,
