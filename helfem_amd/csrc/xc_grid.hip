@@ -352,8 +352,8 @@ __device__ inline void class_sums(const XCArgs &A, int ncs, Table table, Source 
 // [t][x] table (lanes read consecutive x).  Bound by the two Theta tables read
 // from L2 for every radial point (Xe: 2 x 0.35 MB) and the latency of the chain of
 // phases: Xe LDA 811 (ordered pairs, all phi points) -> 156 us, N2 pure-m
-// 629 -> 73 us.
-constexpr int LP_MAX = 512;
+// 629 -> 70 us (512 threads: 182 and 74).
+constexpr int LP_MAX = 256;
 
 __global__ void __launch_bounds__(LP_MAX) k_xc_point(XCArgs A) {
   const int e = blockIdx.x / A.nrad, i = blockIdx.x - e * A.nrad;
@@ -800,10 +800,8 @@ void launch_general(const XCGridDevice &g, const XCArgs &a, const XCArgs &b, boo
     if constexpr (MODE == 0) {
       const size_t lds = sizeof(double) * ns *
                          ((size_t)g.npair + (size_t)g.lang * nd + (size_t)g.lang * std::max(g.nk, g.npiece));
-      // few points per CU: more threads on each
-      const int threads = points >= 1024 ? 256 : 512;
       allow_lds(&k_xc_point, lds, "xc_point LDS size");
-      hipLaunchKernelGGL(k_xc_point, dim3(points), dim3(threads), lds, s, a);
+      hipLaunchKernelGGL(k_xc_point, dim3(points), dim3(LP_MAX), lds, s, a);
     } else {
       const size_t lds = xc_gga_point_lds(g, ns, MODE == 2);
       const int threads = std::min(XP_MAX, std::max(256, (g.lang * g.nk + 63) / 64 * 64));
