@@ -107,10 +107,12 @@ __device__ inline int batch_find(const int *start, int n, int b) {
 // included: tile T(a,b) = T[a + 16 b] in rows f0 + a, and in the last column the
 // next element's first column N[0 .. nn) (nn = 0 without one; N[0] is in T).
 // Block rows start at J, its first column at J; the shells leave out their first
-// roff and coff functions.  A wave per column, lanes along rows in 16-byte pairs
-// from the first aligned address on.
+// roff and coff functions, and may then have none (one element of two nodes: a
+// shell of m != 0).  A wave per column, lanes along rows in 16-byte pairs from the
+// first aligned address on.
 __device__ inline void j_store_columns(double *J, int64_t ldj, int nrow, int roff, int coff, int f0, int ni, int nn,
                                        int b0, const double *T, const double *N) {
+  if (nrow <= 0) return;
   const int lane = threadIdx.x & 63;
   for (int b = b0 + (int)(threadIdx.x >> 6); b < ni; b += (int)(blockDim.x >> 6)) {
     const int c = f0 + b - coff;

@@ -1,6 +1,7 @@
 """J is written in whole columns, zeros included: 8- and 16-byte aligned targets,
 padded leading dimensions, one to many elements of few or 15 functions, shells
-without their first function, and density pairs that do not fill a wave's run.
+without their first function, shells without any (one element of two nodes, m != 0),
+and density pairs that do not fill a wave's run.
 
 Bar: the oracle's J agrees to the rounding of sums over at most Nbf^2 products of
 which a J entry sees a few thousand; 1e-12 of the largest entry covers 4500 * 2^-52.
@@ -18,7 +19,8 @@ pytestmark = pytest.mark.gpu
 TOL, MARK = 1e-12, -7.25
 
 ATOMS = [(0, 0, 1, 15), (0, 0, 7, 2), (1, 1, 3, 2), (1, 0, 1, 3), (2, 2, 3, 15), (3, 1, 2, 6)]
-DIATOMICS = [([1], 1, 15), ([0, 1], 2, 15), ([2, 1], 5, 3), ([3, 2, 1], 2, 8)]
+DIATOMICS = [([1], 1, 15), ([0, 1], 2, 15), ([2, 1], 5, 3), ([3, 2, 1], 2, 8),
+             ([0, 1], 1, 2), ([1, 1], 1, 2), ([2, 1], 1, 2)]
 
 
 def _check(ob, hb, fn, ctx, pad, offset):
