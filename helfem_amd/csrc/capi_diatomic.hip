@@ -151,7 +151,11 @@ void diatomic_upload(hf_diatomic *h) {
   d.pq.upload(pq, s);
   // log scale per (L,|M|, element) that brings the P and Q tiles to the same
   // magnitude, sqrt(max|P| max|Q|): P_L(cosh mu) reaches 1e75 and Q_L 1e-56
-  // at L = 34, outside FP32, while their products across elements are O(1)
+  // at L = 34, outside FP32, while their products across elements are O(1).
+  // Pairs take P of the lower and Q of the upper element: the first element's Q
+  // (~ mu^-|M|, 1e60 at its first points) and the last one's P have no part in it;
+  // the tile that is used there is scaled to sqrt((L+|M|)!/(L-|M|)!), the usual
+  // magnitude.
   {
     std::vector<double> lsig((size_t)std::max(nlm, 1) * Nel, 0.0);
     for (size_t x = 0; x < (size_t)nlm * Nel; ++x) {
@@ -164,7 +168,14 @@ void diatomic_upload(hf_diatomic *h) {
           else
             mq = std::max(mq, v);
         }
-      if (mp > 0.0 && mq > 0.0) lsig[x] = 0.5 * (std::log(mp) - std::log(mq));
+      const int e = (int)(x % Nel);
+      const double usual = -0.5 * std::log(std::fabs(S.LMfac(S.lm_map[x / Nel].first, S.lm_map[x / Nel].second)));
+      if (e == 0 && mp > 0.0)
+        lsig[x] = std::log(mp) - usual;
+      else if (e == Nel - 1 && mq > 0.0)
+        lsig[x] = usual - std::log(mq);
+      else if (mp > 0.0 && mq > 0.0)
+        lsig[x] = 0.5 * (std::log(mp) - std::log(mq));
     }
     d.lsig.upload(lsig, s);
   }
@@ -228,6 +239,11 @@ void diatomic_upload(hf_diatomic *h) {
     oq.push_back(0);
     oc.assign(2, 0.0);
   }
+  // power of two that brings the coupling factor of each (L,|M|) to [1, 4)
+  d.h_fexp.assign(std::max(nlm, 1), 0);
+  for (int q = 0; q < nLM; ++q)
+    d.h_fexp[LMilm[q]] = LMfac[q] != 0.0 ? -2 * (int)std::floor(0.5 * std::ilogb(LMfac[q])) : 0;
+  d.fexp.upload(d.h_fexp, s);
   d.LM_ilm.upload(LMilm, s);
   d.LM_fac.upload(LMfac, s);
   d.pstart.upload(pstart, s);
@@ -313,8 +329,9 @@ void diatomic_upload(hf_diatomic *h) {
 // (basis.cpp:1905-1960), so R(j,k) = fac sum_i u(j,i) (x) V(i) with V_b(i) =
 // sum_l v_b(k,l) P(i,l), and the V tiles serve every row j.  A slot is one
 // (M, i); its lt entries are the (tile of (i,l), v0, v1) that pass the screen;
-// a row's jt entries are (slot, fac u0, fac u1).  l_j + L + l_i is even for
-// every coupling, so the slots of one parity of l_i have rows of their own.
+// a row's jt entries are (slot, fac u0, fac u1), fac times its power of two
+// (h_fexp).  l_j + L + l_i is even for every coupling, so the slots of one parity
+// of l_i have rows of their own.
 struct CoupleGroup {
   typedef std::pair<int, std::pair<double, double>> Entry;
   int ilm, par;
@@ -357,7 +374,7 @@ std::vector<std::vector<CoupleGroup>> couple_groups(hf_diatomic *h, const std::v
         if (Lk.empty()) continue;
         const size_t lm = (size_t)L * Mext + M + dmoff;
         const int ilm = ilm_of[lm];
-        const double fac = fac_of[lm];
+        const double fac = std::ldexp(fac_of[lm], d.h_fexp[ilm]);
         for (size_t q = 0; q < js.size(); ++q) {
           const int j = js[q], mi = mv[j] - M;
           if (std::abs(mi) > dmoff / 2) continue;

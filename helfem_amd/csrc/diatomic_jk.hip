@@ -962,10 +962,11 @@ __global__ void __launch_bounds__(KL_THREADS) k_dia_kin_lds(DKLArgs<T> A) {
 
 struct DFoldBuildArgs {
   const double *chol, *sigma;
-  const int *chol_off, *chol_rank, *ni;
+  const int *chol_off, *chol_rank, *ni, *fexp;
   int Nel;
-  size_t size;
-  double *T;  // [ilm*Nel + e][size]
+  size_t size, x0;  // x0: first ilm*Nel + e of the launch
+  double *T;        // [ilm*Nel + e][size]
+  double *scale;    // [ilm*Nel + e]
 };
 
 // q-th pair a <= b (anti: a < b) in the order b (b + 1) / 2 + a (b (b - 1) / 2 + a)
@@ -980,7 +981,8 @@ __device__ inline void fold_pair(int q, bool anti, int &a, int &b) {
 
 // Workgroups ((ilm, e), one of FB_PARTS shares of the row tiles); the channel
 // tiles sit in LDS when the rank allows (LDS), else they are read in place.
-// Bound by LDS reads (two per product and vector); N2: 1792 operators of 0.9 MB
+// |W(ca,bd)| <= max sum_p B_p^2 over the channels' entries (Cauchy-Schwarz), so
+// T is stored divided by that bound's power of two.  Bound by LDS reads (two per product and vector); N2: 1792 operators of 0.9 MB
 // in 3 ms (21 ms with the tiles read from L2).
 constexpr int FB_THREADS = 1024, FB_PARTS = 4;
 
@@ -989,7 +991,8 @@ __global__ void __launch_bounds__(FB_THREADS) k_dia_fold_build(DFoldBuildArgs A)
   __shared__ double Ml[LDS ? KL_RANK_MAX * 2 * TILE2 : 1];
   __shared__ double sgl[LDS ? KL_RANK_MAX : 1];
   __shared__ int2 pairs[2][TILE * (TILE + 1) / 2];
-  const int x = blockIdx.y, e = x % A.Nel, n = A.ni[e];
+  const size_t x = A.x0 + blockIdx.y;
+  const int e = (int)(x % A.Nel), n = A.ni[e];
   const int rank = A.chol_rank[x], off = A.chol_off[x];
   const double *Mg = A.chol + (size_t)off * 2 * TILE2, *sg = A.sigma + off;
   if (LDS) {
@@ -1007,6 +1010,20 @@ __global__ void __launch_bounds__(FB_THREADS) k_dia_fold_build(DFoldBuildArgs A)
   }
   __syncthreads();
   const double *M = LDS ? Ml : Mg, *sv = LDS ? sgl : sg;
+  double top = 0.0;
+  for (int q = threadIdx.x; q < 2 * TILE2; q += FB_THREADS) {  // zero outside the element
+    double v = 0.0;
+    for (int p = 0; p < rank; ++p) v += M[p * 2 * TILE2 + q] * M[p * 2 * TILE2 + q];
+    top = fmax(top, v);
+  }
+  __shared__ double red[FB_THREADS / 64];
+  for (int o = 32; o > 0; o >>= 1) top = fmax(top, __shfl_xor(top, o));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = top;
+  __syncthreads();
+  for (int w = 0; w < FB_THREADS / 64; ++w) top = fmax(top, red[w]);
+  const int ex = top > 0.0 && top < HUGE_VAL ? ilogb(top) : 0;
+  const double down = ldexp(1.0, -ex);
+  if (blockIdx.x == 0 && threadIdx.x == 0) A.scale[x] = ldexp(1.0, ex - A.fexp[x / A.Nel]);
   // sum_p sigma_p Mx(c,a) My(b,d) + sn sum_p sigma_p Mx(c2,a2) My(b2,d2)
   auto two = [&](int cx, int cy, int o1, int o2, int o3, int o4, double sn) {
     const double *p1 = M + cx * TILE2 + o1, *p2 = M + cy * TILE2 + o2, *p3 = M + cx * TILE2 + o3,
@@ -1044,7 +1061,7 @@ __global__ void __launch_bounds__(FB_THREADS) k_dia_fold_build(DFoldBuildArgs A)
           v = 0.5 * two(0, 1, at(c, a), at(b, d), at(c, b), at(a, d), sn);
         }
       }
-      out[q] = v;
+      out[q] = v * down;
     }
   }
 }
@@ -1058,6 +1075,7 @@ struct DFoldArgs {
   const long long *poff;
   const T *Top;
   size_t size;
+  const double *scale;
   const int4 *wg;
   const int *jk, *ent;
   const int4 *rec, *more;
@@ -1225,7 +1243,8 @@ __global__ void __launch_bounds__(KF_THREADS) k_dia_kin_fold(DFoldArgs<T> A) {
     fold_gemm<T>(top + (size_t)16 * rS * 16 * qS, X, wv - hA * rA, qA, qA * hA / kA, qA * (hA + 1) / kA, lane, aA);
   __syncthreads();
   // 4. partial tiles to LDS (rows rotated as the columns above), then the
-  // blocks' entries: Y(a,b) = Y_s + Y_a, Y(b,a) = Y_s - Y_a
+  // blocks' entries: Y(a,b) = Y_s + Y_a, Y(b,a) = Y_s - Y_a, scaled back
+  const double scale = A.scale[ilm * A.Nel + e];
   T *Ys = X, *Ya = X + kS * rS * 512;
   auto partial = [&](T *Y, int h, int rt, int nr, const vec acc[2]) {
 #pragma unroll
@@ -1274,6 +1293,8 @@ __global__ void __launch_bounds__(KF_THREADS) k_dia_kin_fold(DFoldArgs<T> A) {
         for (int h = 0; h < kA; ++h) va += (double)Ya[oa + h * rA * 512];
       }
       if (lo[i] > hi[i]) va = -va;  // Y(lo, hi) = Y_s + Y_a for lo < hi
+      vs *= scale;
+      va *= scale;
       if (fe + lo[i] >= sj && fe + hi[i] >= sk) atomicAdd(A.K + (oj + lo[i]) + (ok + hi[i]) * A.ldk, -(vs + va));
       if (both && fe + lo[i] >= sk && fe + hi[i] >= sj)
         atomicAdd(A.K + (ok + lo[i]) + (oj + hi[i]) * A.ldk, -(vs - va));
@@ -1562,24 +1583,28 @@ __global__ void __launch_bounds__(NT) k_dia_mirror(double *K, int64_t ldk, int N
 }  // namespace
 
 namespace {
-// P/Q tiles in matrix-core operand order (FP64 lanes).
-__global__ void __launch_bounds__(NT) k_pq_operands(const double *pq, double *pqo) {
+// P/Q tiles in matrix-core operand order (FP64 lanes), each with its half of the
+// power of two that the lists' coupling factors carry.
+__global__ void __launch_bounds__(NT) k_pq_operands(const double *pq, const int *fexp, double *pqo, int Nel) {
   const size_t o = (size_t)blockIdx.x * TILE2;
   const int u = threadIdx.x, lane = u >> 2;
-  pqo[o + u] = pq[o + (lane & 15) + TILE * Mma<double>::row(lane >> 4, u & 3)];
+  const double f = ldexp(1.0, -fexp[blockIdx.x / (4 * Nel)] / 2);
+  pqo[o + u] = f * pq[o + (lane & 15) + TILE * Mma<double>::row(lane >> 4, u & 3)];
 }
 }  // namespace
 
 void diatomic_op_build(DiatomicDevice &d, const std::vector<int> &ni, hipStream_t s) {
   d.pqo.alloc(d.pq.n);
   static_assert(NT == TILE2, "one thread per tile entry");
-  hipLaunchKernelGGL(k_pq_operands, dim3((unsigned)(d.pq.n / TILE2)), dim3(NT), 0, s, d.pq.p, d.pqo.p);
-  hip_check(hipGetLastError(), "pq_operands");
+  const size_t nx = (size_t)d.n_lm * d.Nel;
+  if (nx) {
+    hipLaunchKernelGGL(k_pq_operands, dim3((unsigned)(4 * nx)), dim3(NT), 0, s, d.pq.p, d.fexp.p, d.pqo.p, d.Nel);
+    hip_check(hipGetLastError(), "pq_operands");
+  }
   d.op_in = d.fold_in = false;
   d.Top2.release();
   d.Tfold.release();
   d.Tfold32.release();
-  const size_t nx = (size_t)d.n_lm * d.Nel;
   if (nx == 0 || d.max_rank > 2 * TILE2) return;
   const char *env = std::getenv("HFGPU_EXCHANGE_OP");
   if (env && std::atoi(env) == 0) return;
@@ -1601,11 +1626,12 @@ void diatomic_op_build(DiatomicDevice &d, const std::vector<int> &ni, hipStream_
   const size_t size = kf_size(d.fold_n);
   if (nx * size * sizeof(double) > fr / 4) return;
   d.Tfold.alloc(nx * size);
+  d.kf_scale.alloc(nx);
   const size_t step = (size_t)(65535 / d.Nel) * d.Nel;  // whole (L,|M|) within the grid's y limit
   for (size_t x = 0; x < nx; x += step) {
     const unsigned cnt = (unsigned)std::min(step, nx - x);
-    DFoldBuildArgs a{d.chol.p, d.sigma.p, d.chol_off.p + x, d.chol_rank.p + x, d.ni.p, d.Nel, size,
-                     d.Tfold.p + x * size};
+    DFoldBuildArgs a{d.chol.p, d.sigma.p, d.chol_off.p, d.chol_rank.p, d.ni.p, d.fexp.p, d.Nel, size, x,
+                     d.Tfold.p, d.kf_scale.p};
     if (d.max_rank <= KL_RANK_MAX)
       hipLaunchKernelGGL(k_dia_fold_build<true>, dim3(FB_PARTS, cnt), dim3(FB_THREADS), 0, s, a);
     else
@@ -1710,24 +1736,26 @@ void launch_fold(const DiatomicDevice &d, const T *top, const T *u, const T *v, 
   const void *f = reinterpret_cast<const void *>(&k_dia_kin_fold<T>);
   if (lds > 64 * 1024)
     hip_check(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "fold LDS size");
-  DFoldArgs<T> a{K, ldk, d.Nel, d.Nang, d.first.p, d.ni.p, d.skip.p, d.poff.p, top, kf_size(n), d.wg_kf.p, d.kf_jk.p,
+  DFoldArgs<T> a{K, ldk, d.Nel, d.Nang, d.first.p, d.ni.p, d.skip.p, d.poff.p, top, kf_size(n), d.kf_scale.p, d.wg_kf.p, d.kf_jk.p,
                  d.kf_ent.p, d.kf_rec.p, d.kf_more.p, u, v, pt, d.n_src, (int)d.sym};
   hipLaunchKernelGGL(k_dia_kin_fold<T>, dim3(d.n_wg_kf), dim3(KF_THREADS), lds, s, a);
   hip_check(hipGetLastError(), "diatomic_kin_fold");
 }
 
 // FP32 copy of the P/Q tiles with P kinds divided and Q kinds multiplied by
-// exp(lsig) of their (ilm, element), in storage and in operand order.
-__global__ void k_scale_pq_f32(const double *pq, const double *lsig, float *pq32, float *pqo32, int n_x) {
+// exp(lsig) of their (ilm, element), in storage order and, with their share of the
+// coupling factor's power of two, in operand order.
+__global__ void k_scale_pq_f32(const double *pq, const double *lsig, const int *fexp, float *pq32, float *pqo32,
+                               int n_x, int Nel) {
   const int x = blockIdx.x;
   if (x >= n_x) return;
-  const double up = exp(-lsig[x]), dn = exp(lsig[x]);
+  const double up = exp(-lsig[x]), dn = exp(lsig[x]), h = ldexp(1.0, -fexp[x / Nel] / 2);
   for (int u = threadIdx.x; u < 4 * TILE2; u += NT) {
     const int kind = u / TILE2, lane = (u & 255) >> 2;
     const size_t o = ((size_t)x * 4 + kind) * TILE2;
     const double f = kind < 2 ? up : dn;
     pq32[(size_t)x * 4 * TILE2 + u] = (float)(pq[(size_t)x * 4 * TILE2 + u] * f);
-    pqo32[o + (u & 255)] = (float)(pq[o + (lane & 15) + TILE * Mma<float>::row(lane >> 4, u & 3)] * f);
+    pqo32[o + (u & 255)] = (float)(pq[o + (lane & 15) + TILE * Mma<float>::row(lane >> 4, u & 3)] * f * h);
   }
 }
 }  // namespace
@@ -1742,9 +1770,9 @@ void diatomic_exchange_kernels(DiatomicDevice &d, const double *P, int64_t ldp, 
       d.pqo32.alloc(d.pq.n);
       d.chol32.alloc(d.chol.n);
       d.sigma32.alloc(d.sigma.n);
-      const int n_x = (int)(d.pq.n / (4 * TILE2));
-      hipLaunchKernelGGL(k_scale_pq_f32, dim3(n_x), dim3(NT), 0, s, d.pq.p, d.lsig.p, d.pq32.p, d.pqo32.p,
-                         n_x);
+      const int n_x = d.n_lm * d.Nel;
+      hipLaunchKernelGGL(k_scale_pq_f32, dim3(n_x), dim3(NT), 0, s, d.pq.p, d.lsig.p, d.fexp.p, d.pq32.p,
+                         d.pqo32.p, n_x, d.Nel);
       hip_check(hipGetLastError(), "scale_pq_f32");
       to_f32_launch(d.chol.p, d.chol32.p, d.chol.n, s);
       to_f32_launch(d.sigma.p, d.sigma32.p, d.sigma.n, s);

@@ -351,10 +351,17 @@ struct DiatomicDevice {
   // symmetries (k_dia_kin_fold), built on the device before the first exchange
   // when they fit the budget; per workgroup (ilm, e, first unit, units); per unit two rows
   // (output blocks jk, -1: none) and its entries: a slot's source record and
-  // the rows' weights (fac u0, fac u1)
+  // the rows' weights 2^fexp (fac u0, fac u1)
   bool fold_in = false;
   bool op_ready = false;                  // diatomic_op_build has run for the uploaded tables
   int fold_n = 0;                         // largest element size
+  // Operators reach (L+M)!/(L-M)!, 1e40 at |m| = 7, and the coupling factor its
+  // inverse, both beyond FP32: T holds 2^-x times its operator, x the exponent of
+  // its largest entry's bound, the lists 2^fexp times the factor (in [1, 4), fexp
+  // even), kf_scale 2^(x - fexp), applied in FP64 to the finished tiles.
+  std::vector<int> h_fexp;                // per (L,|M|)
+  DevArray<int> fexp;
+  DevArray<double> kf_scale;              // [n_lm*Nel]
   DevArray<double> Tfold;                 // [n_lm*Nel][kf_size(fold_n)]
   DevArray<float> Tfold32;
   DevArray<int4> wg_kf;
@@ -393,9 +400,10 @@ struct DiatomicDevice {
   DevArray<int> k2_kg, k2_gilm, k2_gslot;  // per k index: groups; per group: ilm, slot range
   DevArray<int> k2_sl, k2_lt;        // per slot: lt range; per lt: tile id
   DevArray<int> k2_jo, k2_js;        // per (group, wave): jt range; per jt: slot
-  DevArray<double> k2_ltv, k2_jtc;   // (v0, v1) per lt; K2_ROWS x (fac u0, -fac u1) per jt
+  DevArray<double> k2_ltv, k2_jtc;   // (v0, v1) per lt; K2_ROWS x 2^fexp (fac u0, -fac u1) per jt
   DevArray<float> k2_ltv32, k2_jtc32;  // FP32 copies (with list_gen as term_f32)
-  DevArray<double> pqo;              // pq in matrix-core operand order: lane (g,c) holds X(c, row(g,s)) in entry s
+  // 2^(-fexp / 2) pq in matrix-core operand order: lane (g,c) holds X(c, row(g,s)) in entry s
+  DevArray<double> pqo;
   DevArray<float> pqo32;
   double flops_off_k2 = 0.0;
 };

@@ -65,3 +65,27 @@ def test_one_element_and_density_holes(gpu_ctx):
         keep = keep & keep.T
         P = P * keep[sh][:, sh]
         assert relerr(hb.exchange(torch.as_tensor(P, device="cuda")).cpu().numpy(), ob.exchange(P)) <= TOL
+
+
+@pytest.mark.parametrize("lmm,top", [([2, 3, 4, 5, 6, 7, 8, 9], 7), (list(range(11)), 10)], ids=["m7", "m10"])
+def test_fp32_high_m(lmm, top, gpu_ctx):
+    """|m| where the in-element operators ((L+M)!/(L-M)!: 1e40 at M = 14, 1e58 at
+    M = 20) and the coupling factors, their inverse, leave FP32's range: every
+    block, and those that the largest M alone feeds (the density of m = -top in the
+    output of m = top), at the FP32 exchange's bar of the other tests, 2e-6 of the
+    largest entry."""
+    import torch
+    print(f"[gpu] FP32 diatomic exchange at |m| = {top}", flush=True)
+    hb = H.DiatomicBasis(7, 7, 2.074, lmm, 3, nnodes=8, ctx=gpu_ctx)
+    hb.compute_tei()
+    m = np.asarray(hb.mval)[np.asarray(hb.pure_idx) // hb.Nrad]
+    P = random_symmetric(hb.Nbf, seed=2105)
+    low = np.where((m[:, None] == -top) & (m[None, :] == -top), P, 0.0)
+    out = np.ix_(m == top, m == top)
+    for X, sel in ((P, np.ix_(m == m, m == m)), (low, out)):
+        Xd = torch.as_tensor(np.ascontiguousarray(X), device="cuda")
+        K64 = hb.exchange(Xd).cpu().numpy()[sel]
+        K32 = hb.exchange(Xd, precision="fp32").cpu().numpy()[sel]
+        assert np.max(np.abs(K64)) > 0.0 and np.all(np.isfinite(K32))
+        print(f"fp32 error {relerr(K32, K64):.2e}", flush=True)
+        assert relerr(K32, K64) <= 2e-6
