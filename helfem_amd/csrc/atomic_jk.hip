@@ -1543,7 +1543,8 @@ void atomic_rs_exchange_launch(AtomicDevice &d, const double *P, int64_t ldp, do
                       d.y_rb.p, d.y_chol.p, d.y_chol_off.p, d.y_chol_rank.p, d.act_jk.p, d.term_start.p,
                       d.term_off.p, d.term_c.p, efl, n_ef, d.rs_Lscale.p,
                       d.tiled ? d.ptile.p : nullptr, d.term_tile.p, d.n_src, (int)d.sym};
-      TimedLaunch tl(timer, "atomic_rs_k_yukawa", s);
+      TimedLaunch tl(timer, "atomic_rs_k_yukawa", s, 0.0,
+                     part == 1 ? "k_atomic_k_in" : d.kc ? "k_atomic_kc_off" : "k_atomic_k_off");
       if (part == 0 && d.kc) {
         launch_kc<double>(d, kc_args<double>(d, d.ptile.p, d.y_rs.p, d.y_rb.p, d.rs_Lscale.p, d.kc_ec.p, K, ldk, efl, n_ef),
                           s);
@@ -1595,7 +1596,8 @@ void atomic_exchange_launch(AtomicDevice &d, const double *P, int64_t ldp, doubl
     const int64_t grid = (int64_t)n_ef_pad * d.n_act;
     if (grid > 0x7fffffff) throw Error(-1, "exchange grid too large");
     const int *efl = part == 0 ? (d.sym ? d.ef_low.p : d.ef_off.p) : d.ef_in.p;
-    TimedLaunch tl(timer, name, s, part == 0 && d.kc ? d.frad_off + d.flops_kc : flops);
+    TimedLaunch tl(timer, name, s, part == 0 && d.kc ? d.frad_off + d.flops_kc : flops,
+                   part == 1 ? "k_atomic_k_in" : d.kc ? "k_atomic_kc_off" : "k_atomic_k_off");
     if (part == 0 && d.kc) {
       if (fp32)
         launch_kc<float>(d, kc_args<float>(d, d.ptile32.p, d.rs32.p, d.rb32.p, nullptr, d.kc_ec32.p, K, ldk, efl, n_ef), s);

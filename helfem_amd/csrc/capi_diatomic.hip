@@ -651,7 +651,7 @@ void build_fold(hf_diatomic *h, const std::vector<std::vector<int>> &rows,
   DiatomicDevice &d = h->dev;
   const int Na = S.Nang(), Nel = S.Nel(), nlm = d.n_lm;
   d.n_wg_kf = 0;
-  if (!d.fold_in || !d.tiled || !d.finite || d.dense_in) return;
+  if (!d.list_fold || !d.tiled || !d.finite || d.dense_in) return;
   struct Unit {
     int jk[KF_ROWS];
     std::vector<int4> rec;
@@ -790,8 +790,14 @@ void build_exchange_lists(hf_diatomic *h, hipStream_t s) {
   // no shared rows)
   bool finite = true;
   for (size_t q = 0; q < mask.size(); ++q) finite = finite && d.h_bnorm.p[q] < 1e30;
-  if (!d.screen_mask.empty() && mask == d.screen_mask && d.sym == d.list_sym && finite == d.finite) return;
+  if (!d.screen_mask.empty() && mask == d.screen_mask && d.sym == d.list_sym && finite == d.finite &&
+      (d.fold_in ? d.list_fold : d.list_terms))
+    return;
   d.finite = finite;
+  // the lists serve both precisions where one has the folded operators and the
+  // other does not
+  d.list_fold = d.fold_state[0] == 1 || d.fold_state[1] == 1;
+  const bool want_terms = d.fold_state[0] == -1 || d.fold_state[1] == -1;
   d.screen_mask.clear();  // no lists until all of them are there
   auto done = [&] {
     d.screen_mask = mask;
@@ -888,7 +894,8 @@ void build_exchange_lists(hf_diatomic *h, hipStream_t s) {
   // 3.8 M terms, 0.2 GB): the one-step, Cholesky-form and dense ones
   d.n_wg_kl = 0;
   d.n_wg_op = 0;
-  if (act.empty() || ((S.Nel() < 2 || d.k2) && d.n_wg_kf > 0)) {
+  d.list_terms = act.empty() || want_terms || !((S.Nel() < 2 || d.k2) && d.n_wg_kf > 0);
+  if (act.empty() || !d.list_terms) {
     done();
     return;
   }
@@ -1079,11 +1086,12 @@ void exchange_launch(hf_diatomic *h, const double *P, int64_t ldp, double *K, in
   DiatomicDevice &d = h->dev;
   hipStream_t s = h->ctx->cur;
   if (!d.op_ready) {
-    // the in-element operators, before the first exchange of these tables
-    // (density-functional builds without exact exchange never need them)
+    // before the first exchange of these tables (density-functional builds
+    // without exact exchange never need it)
     diatomic_op_build(d, h->host.rad.ni, s);
     d.op_ready = true;
   }
+  d.fold_in = diatomic_fold_ready(d, fp32, !d.dense_in, s);
   block_stats_launch(P, ldp, d.Nrad, d.Nang, d.skip.p, d.poff.p, d.stats.p, d.h_stats.p, s);
   hip_check(hipStreamSynchronize(s), "block statistics sync");
   const bool symmetric = block_stats_reduce(d.h_stats.p, d.Nrad, d.Nang, d.h_bnorm.p);

@@ -960,12 +960,13 @@ __global__ void __launch_bounds__(KL_THREADS) k_dia_kin_lds(DKLArgs<T> A) {
 // matrix pipe's, the gathers 0.65, the output 0.55, the folding the rest (one
 // workgroup per CU, its phases one after another).
 
+template <typename T>
 struct DFoldBuildArgs {
   const double *chol, *sigma;
   const int *chol_off, *chol_rank, *ni, *fexp;
   int Nel;
   size_t size, x0;  // x0: first ilm*Nel + e of the launch
-  double *T;        // [ilm*Nel + e][size]
+  T *out;           // [ilm*Nel + e][size]
   double *scale;    // [ilm*Nel + e]
 };
 
@@ -986,8 +987,8 @@ __device__ inline void fold_pair(int q, bool anti, int &a, int &b) {
 // in 3 ms (21 ms with the tiles read from L2).
 constexpr int FB_THREADS = 1024, FB_PARTS = 4;
 
-template <bool LDS>
-__global__ void __launch_bounds__(FB_THREADS) k_dia_fold_build(DFoldBuildArgs A) {
+template <bool LDS, typename T>
+__global__ void __launch_bounds__(FB_THREADS) k_dia_fold_build(DFoldBuildArgs<T> A) {
   __shared__ double Ml[LDS ? KL_RANK_MAX * 2 * TILE2 : 1];
   __shared__ double sgl[LDS ? KL_RANK_MAX : 1];
   __shared__ int2 pairs[2][TILE * (TILE + 1) / 2];
@@ -1043,7 +1044,7 @@ __global__ void __launch_bounds__(FB_THREADS) k_dia_fold_build(DFoldBuildArgs A)
     const int rt = anti ? tile - rs : tile;
     const int np = kf_pairs(n, anti), K = kf_inner(n, anti);
     const double sn = anti ? -1.0 : 1.0;
-    double *out = A.T + (size_t)x * A.size + (anti ? (size_t)16 * rs * kf_inner(n, false) : 0) + (size_t)16 * rt * K;
+    T *out = A.out + x * A.size + (anti ? (size_t)16 * rs * kf_inner(n, false) : 0) + (size_t)16 * rt * K;
     for (int q = threadIdx.x; q < 16 * K; q += FB_THREADS) {
       const int quad = q >> 8, lane = (q >> 2) & 63, st = q & 3;
       const int row = 16 * rt + (lane & 15), k = 16 * quad + 4 * st + (lane >> 4);
@@ -1061,7 +1062,7 @@ __global__ void __launch_bounds__(FB_THREADS) k_dia_fold_build(DFoldBuildArgs A)
           v = 0.5 * two(0, 1, at(c, a), at(b, d), at(c, b), at(a, d), sn);
         }
       }
-      out[q] = v * down;
+      out[q] = (T)(v * down);
     }
   }
 }
@@ -1602,6 +1603,53 @@ __global__ void __launch_bounds__(NT) k_pq_operands(const double *pq, const int 
 }
 }  // namespace
 
+namespace {
+template <typename T>
+void fold_build(DiatomicDevice &d, DevArray<T> &out, hipStream_t s) {
+  const size_t nx = (size_t)d.n_lm * d.Nel, size = kf_size(d.fold_n);
+  out.alloc(nx * size);
+  d.kf_scale.alloc(nx);
+  const size_t step = (size_t)(65535 / d.Nel) * d.Nel;  // whole (L,|M|) within the grid's y limit
+  for (size_t x = 0; x < nx; x += step) {
+    const unsigned cnt = (unsigned)std::min(step, nx - x);
+    DFoldBuildArgs<T> a{d.chol.p, d.sigma.p, d.chol_off.p, d.chol_rank.p, d.ni.p, d.fexp.p, d.Nel, size, x,
+                        out.p, d.kf_scale.p};
+    if (d.max_rank <= KL_RANK_MAX)
+      hipLaunchKernelGGL((k_dia_fold_build<true, T>), dim3(FB_PARTS, cnt), dim3(FB_THREADS), 0, s, a);
+    else
+      hipLaunchKernelGGL((k_dia_fold_build<false, T>), dim3(FB_PARTS, cnt), dim3(FB_THREADS), 0, s, a);
+    hip_check(hipGetLastError(), "diatomic_fold_build");
+  }
+}
+}  // namespace
+
+bool diatomic_fold_ready(DiatomicDevice &d, bool fp32, bool allowed, hipStream_t s) {
+  int &state = d.fold_state[fp32];
+  if (state == 0) {
+    state = -1;
+    if (d.fold_form && allowed) {
+      size_t fr = 0, tot = 0;
+      hip_check(hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
+      double budget = fr / 4;  // keep three quarters of the free memory for densities and tiles
+      if (const char *env = std::getenv("HFGPU_EXCHANGE_FOLD_GIB")) budget = std::atof(env) * (1ull << 30);
+      const double bytes =
+          (double)d.n_lm * d.Nel * kf_size(d.fold_n) * (fp32 ? sizeof(float) : sizeof(double));
+      if (bytes <= budget) try {
+          if (fp32)
+            fold_build(d, d.Tfold32, s);
+          else
+            fold_build(d, d.Tfold, s);
+          state = 1;
+        } catch (const Error &e) {
+          if (e.code != -4) throw;  // no room after all: the Cholesky form needs none
+          (void)hipGetLastError();
+          (void)(fp32 ? d.Tfold32.release() : d.Tfold.release());
+        }
+    }
+  }
+  return state == 1;
+}
+
 void diatomic_op_build(DiatomicDevice &d, const std::vector<int> &ni, hipStream_t s) {
   d.pqo.alloc(d.pq.n);
   static_assert(NT == TILE2, "one thread per tile entry");
@@ -1610,20 +1658,20 @@ void diatomic_op_build(DiatomicDevice &d, const std::vector<int> &ni, hipStream_
     hipLaunchKernelGGL(k_pq_operands, dim3((unsigned)(4 * nx)), dim3(NT), 0, s, d.pq.p, d.fexp.p, d.pqo.p, d.Nel);
     hip_check(hipGetLastError(), "pq_operands");
   }
-  d.op_in = d.fold_in = false;
+  d.op_in = d.fold_form = d.fold_in = false;
+  d.fold_state[0] = d.fold_state[1] = 0;
   d.Top2.release();
   d.Tfold.release();
   d.Tfold32.release();
   if (nx == 0 || d.max_rank > 2 * TILE2) return;
   const char *env = std::getenv("HFGPU_EXCHANGE_OP");
   if (env && std::atoi(env) == 0) return;
-  size_t fr = 0, tot = 0;
-  hip_check(hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
-  // keep three quarters of the free memory for densities and tiles
   if (env) {
+    size_t fr = 0, tot = 0;
+    hip_check(hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
     // on N2 (lmax 16) slower than the Cholesky-form kernel (16.2 against 13.1
     // ms): each workgroup streams its 1.75 MB operator for 16 runs
-    if (nx * OP_TSIZE * sizeof(double) > fr / 4) return;
+    if (nx * OP_TSIZE * sizeof(double) > fr / 4) return;  // keep three quarters of the free memory
     d.Top2.alloc(nx * OP_TSIZE);
     DOpBuildArgs a{d.chol.p, d.sigma.p, d.chol_off.p, d.chol_rank.p, d.ni.p, d.Nel, d.Top2.p};
     hipLaunchKernelGGL(k_dia_op_build, dim3((unsigned)(nx * OP_KS)), dim3(NT), 0, s, a);
@@ -1632,22 +1680,7 @@ void diatomic_op_build(DiatomicDevice &d, const std::vector<int> &ni, hipStream_
     return;
   }
   d.fold_n = *std::max_element(ni.begin(), ni.end());
-  const size_t size = kf_size(d.fold_n);
-  if (nx * size * sizeof(double) > fr / 4) return;
-  d.Tfold.alloc(nx * size);
-  d.kf_scale.alloc(nx);
-  const size_t step = (size_t)(65535 / d.Nel) * d.Nel;  // whole (L,|M|) within the grid's y limit
-  for (size_t x = 0; x < nx; x += step) {
-    const unsigned cnt = (unsigned)std::min(step, nx - x);
-    DFoldBuildArgs a{d.chol.p, d.sigma.p, d.chol_off.p, d.chol_rank.p, d.ni.p, d.fexp.p, d.Nel, size, x,
-                     d.Tfold.p, d.kf_scale.p};
-    if (d.max_rank <= KL_RANK_MAX)
-      hipLaunchKernelGGL(k_dia_fold_build<true>, dim3(FB_PARTS, cnt), dim3(FB_THREADS), 0, s, a);
-    else
-      hipLaunchKernelGGL(k_dia_fold_build<false>, dim3(FB_PARTS, cnt), dim3(FB_THREADS), 0, s, a);
-    hip_check(hipGetLastError(), "diatomic_fold_build");
-  }
-  d.fold_in = true;
+  d.fold_form = true;
 }
 
 void diatomic_coulomb_launch(const DiatomicDevice &d, const double *P, int64_t ldp, double *J, int64_t ldj,
@@ -1796,7 +1829,7 @@ void diatomic_exchange_kernels(DiatomicDevice &d, const double *P, int64_t ldp, 
         to_f32_launch(d.k2_ltv.p, d.k2_ltv32.p, d.k2_ltv.n, s);
         to_f32_launch(d.k2_jtc.p, d.k2_jtc32.p, d.k2_jtc.n, s);
       }
-      if (d.n_wg_kf > 0) {
+      if (d.fold_in && d.n_wg_kf > 0) {
         d.kf_u32.alloc(d.kf_u.n);
         d.kf_v32.alloc(d.kf_v.n);
         to_f32_launch(d.kf_u.p, d.kf_u32.p, d.kf_u.n, s);
@@ -1838,30 +1871,25 @@ void diatomic_exchange_kernels(DiatomicDevice &d, const double *P, int64_t ldp, 
                  d.ilm_rstart.p, d.ilm_runs.p, d.lrun_tstart.p, d.term_il.p, d.term_f.p, d.Ypart.p};
       DKRedArgs r{K, ldk, d.Nel, d.Nang, d.first.p, d.ni.p, d.skip.p, d.poff.p, d.act_jk.p, d.act_lstart.p,
                   d.Ypart.p};
-      TimedLaunch tl(timer, name, s, flops);
+      TimedLaunch tl(timer, name, s, flops, "k_dia_kin_gemm");
       hipLaunchKernelGGL(k_dia_kin_gemm, dim3(d.n_wg_in), dim3(NT), 0, s, g);
       hip_check(hipGetLastError(), "diatomic_kin_gemm");
       hipLaunchKernelGGL(k_dia_kin_reduce, dim3(d.n_act * d.Nel), dim3(NT), 0, s, r);
       hip_check(hipGetLastError(), "diatomic_kin_reduce");
       continue;
     }
-    if (part == 1 && d.n_wg_kf > 0) {
-      TimedLaunch tl(timer, name, s, d.flops_in_kf);
-      if (fp32) {
-        if (d.Tfold32.n != d.Tfold.n) {
-          d.Tfold32.alloc(d.Tfold.n);
-          to_f32_launch(d.Tfold.p, d.Tfold32.p, d.Tfold.n, s);
-        }
+    if (part == 1 && d.fold_in && d.n_wg_kf > 0) {
+      TimedLaunch tl(timer, name, s, d.flops_in_kf, "k_dia_kin_fold");
+      if (fp32)
         launch_fold<float>(d, d.Tfold32.p, d.kf_u32.p, d.kf_v32.p, d.ptile32.p, K, ldk, s);
-      } else {
+      else
         launch_fold<double>(d, d.Tfold.p, d.kf_u.p, d.kf_v.p, d.ptile.p, K, ldk, s);
-      }
       continue;
     }
     if (part == 1 && d.op_in && d.tiled && !fp32 && d.n_wg_op > 0) {
       // timed against the Cholesky-form flop count of the same results (the
       // reference's algorithm), so the rate compares with the other form
-      TimedLaunch tl(timer, name, s, flops);
+      TimedLaunch tl(timer, name, s, flops, "k_dia_kin_op");
       DOpArgs a{K, ldk, d.Nel, d.Nang, d.first.p, d.ni.p, d.skip.p, d.poff.p, d.Top2.p, d.act_jk.p,
                 d.lrun_tstart.p, d.term_f.p, d.wg_op.p, d.kl_runs.p, d.run_act.p, d.ptile.p, d.term_tile.p,
                 d.n_src, (int)d.sym};
@@ -1870,7 +1898,7 @@ void diatomic_exchange_kernels(DiatomicDevice &d, const double *P, int64_t ldp, 
       continue;
     }
     if (part == 1 && d.n_wg_kl > 0) {
-      TimedLaunch tl(timer, name, s, flops);
+      TimedLaunch tl(timer, name, s, flops, "k_dia_kin_lds");
       if (fp32) {
         DKLArgs<float> a{d.P32.p, d.Nbf, K, ldk, d.Nel, d.Nang, d.first.p, d.ni.p, d.skip.p, d.poff.p,
                          d.chol32.p, d.sigma32.p, d.chol_off.p, d.chol_rank.p, d.act_jk.p, d.lrun_tstart.p,
@@ -1894,7 +1922,7 @@ void diatomic_exchange_kernels(DiatomicDevice &d, const double *P, int64_t ldp, 
       continue;
     }
     if (part == 0 && d.k2) {
-      TimedLaunch tl(timer, name, s, d.flops_off_k2);
+      TimedLaunch tl(timer, name, s, d.flops_off_k2, "k_dia_k2_off");
       if (fp32) {
         DK2Args<float> a{d.ptile32.p, d.n_src, K, ldk, d.Nel, d.Nang, d.first.p, d.ni.p, d.skip.p, d.poff.p,
                          d.pqo32.p, d.lsig.p, d.k2_wg.p, d.k2_kshell.p, d.k2_rows.p, d.k2_kg.p, d.k2_gilm.p,
@@ -1914,7 +1942,7 @@ void diatomic_exchange_kernels(DiatomicDevice &d, const double *P, int64_t ldp, 
     const int64_t grid = (int64_t)n_ef_pad * d.n_act;
     if (grid > 0x7fffffff) throw Error(-1, "exchange grid too large");
     const int *efl = part == 0 ? (d.sym ? d.ef_low.p : d.ef_off.p) : d.ef_in.p;
-    TimedLaunch tl(timer, name, s, flops);
+    TimedLaunch tl(timer, name, s, flops, part == 0 ? "k_dia_k_off" : "k_dia_k_in");
     if (fp32) {
       DKArgs<float> a{d.P32.p, d.Nbf, K, ldk, d.Nel, d.Nang, d.n_act, d.first.p, d.ni.p, d.skip.p, d.poff.p,
                       d.pq32.p, d.chol32.p, d.sigma32.p, d.chol_off.p, d.chol_rank.p, d.act_jk.p, d.act_lstart.p,

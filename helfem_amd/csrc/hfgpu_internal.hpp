@@ -65,11 +65,12 @@ inline void hip_check(hipError_t e, const char *what) {
   if (e != hipSuccess) throw Error(-3, std::string(what) + ": " + hipGetErrorString(e));
 }
 
-// Optional per-kernel timing with HIP events recorded on the launch stream.
+// Optional per-kernel timing with HIP events recorded on the launch stream; a
+// launch with several forms counts under its own name and its kernel's.
 struct KernelTimer {
   bool on = false;
   struct Pending {
-    const char *name;
+    const char *name, *kernel;
     hipEvent_t a, b;
     double work;
   };
@@ -79,12 +80,12 @@ struct KernelTimer {
     long count = 0;
   };
   std::map<std::string, Acc> acc;
-  void begin(const char *name, hipStream_t s, double work, hipEvent_t *ev) {
+  void begin(const char *name, hipStream_t s, double work, hipEvent_t *ev, const char *kernel = nullptr) {
     if (!on) return;
     hip_check(hipEventCreate(&ev[0]), "hipEventCreate");
     hip_check(hipEventCreate(&ev[1]), "hipEventCreate");
     hip_check(hipEventRecord(ev[0], s), "hipEventRecord");
-    pending.push_back({name, ev[0], ev[1], work});
+    pending.push_back({name, kernel, ev[0], ev[1], work});
   }
   void end(hipStream_t s, hipEvent_t *ev) {
     if (!on) return;
@@ -95,10 +96,13 @@ struct KernelTimer {
       hip_check(hipEventSynchronize(p.b), "hipEventSynchronize");
       float ms = 0.f;
       hip_check(hipEventElapsedTime(&ms, p.a, p.b), "hipEventElapsedTime");
-      Acc &a = acc[p.name];
-      a.ms += ms;
-      a.work += p.work;
-      a.count += 1;
+      for (const char *n : {p.name, p.kernel}) {
+        if (!n) continue;
+        Acc &a = acc[n];
+        a.ms += ms;
+        a.work += p.work;
+        a.count += 1;
+      }
       (void)hipEventDestroy(p.a);
       (void)hipEventDestroy(p.b);
     }
@@ -111,8 +115,9 @@ struct TimedLaunch {
   KernelTimer *t;
   hipStream_t s;
   hipEvent_t ev[2];
-  TimedLaunch(KernelTimer *t_, const char *name, hipStream_t s_, double work = 0.0) : t(t_), s(s_) {
-    if (t) t->begin(name, s, work, ev);
+  TimedLaunch(KernelTimer *t_, const char *name, hipStream_t s_, double work = 0.0, const char *kernel = nullptr)
+      : t(t_), s(s_) {
+    if (t) t->begin(name, s, work, ev, kernel);
   }
   ~TimedLaunch() {
     if (t && t->on) (void)hipEventRecord(ev[1], s);
@@ -348,12 +353,15 @@ struct DiatomicDevice {
   DevArray<int> wg_op;
   int n_wg_op = 0;
   // in-element exchange as dense operators folded by the transposition
-  // symmetries (k_dia_kin_fold), built on the device before the first exchange
-  // when they fit the budget; per workgroup (ilm, e, first unit, units); per unit two rows
-  // (output blocks jk, -1: none) and its entries: a slot's source record and
-  // the rows' weights 2^fexp (fac u0, fac u1)
-  bool fold_in = false;
+  // symmetries (k_dia_kin_fold), built on the device before the first exchange of
+  // a precision when they fit the budget; per workgroup (ilm, e, first unit,
+  // units); per unit two rows (output blocks jk, -1: none) and its entries: a
+  // slot's source record and the rows' weights 2^fexp (fac u0, fac u1)
   bool op_ready = false;                  // diatomic_op_build has run for the uploaded tables
+  bool fold_form = false;                 // ... and chose the folded operators
+  int fold_state[2] = {0, 0};             // FP64, FP32 operators: 0 not asked for yet, 1 ready, -1 not used
+  bool fold_in = false;                   // this call's precision has them
+  bool list_fold = false, list_terms = false;  // the lists are for the folded form; hold every single term
   int fold_n = 0;                         // largest element size
   // Operators reach (L+M)!/(L-M)!, 1e40 at |m| = 7, and the coupling factor its
   // inverse, both beyond FP32: T holds 2^-x times its operator, x the exponent of
@@ -567,11 +575,16 @@ bool symmetric_exchange_allowed();
 void diatomic_exchange_kernels(DiatomicDevice &d, const double *P, int64_t ldp, double *K, int64_t ldk,
                                hipStream_t s, KernelTimer *timer, bool fp32 = false);
 void diatomic_build_operator(const DiatomicSetup &S, DiatomicDevice &d, hipStream_t s);
-// the in-element operators from the device Cholesky tiles, when they fit the
-// budget: folded ones (k_dia_kin_fold, sets d.fold_in; the default), or the
-// plain ones of k_dia_kin_op with HFGPU_EXCHANGE_OP=1 (d.op_in); neither with
+// chooses the in-element form of the uploaded tables: folded operators
+// (k_dia_kin_fold; the default), the plain ones of k_dia_kin_op with
+// HFGPU_EXCHANGE_OP=1 (d.op_in, built here when they fit the budget), neither with
 // HFGPU_EXCHANGE_OP=0 (the Cholesky-form kernel)
 void diatomic_op_build(DiatomicDevice &d, const std::vector<int> &ni, hipStream_t s);
+// true when the folded operators of this precision are on the device; its first
+// call builds them from the Cholesky tiles.  False, and the Cholesky form runs,
+// where they exceed the budget (HFGPU_EXCHANGE_FOLD_GIB, default a quarter of the
+// free memory), their allocation fails, or allowed is false.
+bool diatomic_fold_ready(DiatomicDevice &d, bool fp32, bool allowed, hipStream_t s);
 constexpr int OP_RUNS = 16;  // runs per k_dia_kin_op workgroup
 
 }  // namespace hfg

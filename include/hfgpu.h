@@ -60,7 +60,8 @@ int hf_ctx_get_stream(hf_ctx *ctx, void **stream);
 int hf_ctx_synchronize(hf_ctx *ctx);
 /* Per-kernel timing: with timing on, every kernel launch of this context is
  * bracketed by HIP events on its stream.  hf_ctx_kernel_stats returns, for
- * kernel `name`, out[0] = launches, out[1] = summed milliseconds, out[2] =
+ * kernel `name` (a launch of the exchange under its own name and under that of
+ * the kernel it chose), out[0] = launches, out[1] = summed milliseconds, out[2] =
  * summed algorithmic flops.  Turning timing off clears the totals.  (No
  * counterpart in the reference, which has only wall-clock FockTimer,
  * src/general/scf_driver_common.h:69-170.) */

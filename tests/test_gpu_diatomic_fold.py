@@ -13,6 +13,7 @@ import pytest
 
 import helfem_amd as H
 import oracle as O
+from helfem_amd._lib import check, lib
 from helfem_amd.synthetic import random_symmetric
 
 pytestmark = pytest.mark.gpu
@@ -21,6 +22,18 @@ TOL = 1e-12
 
 def relerr(a, b):
     return float(np.max(np.abs(a - b)) / max(np.max(np.abs(b)), 1e-300))
+
+
+def launched(ctx, run):
+    """The result and the in-element kernels that made it."""
+    check(lib().hf_ctx_set_timing(ctx.handle, 1))
+    K = run().cpu().numpy()
+    v, ran = np.zeros(3), {}
+    for name in ("k_dia_kin_fold", "k_dia_kin_lds", "k_dia_kin_op", "k_dia_kin_gemm", "k_dia_k_in"):
+        check(lib().hf_ctx_kernel_stats(ctx.handle, name.encode(), v.ctypes.data))
+        ran[name] = int(v[0])
+    check(lib().hf_ctx_set_timing(ctx.handle, 0))
+    return K, ran
 
 
 @pytest.mark.parametrize("nodes", [2, 3, 4, 6, 9, 12, 16])
@@ -126,3 +139,34 @@ def test_sums_no_further_off(nel, gpu_ctx, monkeypatch):
     ratio = np.array(e)[:, 0] / np.array(e)[:, 1]
     print("folded / Cholesky form error", ratio, flush=True)
     assert np.exp(np.mean(np.log(ratio))) <= 1.0
+
+
+def test_operators_of_one_precision_only(gpu_ctx, monkeypatch):
+    """A budget that holds the FP32 operators and not the FP64 ones: FP64 takes the
+    Cholesky form, FP32 the folded one, in turn on one handle and over two screening
+    patterns; with no room at all both take the Cholesky form."""
+    import torch
+    print("[gpu] folded operators under a memory budget", flush=True)
+    n, nel = 9, 3
+    s, a = n * (n + 1) // 2, n * (n - 1) // 2
+    per = sum((p + 15) // 16 * 16 * ((2 * p + n * n + 15) // 16 * 16) for p in (s, a))
+    ob = O.DiatomicBasis(3, 1, 3.0, [3, 2], nel, nnodes=n)
+    ob.compute_tei()
+    hb, none = (H.DiatomicBasis(3, 1, 3.0, [3, 2], nel, nnodes=n, ctx=gpu_ctx) for _ in range(2))
+    sizes = np.zeros(7, dtype=np.int64)
+    check(lib().hf_diatomic_sizes(hb._h, sizes.ctypes.data))
+    gib = 6.0 * per * nel * int(sizes[5]) / 2.0 ** 30  # bytes between four and eight per entry
+    for b in (hb, none):
+        b.compute_tei()
+    S = random_symmetric(ob.Nbf, seed=2110)
+    sh = np.asarray(hb.pure_idx) // hb.Nrad
+    D = np.where((sh[:, None] == 0) | (sh[None, :] == 0), 0.0, S)
+    for P in (S, D, S):
+        Kr = ob.exchange(P)
+        Pd = torch.as_tensor(P, device="cuda")
+        for b, env, forms in ((hb, gib, ("k_dia_kin_lds", "k_dia_kin_fold")), (none, 0.0, ("k_dia_kin_lds",) * 2)):
+            monkeypatch.setenv("HFGPU_EXCHANGE_FOLD_GIB", repr(env))
+            for prec, form, tol in (("fp64", forms[0], TOL), ("fp32", forms[1], 2e-6), ("fp64", forms[0], TOL)):
+                K, ran = launched(gpu_ctx, lambda: b.exchange(Pd, precision=prec))
+                assert ran[form] == 1 and sum(ran.values()) == 1
+                assert relerr(K, Kr) <= tol
