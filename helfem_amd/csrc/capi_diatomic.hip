@@ -1082,6 +1082,13 @@ void ensure_ready(hf_diatomic *h) {
   if (!h->uploaded) diatomic_upload(h);
 }
 
+// whether the folded operators keep FP32's accuracy on this basis
+bool fold_fp32(const DiatomicSetup &S) {
+  for (int e = 0; e < S.Nel(); ++e)
+    if (S.rad.ni[e] < KF_MIN_N32 || S.rad.bval[e + 1] - S.rad.bval[e] > KF_MAX_MU32) return false;
+  return true;
+}
+
 void exchange_launch(hf_diatomic *h, const double *P, int64_t ldp, double *K, int64_t ldk, bool fp32 = false) {
   DiatomicDevice &d = h->dev;
   hipStream_t s = h->ctx->cur;
@@ -1091,7 +1098,7 @@ void exchange_launch(hf_diatomic *h, const double *P, int64_t ldp, double *K, in
     diatomic_op_build(d, h->host.rad.ni, s);
     d.op_ready = true;
   }
-  d.fold_in = diatomic_fold_ready(d, fp32, !d.dense_in, s);
+  d.fold_in = diatomic_fold_ready(d, fp32, !d.dense_in && (!fp32 || fold_fp32(h->host)), s);
   block_stats_launch(P, ldp, d.Nrad, d.Nang, d.skip.p, d.poff.p, d.stats.p, d.h_stats.p, s);
   hip_check(hipStreamSynchronize(s), "block statistics sync");
   const bool symmetric = block_stats_reduce(d.h_stats.p, d.Nrad, d.Nang, d.h_bnorm.p);

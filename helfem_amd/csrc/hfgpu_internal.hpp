@@ -52,6 +52,15 @@ static_assert(KF_COLS == 32, "two 16-column tiles");
 constexpr int kf_pairs(int n, bool anti) { return anti ? n * (n - 1) / 2 : n * (n + 1) / 2; }
 constexpr int kf_inner(int n, bool anti) { return (2 * kf_pairs(n, anti) + n * n + 15) / 16 * 16; }
 constexpr int kf_tiles(int n, bool anti) { return (kf_pairs(n, anti) + 15) / 16; }
+// FP32 takes the folded operators where its error is then no larger than the
+// Cholesky form's: elements of at least KF_MIN_N32 functions (sums long enough for
+// their FP64 parts to tell) and at most KF_MAX_MU32 long in mu (beyond, the
+// operators' entries cancel, which the factors' products do not).  Error ratio,
+// geometric mean of 8 smooth densities, over bases of l <= 4 .. 10, |m| <= 2, R = 1
+// .. 6: 5 functions 0.93 .. 1.72; 8 and 15 functions 0.37 .. 0.99 up to mu 2.52, 1.36
+// and 1.38 at 2.75, 0.99 .. 2.0 from 3.06 on.
+constexpr int KF_MIN_N32 = 7;
+constexpr double KF_MAX_MU32 = 2.6;
 constexpr size_t kf_size(int n) {
   return (size_t)16 * kf_tiles(n, false) * kf_inner(n, false) + (size_t)16 * kf_tiles(n, true) * kf_inner(n, true);
 }
@@ -583,7 +592,8 @@ void diatomic_op_build(DiatomicDevice &d, const std::vector<int> &ni, hipStream_
 // true when the folded operators of this precision are on the device; its first
 // call builds them from the Cholesky tiles.  False, and the Cholesky form runs,
 // where they exceed the budget (HFGPU_EXCHANGE_FOLD_GIB, default a quarter of the
-// free memory), their allocation fails, or allowed is false.
+// free memory), their allocation fails, or allowed is false (dense-operator mode;
+// FP32 outside KF_MIN_N32 and KF_MAX_MU32).
 bool diatomic_fold_ready(DiatomicDevice &d, bool fp32, bool allowed, hipStream_t s);
 constexpr int OP_RUNS = 16;  // runs per k_dia_kin_op workgroup
 

@@ -1,7 +1,8 @@
 """The in-element diatomic exchange with folded operators at every shape of its
 tiles: element sizes from one function to a full 16 x 16 tile (row tiles, inner
 extents and their splits over the waves all follow the size), units with one
-and two rows, and the forms it stands in for.
+and two rows, and the forms it stands in for.  FP32 takes it on elements of at
+least 7 functions and at most 2.6 long in mu.
 
 Bar: FP64 1e-12 of max|K| against the oracle (src/diatomic/basis.cpp:1818-2089),
 as the other parity tests; FP32 1.25 times the Cholesky-form kernel's error on
@@ -58,6 +59,9 @@ def test_element_sizes(nodes, gpu_ctx, monkeypatch):
         e32 = {f: relerr(x.exchange(Pd, precision="fp32").cpu().numpy(), Kr) for f, x in b.items()}
         print(e64, e32, flush=True)
         assert e64["fold"] <= TOL and e64["0"] <= TOL
+        ran = {f: launched(gpu_ctx, lambda: x.exchange(Pd))[1] for f, x in b.items()}
+        # 16 functions: a rank beyond the LDS of k_dia_kin_lds
+        assert ran["fold"]["k_dia_kin_fold"] == 1 and ran["0"]["k_dia_kin_lds"] + ran["0"]["k_dia_k_in"] == 1
         assert e32["fold"] <= max(1.25 * e32["0"], 4 * 2.0 ** -24)
 
 
@@ -170,3 +174,25 @@ def test_operators_of_one_precision_only(gpu_ctx, monkeypatch):
                 K, ran = launched(gpu_ctx, lambda: b.exchange(Pd, precision=prec))
                 assert ran[form] == 1 and sum(ran.values()) == 1
                 assert relerr(K, Kr) <= tol
+
+
+@pytest.mark.parametrize("lmm,nel,nodes,R,form", [
+    ([3, 2, 2], 3, 5, 6.0, "k_dia_kin_lds"),   # few functions: 1.7 times the Cholesky form's error when folded
+    ([3, 2, 2], 3, 7, 6.0, "k_dia_kin_lds"),   # the last element has 6
+    ([3, 2, 2], 3, 8, 6.0, "k_dia_kin_fold"),
+    ([4], 1, 8, 1.0, "k_dia_kin_lds"),         # one element of mu 0 .. 5.1: 2.0 times
+    ([4], 3, 15, 1.0, "k_dia_kin_lds"),        # longest element 2.75: 1.4 times
+    ([6, 6], 3, 15, 2.0, "k_dia_kin_fold"),    # 2.31
+])
+def test_fp32_form_by_basis(lmm, nel, nodes, R, form, gpu_ctx):
+    import torch
+    print(f"[gpu] FP32 in-element form {lmm} {nel} {nodes} R {R}", flush=True)
+    hb = H.DiatomicBasis(7, 7, R, lmm, nel, nnodes=nodes, ctx=gpu_ctx)
+    hb.compute_tei()
+    Pd = torch.as_tensor(random_symmetric(hb.Nbf, seed=2111), device="cuda")
+    K64, r64 = launched(gpu_ctx, lambda: hb.exchange(Pd))
+    K32, r32 = launched(gpu_ctx, lambda: hb.exchange(Pd, precision="fp32"))
+    assert r64["k_dia_kin_fold"] == 1 and r32[form] == 1 and sum(r32.values()) == 1
+    assert relerr(K32, K64) <= 2e-6
+    K64b, _ = launched(gpu_ctx, lambda: hb.exchange(Pd))  # the lists serve both forms
+    assert relerr(K64b, K64) <= TOL
