@@ -1110,31 +1110,39 @@ void atomic_coulomb_launch(const AtomicDevice &d, const double *P, int64_t ldp, 
   }
 }
 
-// Classes, units and entries of k_atomic_kc_off for the density blocks of
-// `mask`; src is reordered so that a class' blocks are consecutive tiles.
-// Leaves d.kc off where its tiles are not used or hold infinities (rows of a
-// wave share sums, and padded sources reread a tile with zero weight).
-static void build_classes(AtomicDevice &d, const std::vector<unsigned char> &mask, int64_t n_runs,
-                          std::vector<int> &src, hipStream_t s) {
-  const int Na = d.Nang, nL = d.N_L;
-  const std::vector<int> &lv = d.h_lv, &mv = d.h_mv;
-  d.kc = false;
-  d.n_wg_kc = 0;
-  // class of a block: m_i - m_l, parities; then row shell by m, l; column shell by l
-  typedef std::array<int, 3> Cls;
-  auto cls = [&](int il) { return Cls{mv[il / Na] - mv[il % Na], lv[il / Na] & 1, lv[il % Na] & 1}; };
-  src.clear();
-  for (int il = 0; il < Na * Na; ++il)
+// Class of a density block: m_i - m_l, parities.
+typedef std::array<int, 3> Cls;
+static Cls block_class(const AtomicDevice &d, int il) {
+  const int i = il / d.Nang, l = il % d.Nang;
+  return Cls{d.h_mv[i] - d.h_mv[l], d.h_lv[i] & 1, d.h_lv[l] & 1};
+}
+
+// The density blocks of `mask` by class, then row shell by m, l, then column shell
+// by l: a class' blocks are consecutive tiles.
+static std::vector<int> class_order(const AtomicDevice &d, const std::vector<unsigned char> &mask) {
+  std::vector<int> src;
+  for (int il = 0; il < d.Nang * d.Nang; ++il)
     if (mask[il]) src.push_back(il);
   auto key = [&](int il) {
-    const int i = il / Na, l = il % Na;
-    const Cls x = cls(il);
-    return std::array<int, 7>{x[0], x[1], x[2], mv[i], lv[i], i, lv[l]};
+    const int i = il / d.Nang, l = il % d.Nang;
+    const Cls x = block_class(d, il);
+    return std::array<int, 7>{x[0], x[1], x[2], d.h_mv[i], d.h_lv[i], i, d.h_lv[l]};
   };
   std::sort(src.begin(), src.end(), [&](int a, int b) { return key(a) < key(b); });
+  return src;
+}
+
+// Classes, units and entries of k_atomic_kc_off for the density blocks src (in
+// class_order).  Leaves d.kc off where its tiles are not used or hold infinities
+// (rows of a wave share sums, and padded sources reread a tile with zero weight).
+static void build_classes(AtomicDevice &d, const std::vector<int> &src, hipStream_t s) {
+  const int Na = d.Nang, nL = d.N_L;
+  const std::vector<int> &lv = d.h_lv, &mv = d.h_mv;
+  d.kc_tried = true;
+  auto cls = [&](int il) { return block_class(d, il); };
   if (!d.tiled || !d.finite || d.Nel < 2 || src.empty()) return;
   const char *env = std::getenv("HFGPU_EXCHANGE_CLASSES");
-  if (env ? std::atoi(env) == 0 : (double)d.n_terms < KC_MIN_TERMS * (double)n_runs) return;
+  if (env ? std::atoi(env) == 0 : (double)d.n_terms < KC_MIN_TERMS * (double)d.n_lruns) return;
   // stages of every class, cut between row shells; a row shell holds at most
   // one m_l, so a stage always fits one (at most 129 shells of one m would not)
   struct Stage {
@@ -1313,7 +1321,8 @@ static void build_classes(AtomicDevice &d, const std::vector<unsigned char> &mas
 // Compact the static coupling lists to the density blocks that pass the
 // norm screen (|P_il|_F >= 10 eps, TwoDBasis.cpp:949-952).  The result only
 // changes when the screening pattern does, so it is cached by pattern.
-static void compact_exchange_lists(AtomicDevice &d, hipStream_t s) {
+// classes: with the lists of k_atomic_kc_off, which batched launches do not read.
+static void compact_exchange_lists(AtomicDevice &d, bool classes, hipStream_t s) {
   const int Na = d.Nang, nL = d.N_L;
   std::vector<unsigned char> mask((size_t)Na * Na);
   const double thr = 10.0 * 2.220446049250313e-16;
@@ -1327,15 +1336,24 @@ static void compact_exchange_lists(AtomicDevice &d, hipStream_t s) {
       }
   bool finite = true;
   for (size_t q = 0; q < mask.size(); ++q) finite = finite && d.h_bnorm.p[q] < 1e30;
-  if (mask == d.screen_mask && !d.screen_mask.empty() && d.sym == d.list_sym && finite == d.finite) return;
+  if (mask == d.screen_mask && !d.screen_mask.empty() && d.sym == d.list_sym && finite == d.finite) {
+    if (classes && !d.kc_tried) {
+      build_classes(d, class_order(d, mask), s);
+      if (d.kc) ++d.list_gen;  // weights that have no FP32 copy yet
+    }
+    return;
+  }
   d.finite = finite;
+  d.kc = d.kc_tried = false;
+  d.n_wg_kc = 0;
   d.screen_mask.clear();  // no lists until all of them are there
   std::vector<int> act, tstart(1, 0), til;
   std::vector<double> tc;
   // flops as executed: in the symmetric mode the cross-element launch covers
   // the pairs e > f and the in-element one the blocks j <= k
   double frad_off = 0.0, frad_in = 0.0;
-  int64_t nterm_in = 0, n_runs = 0;  // (block, L) with any term
+  int64_t nterm_in = 0;
+  d.n_lruns = 0;
   for (size_t a = 0; a < d.h_act.size(); ++a) {
     const size_t n0 = til.size();
     const bool in_done = !d.sym || d.h_act[a] / Na <= d.h_act[a] % Na;
@@ -1349,7 +1367,7 @@ static void compact_exchange_lists(AtomicDevice &d, hipStream_t s) {
           tc.push_back(d.h_tc[q]);
         }
       if (til.size() > before) {
-        ++n_runs;
+        ++d.n_lruns;
         frad_off += d.sym ? d.h_radL_low[L] : d.h_radL[L] - d.h_radL_in[L];
         if (in_done) frad_in += d.h_radL_in[L];
       }
@@ -1433,28 +1451,21 @@ static void compact_exchange_lists(AtomicDevice &d, hipStream_t s) {
   d.act_jk.upload(act, s);
   d.term_start.upload(tstart, s);
   d.term_il.upload(til, s);
-  {
-    std::vector<int2> toff(til.size());
-    for (size_t q = 0; q < til.size(); ++q)
-      toff[q] = make_int2((til[q] / d.Nang) * d.Nrad, (til[q] % d.Nang) * d.Nrad);
-    d.term_off.upload(toff, s);
-  }
-  {
-    // source blocks, and each term's tile among them
-    std::vector<int> id((size_t)Na * Na, -1), src, tt(til.size());
-    size_t n_mask = 0;
-    for (unsigned char m : mask) n_mask += m;
-    const double bytes = (double)n_mask * d.Nel * d.Nel * TILE2 * sizeof(double);
-    d.tiled = bytes <= exchange_tile_budget(d.ptile.n * sizeof(double) + d.ptile32.n * sizeof(float));
-    build_classes(d, mask, n_runs, src, s);
-    for (size_t q = 0; q < src.size(); ++q) id[src[q]] = (int)q;
-    for (size_t q = 0; q < til.size(); ++q) tt[q] = std::max(id[til[q]], 0);
-    d.n_src = (int)src.size();
-    if (src.empty()) src.push_back(0);
-    d.src_blk.upload(src, s);
-    d.term_tile.upload(tt, s);
-    hip_check(hipStreamSynchronize(s), "exchange source upload");
-  }
+  std::vector<int2> toff(til.size());
+  for (size_t q = 0; q < til.size(); ++q)
+    toff[q] = make_int2((til[q] / d.Nang) * d.Nrad, (til[q] % d.Nang) * d.Nrad);
+  d.term_off.upload(toff, s);
+  // source blocks, and each term's tile among them
+  std::vector<int> id((size_t)Na * Na, -1), src = class_order(d, mask), tt(til.size());
+  const double bytes = (double)src.size() * d.Nel * d.Nel * TILE2 * sizeof(double);
+  d.tiled = bytes <= exchange_tile_budget(d.ptile.n * sizeof(double) + d.ptile32.n * sizeof(float));
+  if (classes) build_classes(d, src, s);
+  for (size_t q = 0; q < src.size(); ++q) id[src[q]] = (int)q;
+  for (size_t q = 0; q < til.size(); ++q) tt[q] = std::max(id[til[q]], 0);
+  d.n_src = (int)src.size();
+  if (src.empty()) src.push_back(0);
+  d.src_blk.upload(src, s);
+  d.term_tile.upload(tt, s);
   d.term_c.upload(tc, s);
   hip_check(hipStreamSynchronize(s), "exchange list upload");
   d.screen_mask = mask;
@@ -1475,7 +1486,7 @@ static bool exchange_prologue(AtomicDevice &d, const double *P, int64_t ldp, dou
   hip_check(hipStreamSynchronize(s), "block statistics sync");
   const bool symmetric = block_stats_reduce(d.h_stats.p, d.Nrad, d.Nang, d.h_bnorm.p);
   d.sym = allow_sym && !d.dense_in && symmetric_exchange_allowed() && symmetric;
-  compact_exchange_lists(d, s);
+  compact_exchange_lists(d, true, s);
   fill_zero_launch(K, nbf, nbf, ldk, s);
   return d.n_act > 0;
 }
@@ -1917,7 +1928,7 @@ void atomic_batch_exchange(AtomicBatch &b, const double *const *P, const int64_t
     if (d.h_act.empty()) continue;
     const bool symmetric = block_stats_reduce(b.h_stats.p + b.stats_off[i], d.Nrad, d.Nang, d.h_bnorm.p);
     d.sym = !d.dense_in && symmetric_exchange_allowed() && symmetric;
-    compact_exchange_lists(d, s);
+    compact_exchange_lists(d, false, s);
     if (fp32[i] && d.n_act > 0) prepare_f32(d, P[i], ldp[i], s);
     if (d.tiled && d.n_act > 0) {
       const size_t nt = (size_t)d.Nel * d.Nel * d.n_src * TILE2;

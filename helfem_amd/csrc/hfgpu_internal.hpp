@@ -272,6 +272,8 @@ struct AtomicDevice {
   // blocks (L, entries); per entry up to KC_SRC consecutive tiles of one row
   // shell i with their weights g(k,L,l), and the rows' 4pi/(2L+1) g(j,L,i).
   bool kc = false, finite = true;         // finite: no infinite or NaN block norm
+  bool kc_tried = false;                  // build_classes has seen the current lists (batches never ask)
+  int64_t n_lruns = 0;                    // (block, L) with any term in the current lists
   int n_wg_kc = 0;                        // workgroups per element pair
   int kc_rows = 0, kc_tiles = 0, kc_parts = 0;         // most rows of a unit, tiles of a stage, partial row tiles of a workgroup
   std::vector<int> h_lv, h_mv;

@@ -10,6 +10,7 @@ import pytest
 
 import helfem_amd as H
 import oracle as O
+from helfem_amd._lib import check, lib
 from helfem_amd.synthetic import random_symmetric
 
 pytestmark = pytest.mark.gpu
@@ -18,6 +19,18 @@ TOL = 1e-12
 
 def relerr(a, b):
     return float(np.max(np.abs(a - b)) / max(np.max(np.abs(b)), 1e-300))
+
+
+def launched(ctx, run):
+    """The result and how often the class and the block kernel made it."""
+    check(lib().hf_ctx_set_timing(ctx.handle, 1))
+    K = run()
+    v, ran = np.zeros(3), []
+    for name in ("k_atomic_kc_off", "k_atomic_k_off"):
+        check(lib().hf_ctx_kernel_stats(ctx.handle, name.encode(), v.ctypes.data))
+        ran.append(int(v[0]))
+    check(lib().hf_ctx_set_timing(ctx.handle, 0))
+    return K, tuple(ran)
 
 
 def _bases(monkeypatch, ctx, args, kw):
@@ -47,10 +60,14 @@ def test_against_oracle(lmax, mmax, nel, nodes, gpu_ctx, monkeypatch):
     for P in (S, G, D):
         Kr = ob.exchange(P)
         monkeypatch.setenv("HFGPU_EXCHANGE_CLASSES", "1")
-        assert relerr(K(on, P), Kr) <= TOL
-        e1 = relerr(K(on, P, precision="fp32"), Kr)
+        K1, ran = launched(gpu_ctx, lambda: K(on, P))
+        assert relerr(K1, Kr) <= TOL and ran == (1, 0)
+        K1, ran = launched(gpu_ctx, lambda: K(on, P, precision="fp32"))
+        assert ran == (1, 0)
+        e1 = relerr(K1, Kr)
         monkeypatch.setenv("HFGPU_EXCHANGE_CLASSES", "0")
-        assert relerr(K(off, P), Kr) <= TOL
+        K0, ran = launched(gpu_ctx, lambda: K(off, P))
+        assert relerr(K0, Kr) <= TOL and ran == (0, 1)
         e0 = relerr(K(off, P, precision="fp32"), Kr)
         print(f"fp32 error {e1:.2e}, other kernel {e0:.2e}", flush=True)
         assert e1 <= max(1.25 * e0, 4 * 2.0 ** -24)
@@ -65,9 +82,35 @@ def test_several_stages(gpu_ctx, monkeypatch):
     m = np.repeat(on.mval, on.Nrad)
     P[m[:, None] != m[None, :]] = 0.0
     monkeypatch.setenv("HFGPU_EXCHANGE_CLASSES", "1")
-    K1 = K(on, P)
+    K1, ran = launched(gpu_ctx, lambda: K(on, P))
+    assert ran == (1, 0)
     monkeypatch.setenv("HFGPU_EXCHANGE_CLASSES", "0")
-    assert relerr(K1, K(off, P)) <= TOL
+    K0, ran = launched(gpu_ctx, lambda: K(off, P))
+    assert ran == (0, 1)
+    assert relerr(K1, K0) <= TOL
+
+
+def test_batches_and_single_builds_in_turn(gpu_ctx, monkeypatch):
+    """Batched launches do not read the class lists and do not build them: a single
+    build of the same handle, pattern and precision does, before and after a batch."""
+    import torch
+    print("[gpu] class exchange between batched builds", flush=True)
+    (on, off), K = _bases(monkeypatch, gpu_ctx, (10, 3, 2, 3), dict(nnodes=8))
+    P = random_symmetric(on.Nbf, seed=2206)
+    sh = np.arange(on.Nbf) // on.Nrad
+    D = np.where((sh[:, None] == 1) | (sh[None, :] == 1), 0.0, P)
+    monkeypatch.setenv("HFGPU_EXCHANGE_CLASSES", "0")
+    ref = {k: (K(off, X), K(off, X, precision="fp32")) for k, X in (("P", P), ("D", D))}
+    monkeypatch.setenv("HFGPU_EXCHANGE_CLASSES", "1")
+    bt = H.AtomicBatch([on], gpu_ctx)
+    for k, X in (("P", P), ("D", D), ("P", P)):
+        Xd = torch.as_tensor(X, device="cuda")
+        for prec, r, tol in (("fp32", ref[k][1], 2e-6), ("fp64", ref[k][0], TOL)):
+            out = torch.empty_like(Xd)
+            _, ran = launched(gpu_ctx, lambda: bt.exchange([Xd], [out], fp32=[prec == "fp32"]))
+            assert ran == (0, 0) and relerr(out.cpu().numpy(), r) <= tol  # its own kernels
+            K1, ran = launched(gpu_ctx, lambda: K(on, X, precision=prec))
+            assert ran == (1, 0) and relerr(K1, r) <= tol
 
 
 def test_yukawa_and_infinite_density(gpu_ctx, monkeypatch):
