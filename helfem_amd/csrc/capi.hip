@@ -267,6 +267,7 @@ void atomic_upload(hf_atomic *h) {
   d.jbg.alloc((size_t)std::max(nlm, 1) * Nel);
 
   hip_check(hipStreamSynchronize(s), "upload sync");
+  d.f32_tables = false;
   atomic_build_operator(S, d, s);
   h->uploaded = true;
 }

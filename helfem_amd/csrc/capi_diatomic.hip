@@ -319,7 +319,7 @@ void diatomic_upload(hf_diatomic *h) {
   d.db.alloc((size_t)std::max(nLM, 1) * Nel);
   hip_check(hipStreamSynchronize(s), "upload sync");
   diatomic_build_operator(S, d, s);
-  d.op_ready = false;
+  d.op_ready = d.f32_tables = false;
   h->uploaded = true;
 }
 

@@ -16,7 +16,7 @@ import pytest
 
 import helfem_amd as H
 import oracle as O
-from helfem_amd.synthetic import seeded_density
+from helfem_amd.synthetic import random_symmetric, seeded_density
 
 pytestmark = pytest.mark.gpu
 TOL32 = 2e-6
@@ -161,3 +161,22 @@ def test_mixed_scf_uses_split_builds(gpu_ctx):
     rmx = rhf(hb, 10, conv=1e-11, precision="mixed")
     assert rmx.iterations_fp32 > 0 and rmx.iterations_incremental > 0
     assert abs(rmx.E - r64.E) < 1e-10, (rmx.E, r64.E)
+
+
+def test_fp32_tables_follow_the_caches(gpu_ctx):
+    """New caches on a handle whose FP32 exchange has run: the FP32 tables are the
+    new ones."""
+    import torch
+    print("[gpu] FP32 exchange after new caches", flush=True)
+    hb = H.AtomicBasis(10, 1, 1, 3, nnodes=8, ctx=gpu_ctx)
+    hb.compute_tei()
+    Pd = torch.as_tensor(random_symmetric(hb.Nbf, seed=3301), device="cuda")
+    first = hb.exchange(Pd, precision="fp32").cpu().numpy()
+    keys = [(kind, L, e) for kind in range(3) for L in range(3) for e in range(3)]
+    for key, m in [(key, hb.get_cache(*key)) for key in keys]:
+        if m.size:
+            hb.set_cache(*key, 1.5 * m)
+    hb.commit_tei()
+    K64 = hb.exchange(Pd).cpu().numpy()
+    assert relerr(first, K64) > 0.1
+    assert relerr(hb.exchange(Pd, precision="fp32").cpu().numpy(), K64) <= TOL32
