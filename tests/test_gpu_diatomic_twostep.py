@@ -13,6 +13,7 @@ import pytest
 
 import helfem_amd as H
 import oracle as O
+from helfem_amd._lib import check, lib
 from helfem_amd.synthetic import random_symmetric
 
 pytestmark = pytest.mark.gpu
@@ -29,6 +30,18 @@ CASES = {
 
 def relerr(a, b):
     return float(np.max(np.abs(a - b)) / max(np.max(np.abs(b)), 1e-300))
+
+
+def launched(ctx, run):
+    """The result and how often the two-step and the one-step kernel made it."""
+    check(lib().hf_ctx_set_timing(ctx.handle, 1))
+    K = run().cpu().numpy()
+    v, ran = np.zeros(3), []
+    for name in ("k_dia_k2_off", "k_dia_k_off"):
+        check(lib().hf_ctx_kernel_stats(ctx.handle, name.encode(), v.ctypes.data))
+        ran.append(int(v[0]))
+    check(lib().hf_ctx_set_timing(ctx.handle, 0))
+    return K, tuple(ran)
 
 
 @pytest.mark.parametrize("name", list(CASES))
@@ -54,10 +67,17 @@ def test_lists_at_their_edges(name, gpu_ctx, monkeypatch):
     for P in (S, G, D):
         Kr = ob.exchange(P)
         Pd = torch.as_tensor(P, device="cuda")
-        assert relerr(hb.exchange(Pd).cpu().numpy(), Kr) <= TOL
-        e32 = relerr(hb.exchange(Pd, precision="fp32").cpu().numpy(), Kr)
+        K, ran = launched(gpu_ctx, lambda: hb.exchange(Pd))
+        assert relerr(K, Kr) <= TOL
+        K32, ran32 = launched(gpu_ctx, lambda: hb.exchange(Pd, precision="fp32"))
+        if np.any(Kr):  # else no block is coupled
+            assert ran == (1, 0) and ran32 == (1, 0)
+        e32 = relerr(K32, Kr)
         monkeypatch.setenv("HFGPU_EXCHANGE_TWOSTEP", "0")
-        o32 = relerr(one.exchange(Pd, precision="fp32").cpu().numpy(), Kr)
+        K32, ran32 = launched(gpu_ctx, lambda: one.exchange(Pd, precision="fp32"))
+        if np.any(Kr):
+            assert ran32 == (0, 1)
+        o32 = relerr(K32, Kr)
         monkeypatch.delenv("HFGPU_EXCHANGE_TWOSTEP")
         print(f"fp32 error {e32:.2e}, one-step {o32:.2e}", flush=True)
         assert e32 <= 1.25 * o32
@@ -76,7 +96,12 @@ def test_more_rows_and_slots_than_fit(gpu_ctx, monkeypatch):
         hb.compute_tei()
         S = random_symmetric(hb.Nbf, seed=2005)
         G = S + 0.3 * np.triu(random_symmetric(hb.Nbf, seed=2006))
-        K.append([hb.exchange(torch.as_tensor(P, device="cuda")).cpu().numpy() for P in (S, G)])
+        K.append([])
+        for P in (S, G):
+            Pd = torch.as_tensor(P, device="cuda")
+            X, ran = launched(gpu_ctx, lambda: hb.exchange(Pd))
+            assert ran == ((1, 0) if two == "1" else (0, 1))
+            K[-1].append(X)
     for a, b in zip(*K):
         assert relerr(a, b) <= TOL
 
@@ -95,7 +120,9 @@ def test_infinite_density_stays_in_its_blocks(gpu_ctx, monkeypatch):
         P[3, 5] = P[5, 3] = np.inf
         Pd = torch.as_tensor(P, device="cuda")
         hb.exchange(torch.as_tensor(random_symmetric(hb.Nbf, seed=2004), device="cuda"))
-        K.append(hb.exchange(Pd).cpu().numpy())
+        X, ran = launched(gpu_ctx, lambda: hb.exchange(Pd))
+        assert ran == (0, 1)  # not finite: one step either way
+        K.append(X)
     assert np.array_equal(np.isfinite(K[0]), np.isfinite(K[1]))
     ok = np.isfinite(K[0])
     assert relerr(K[0][ok], K[1][ok]) <= TOL
