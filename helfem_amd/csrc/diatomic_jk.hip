@@ -1112,13 +1112,15 @@ __device__ inline void slot_sums(const T *pt, int4 r, const int4 *more, const T 
 
 // One half (symmetric or antisymmetric) of the GEMM: the wave's row tile rt
 // over the quads [q0, q1) and both column tiles.  Every quad's 16 products are a
-// sum of their own, added in FP64.  One chain over up to 480 products, whose two
-// channels cancel, was further off than the Cholesky form: R = 6, l <= 3, 6
-// elements of 15 functions, FP32 1.6 times its error (now 0.56), FP64 against 64-bit
-// sums 1.9e-15 (now 1.65e-15, Cholesky form 1.7e-15).  N2 10.59 -> 10.73 ms, FP32
-// (lmax 12, 6 elements) 2.08 -> 2.15 ms.
+// sum of their own.  One chain of matrix instructions over up to 480 products, whose
+// two channels cancel, was further off than the Cholesky form: R = 6, l <= 3, 6
+// elements of 15 functions, FP32 1.6 times its error (now 0.69), FP64 against 64-bit
+// sums 1.9e-15 (now 1.65e-15, Cholesky form 1.7e-15).  N2 10.58 -> 10.74 ms, FP32
+// (lmax 12, 6 elements) 2.08 -> 2.11 ms; the FP32 parts added in FP64 0.56 times, but
+// 2.15 ms.
 template <typename T>
-__device__ inline void fold_gemm(const T *top, const T *X, int rt, int nq, int q0, int q1, int lane, v4d sum[2]) {
+__device__ inline void fold_gemm(const T *top, const T *X, int rt, int nq, int q0, int q1, int lane,
+                                 typename Mma<T>::acc_t sum[2]) {
   typedef Mma<T> MM;
   typedef typename MM::acc_t vec;
   const int g = lane >> 4, c = lane & 15;
@@ -1137,9 +1139,7 @@ __device__ inline void fold_gemm(const T *top, const T *X, int rt, int nq, int q
       acc[1] = MM::step(cur[st], b1, acc[1]);
     }
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct)
-#pragma unroll
-      for (int s = 0; s < 4; ++s) sum[ct][s] += (double)acc[ct][s];
+    for (int ct = 0; ct < 2; ++ct) sum[ct] += acc[ct];
     cur = nxt;
   }
 }
@@ -1239,7 +1239,7 @@ __global__ void __launch_bounds__(KF_THREADS) k_dia_kin_fold(DFoldArgs<T> A) {
       X[(q & 1) * nq * 256 + (k0 + (q >> 5)) * 16 + ((q >> 1) & 15)] = T(0);
   };
   const T *top = A.Top + (size_t)(ilm * A.Nel + e) * A.size;
-  v4d aS[2] = {v4d{0, 0, 0, 0}, v4d{0, 0, 0, 0}}, aA[2] = {v4d{0, 0, 0, 0}, v4d{0, 0, 0, 0}};
+  vec aS[2] = {vec{0, 0, 0, 0}, vec{0, 0, 0, 0}}, aA[2] = {vec{0, 0, 0, 0}, vec{0, 0, 0, 0}};
   // waves: row tile, and a share of the inner extent
   const int kS = KF_WAVES / rS, kA = rA > 0 ? KF_WAVES / rA : 1;
   columns(false);
@@ -1256,13 +1256,13 @@ __global__ void __launch_bounds__(KF_THREADS) k_dia_kin_fold(DFoldArgs<T> A) {
   // blocks' entries: Y(a,b) = Y_s + Y_a, Y(b,a) = Y_s - Y_a, scaled back
   const double scale = A.scale[ilm * A.Nel + e];
   T *Ys = X, *Ya = X + kS * rS * 512;
-  auto partial = [&](T *Y, int h, int rt, int nr, const v4d acc[2]) {
+  auto partial = [&](T *Y, int h, int rt, int nr, const vec acc[2]) {
 #pragma unroll
     for (int ct = 0; ct < 2; ++ct)
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const int row = kk[s];
-        Y[((h * nr + rt) * 2 + ct) * 256 + row * 16 + ((c + (row >> 1)) & 15)] = (T)acc[ct][s];
+        Y[((h * nr + rt) * 2 + ct) * 256 + row * 16 + ((c + (row >> 1)) & 15)] = acc[ct][s];
       }
   };
   if (hS < kS) partial(Ys, hS, wv - hS * rS, rS, aS);

@@ -54,11 +54,11 @@ constexpr int kf_inner(int n, bool anti) { return (2 * kf_pairs(n, anti) + n * n
 constexpr int kf_tiles(int n, bool anti) { return (kf_pairs(n, anti) + 15) / 16; }
 // FP32 takes the folded operators where its error is then no larger than the
 // Cholesky form's: elements of at least KF_MIN_N32 functions (sums long enough for
-// their FP64 parts to tell) and at most KF_MAX_MU32 long in mu (beyond, the
-// operators' entries cancel, which the factors' products do not).  Error ratio,
-// geometric mean of 8 smooth densities, over bases of l <= 4 .. 10, |m| <= 2, R = 1
-// .. 6: 5 functions 0.93 .. 1.72; 8 and 15 functions 0.37 .. 0.99 up to mu 2.52, 1.36
-// and 1.38 at 2.75, 0.99 .. 2.0 from 3.06 on.
+// their parts to tell) and at most KF_MAX_MU32 long in mu (beyond, the operators'
+// entries cancel, which the factors' products do not).  Error ratio, geometric mean
+// of 8 smooth densities, over bases of l <= 4 .. 10, |m| <= 2, R = 1 .. 6: 5 functions
+// 0.93 .. 1.72; 8 and 15 functions 0.39 .. 0.99 up to mu 2.52, 1.36 and 1.38 at 2.75,
+// 0.99 .. 2.0 from 3.06 on.
 constexpr int KF_MIN_N32 = 7;
 constexpr double KF_MAX_MU32 = 2.6;
 constexpr size_t kf_size(int n) {

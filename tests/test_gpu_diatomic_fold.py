@@ -113,7 +113,7 @@ def test_sums_no_further_off(nel, gpu_ctx, monkeypatch):
     """Long sums (15 functions, 465 products, channels that cancel): the error of
     the folded FP32 form against FP64, over several smooth densities, is at most the
     Cholesky form's.  Both round the same inputs; a single FP32 chain is 1.6 to 1.9
-    times as far off, sums of 16 added in FP64 half as far."""
+    times as far off, sums of 16 products 0.7 times."""
     import torch
     print(f"[gpu] folded FP32 sums, {nel} elements", flush=True)
     args, kw = (7, 7, 6.0, [3, 2, 2], nel), dict(nnodes=15, ctx=gpu_ctx)
