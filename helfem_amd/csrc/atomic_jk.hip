@@ -13,8 +13,9 @@
 //   only the element-diagonal Ni x Ni bands of each P block enter J, and J
 //   is nonzero only on those bands.  Kernel 1 gathers the Gaunt-weighted
 //   band of every (L,M) into LDS, reduces the two multipole traces and the
-//   Cholesky matvec; kernel 2 prefix-sums the cross-element traces; kernel 3
-//   expands the (L,M) bands back into the angular blocks of J.
+//   Cholesky matvec; kernel 2 adds the other elements' traces times r^L and
+//   r^-L-1, the whole band; kernel 3 expands the (L,M) bands back into the angular
+//   blocks of J.
 // Exchange (TwoDBasis.cpp:880-999 + CoulombExchangeFE.h:484-530):
 //   one workgroup per (output block, element pair (e,f)): the Gaunt-weighted
 //   density sub-block R_L(e,f) is formed in registers for each coupled L and
@@ -474,8 +475,8 @@ void launch_atomic_k(int part, bool tiled, int64_t grid, hipStream_t s, const KA
 // K_jk(e,f) = sum_L A_L [sum_il g(j,L,i) g(k,L,l) P_il(e,f)] B_L', M = m_j - m_i =
 // m_k - m_l.  l_j + L + l_i and l_k + L + l_l are even, so the outputs of one
 // (m_j - m_k, parities) draw on two classes of density blocks, one for even and
-// one for odd L: at most 58 of the 231 blocks of an m-diagonal lmax = 6 density,
-// 116 KB.  One workgroup per (element pair, up to eight units of one output
+// one for odd L: at most 72 of the 231 blocks of an m-diagonal lmax = 6 density,
+// 144 KB.  One workgroup per (element pair, up to eight units of one output
 // class) loads them into LDS, one class after the other; a wave's unit is one
 // column k with up to four rows j of one m and parity, which share the column
 // sums w = sum_l g(k,L,l) P_il; the multipoles of a unit are split over two to
@@ -484,9 +485,13 @@ void launch_atomic_k(int part, bool tiled, int64_t grid, hipStream_t s, const KA
 // adds A R B'.  Eight entries' coefficients come in one vector load (a value per
 // lane, broadcast by readlane): as scalar loads they would share their counter
 // with the LDS reads, and every tile read would wait for them.
-// Bound by the LDS reads and the vector sums between them.  Xe (lmax = mmax = 6,
-// 25 elements): 2.86 ms one block at a time from L2 (k_atomic_k_off_f64), 1.75 ms
-// here (1.87 with one wave per unit, 2.83 with uniform coefficient loads).
+// Bound by the LDS reads and the vector sums between them (27 vector instructions
+// per matrix one, the matrix pipe 9% busy).  Xe (lmax = mmax = 6, 25 elements): 2.86
+// ms one block at a time from L2 (k_atomic_k_off_f64), 1.75 ms here (1.87 with one
+// wave per unit, 2.83 with uniform coefficient loads).
+// FP32 rounds two weights where that kernel rounds their product, and sums over l
+// first: its error is 0.99 times that kernel's (lmax 5 and 6, 10 elements, four
+// densities each: 2.68e-7 against 2.70e-7 to 4.03e-7 against 4.06e-7).
 
 template <typename T>
 struct KCArgs {
@@ -1143,8 +1148,9 @@ static void build_classes(AtomicDevice &d, const std::vector<int> &src, hipStrea
   if (!d.tiled || !d.finite || d.Nel < 2 || src.empty()) return;
   const char *env = std::getenv("HFGPU_EXCHANGE_CLASSES");
   if (env ? std::atoi(env) == 0 : (double)d.n_terms < KC_MIN_TERMS * (double)d.n_lruns) return;
-  // stages of every class, cut between row shells; a row shell holds at most
-  // one m_l, so a stage always fits one (at most 129 shells of one m would not)
+  // stages of every class, cut between row shells: the blocks of one row shell, of
+  // one m_l and parity, must fit a stage (not beyond KC_TILES such shells, about 145
+  // consecutive l)
   struct Stage {
     int first, n;
   };

@@ -1,8 +1,8 @@
 // Allocation-free Coulomb entry point (hf_atomic_coulomb_dev_noalloc).
 //
 // The atomic Coulomb build needs per-call work space beside its inputs and
-// outputs: the Gaunt-weighted in-element bands Jin [n_lm][Nel][256], the two
-// multipole traces per ((L,M), element) and their prefix sums.  The ordinary
+// outputs: the Gaunt-weighted bands Jin [n_lm][Nel][256] and the two
+// multipole traces per ((L,M), element).  The ordinary
 // entry point keeps these in buffers the handle allocates at upload; this one
 // takes them from `scratch`, a file-scope device array every GPU holds from
 // module load to process end, so the call itself allocates nothing (for

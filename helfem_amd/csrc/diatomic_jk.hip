@@ -13,17 +13,16 @@
 // Paux0 = sum mod_coeff * P_kl and Paux2 = sum coeff * P_kl, of which only
 // the element-diagonal bands matter.  Kernel 1 gathers both bands, reduces
 // the P/Q traces and applies the in-element kernel through the Cholesky
-// factor; kernel 2 prefix-sums the cross-element traces; kernel 3 expands
-// the bands into the shell blocks of J.
-// Exchange (basis.cpp:1818-2089): one workgroup per (output block (j,k),
-// element pair (e,f)); for each coupled (L,|M|) the four Gaunt-weighted
+// factor; kernel 2 adds the other elements' traces times P and Q, the whole
+// band; kernel 3 expands the bands into the shell blocks of J.
+// Exchange (basis.cpp:1818-2089), one-step form: one workgroup per (output block
+// (j,k), element pair (e,f)); for each coupled (L,|M|) the four Gaunt-weighted
 // density tiles R00, R02, R20, R22 are formed in registers and contracted on
 // the matrix cores with the disjoint P/Q factors (e != f) or the four-channel
 // Cholesky factor (e == f).  The density tiles are first copied out of P into
 // a tiled array (k_dia_ptile: one contiguous, aligned 2 KB tile per (element
 // pair, density block) in operand order), so a term's gather is one aligned
-// 32-byte read per lane and an element pair's slice (3.3 MB for N2 at lmax
-// 16) stays in the L2 of the XCD that works on it.
+// 32-byte read per lane.
 #include "hfgpu_internal.hpp"
 #include "device_common.hpp"
 #include <algorithm>
@@ -634,7 +633,7 @@ __global__ void __launch_bounds__(NT) k_dia_k_in(DKArgs<T> A) {
 // per slot and wave.  FP32 adds each group's products to the rows in FP64 (in
 // FP32 the sum over all groups lost a quarter of a digit).
 // N2 (lmax 16, 8 elements): 5.1 ms, 9.5 ms with the four channel tiles formed
-// per row; 13.6 ms of matrix time over 1024 SIMDs (23% busy), the rest is
+// per row; the matrix pipe is busy 28% of it (1.4 ms), the rest is
 // latency: tile gathers (2.2 ms of it), list loads and the two barriers per
 // group.  Two 512-thread workgroups per CU (16 waves) measured fastest: 384
 // threads 7.3, 256 threads 6.8, one of 1024 over two element pairs 5.4 ms;
@@ -955,8 +954,8 @@ __global__ void __launch_bounds__(KL_THREADS) k_dia_kin_lds(DKLArgs<T> A) {
 // of bank conflicts.  The tiles are added to K atomically (boundary entries are
 // shared with the cross-element launch, the (L,|M|) of a block with other
 // workgroups).
-// N2 (lmax 16, 8 elements, 60 k rows x 8 elements): 4.0 ms against 13.0 of
-// k_dia_kin_lds, FP32 (lmax 12, 6 elements) 1.0 against 2.1; 1.5 ms of it the
+// N2 (lmax 16, 8 elements, 60 k rows x 8 elements): 4.2 ms against 13.0 of
+// k_dia_kin_lds, FP32 (lmax 12, 6 elements) 1.0 against 2.1; 1.6 ms of it the
 // matrix pipe's, the gathers 0.65, the output 0.55, the folding the rest (one
 // workgroup per CU, its phases one after another).
 
@@ -1322,7 +1321,7 @@ __global__ void __launch_bounds__(KF_THREADS) k_dia_kin_fold(DFoldArgs<T> A) {
 // costs 2 n^4 per channel and run against 12 r n^3 / 4 of the Cholesky form
 // (r ~ 30: 3.4x fewer matrix operations).
 //
-// k_dia_op_build (at upload) writes T in the matrix-core operand order: for
+// k_dia_op_build (before the first exchange) writes T in the matrix-core operand order: for
 // k-step ks (inner indices kappa = 4 ks + g, kappa = ch * 228 + c + 15 d) and
 // row tile rt (rows rho = 16 rt + c, rho = a + 15 b), lane (g, c) holds
 // T(rho, kappa); one aligned 512-byte read per wave and (ks, rt).

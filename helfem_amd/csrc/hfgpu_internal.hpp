@@ -30,9 +30,10 @@ constexpr int K2_SLOTS = 32, K2_THREADS = HFG_K2_THREADS, K2_WAVES = K2_THREADS 
 static_assert(K2_THREADS % 64 == 0 && K2_THREADS <= 1024, "two-step exchange workgroup");
 
 // cross-element atomic exchange by density classes: waves per workgroup, units
-// per workgroup, rows per unit, sources per entry, most tiles in LDS at once
-// (the FP64 tiles then take 144 of 160 KB)
-// used from KC_MIN_TERMS terms per coupled (output block, L) on (lmax = 5: 12),
+// per workgroup, rows per unit, sources per entry, most tiles in LDS at once (144 of
+// 160 KB in FP64: the largest class of an m-diagonal lmax = 6 density in one stage)
+// used from KC_MIN_TERMS terms per coupled (output block, L) on (lmax = 5: 12; a
+// density of blocks l = l' <= 2 alone has 3.8 at any lmax and keeps the other kernel),
 // and KC_MIN_WGS workgroups in the launch; exchange of an m-diagonal density
 // without / with it: lmax 4, 20 elements 770 / 799 us (FP32 691 / 669); lmax 5,
 // 25 elements 2493 / 1943; lmax 6, 10 elements 891 / 758, 4 elements 287 / 304
@@ -357,7 +358,7 @@ struct DiatomicDevice {
   int n_wg_kl = 0;
   // in-element exchange as a dense operator on the matrix cores
   // (k_dia_kin_op): the operators of every (ilm, element) in operand order,
-  // built on the device at upload when they fit the budget; per workgroup
+  // built on the device before the first exchange when they fit the budget; per workgroup
   // (ilm, e, first entry in kl_runs, count <= 16)
   bool op_in = false;
   DevArray<double> Top2;
