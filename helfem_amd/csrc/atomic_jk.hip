@@ -489,9 +489,9 @@ void launch_atomic_k(int part, bool tiled, int64_t grid, hipStream_t s, const KA
 // per matrix one, the matrix pipe 9% busy).  Xe (lmax = mmax = 6, 25 elements): 2.86
 // ms one block at a time from L2 (k_atomic_k_off_f64), 1.75 ms here (1.87 with one
 // wave per unit, 2.83 with uniform coefficient loads).
-// FP32 rounds two weights where that kernel rounds their product, and sums over l
-// first: its error is 0.99 times that kernel's (lmax 5 and 6, 10 elements, four
-// densities each: 2.68e-7 against 2.70e-7 to 4.03e-7 against 4.06e-7).
+// FP32 error: 0.987 to 0.999 times that kernel's (lmax 2 to 6, l-diagonal,
+// m-diagonal and full densities), on the density changes of a converging Xe solve
+// 0.98 to 1.00 times; 1.007 and 1.07 with both weights of every product rounded.
 
 template <typename T>
 struct KCArgs {
@@ -1219,8 +1219,18 @@ static void build_classes(AtomicDevice &d, const std::vector<int> &src, hipStrea
                   }
                   if (!any) continue;
                   int first = -1, n = 0, stg = 0;
+                  // an entry's largest source weight is 1 and the rows carry it: that
+                  // source's product of weights is rounded once, as in the other kernel
                   auto flush = [&] {
-                    if (n) ent[stg].push_back({(first - it->second[stg].first) | (n - 1) << 16, c});
+                    if (n) {
+                      auto x = c;
+                      double top = 0.0;
+                      for (int z = 0; z < n; ++z)
+                        if (std::fabs(c[KC_ROWS + z]) > std::fabs(top)) top = c[KC_ROWS + z];
+                      for (int z = 0; z < n; ++z) x[KC_ROWS + z] = c[KC_ROWS + z] / top;
+                      for (int r = 0; r < KC_ROWS; ++r) x[r] = c[r] * top;
+                      ent[stg].push_back({(first - it->second[stg].first) | (n - 1) << 16, x});
+                    }
                     n = 0;
                     for (int z = 0; z < KC_SRC; ++z) c[KC_ROWS + z] = 0.0;
                   };
